@@ -76,9 +76,10 @@ typedef struct tmhd_attn_args {
    * Optional scratch (NULL: none).  The work is one item per (head, 256-row
    * query tile); when the items do not fill the last round of workgroups the
    * device holds at once (one per CU for BF16, two per CU for INT8-QK), the
-   * remaining items are split into key ranges whose partial results go here
-   * and are merged by a second kernel on the same stream.  Without it
-   * (or with fewer bytes than tmhd_attn_split_workspace_bytes) every item runs
+   * key tiles of the remaining items are dealt evenly to workgroups, whose
+   * partial results go here and are merged by a second kernel on the same
+   * stream.  Without it every item runs whole; with fewer bytes than
+   * tmhd_attn_split_workspace_bytes they are dealt to fewer workgroups, or run
    * whole.  Calls that share a workspace must be ordered (same stream).
    */
   void *split_workspace;
@@ -127,10 +128,9 @@ int tmhd_attn_fwd_bf16(const tmhd_attn_args *args, void *stream);
 
 /*
  * Bytes of split_workspace that let every attention call with this head_dim
- * on the current device split its last round, on either backend (six
- * [256][head_dim + 1] fp32 slots per CU: the INT8-QK split round can run up
- * to three sub-rounds of two workgroups per CU; 0 for an unsupported
- * head_dim).  Has no counterpart in the reference: the reference's SDPA /
+ * on the current device split its last round, on either backend (four
+ * [256][head_dim + 1] fp32 slots per CU: two for each workgroup the device
+ * holds at once, two per CU for INT8-QK; 0 for an unsupported head_dim).  Has no counterpart in the reference: the reference's SDPA /
  * SageAttention calls manage their own scratch.
  */
 int64_t tmhd_attn_split_workspace_bytes(int32_t head_dim);
@@ -138,8 +138,8 @@ int64_t tmhd_attn_split_workspace_bytes(int32_t head_dim);
 /*
  * tmhd_attn_fwd_bf16 that allocates nothing: args->split_workspace must be
  * NULL, and the key-range partials of a split last round go to a static
- * device array of the library (33,816,576 bytes per device: one
- * [256][head_dim + 1] fp32 slot for each CU of a device with up to 256 CUs;
+ * device array of the library (67,633,152 bytes per device: two
+ * [256][head_dim + 1] fp32 slots for each CU of a device with up to 256 CUs;
  * a device with more CUs is refused with TMHD_ERR_UNSUPPORTED).  Same
  * results as tmhd_attn_fwd_bf16 with a workspace of
  * tmhd_attn_split_workspace_bytes, bit for bit.  Every call on one GPU

@@ -53,17 +53,18 @@
 // Scores of consecutive sub-tiles alternate between two register sets.
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
 #include "tmhd_internal.h"
 
 // Scratch of tmhd_attn_fwd_bf16_noalloc: the key-range partials of a split
-// last round, sized for one [256 rows][128 + 1] fp32 slot per CU of a
-// 256-CU device (33,816,576 bytes, held by every device the library runs on
+// last round, sized for two [256 rows][128 + 1] fp32 slots per CU of a
+// 256-CU device (67,633,152 bytes, held by every device the library runs on
 // until the process ends).  Host code reaches it only through the address
 // hipGetSymbolAddress gives per device (static_scratch below).
-static __device__ __align__(256) unsigned char scratch[256 * 256 * (128 + 1) * 4];
+static __device__ __align__(256) unsigned char scratch[2 * 256 * 256 * (128 + 1) * 4];
 
 namespace tmhd {
 namespace {
@@ -93,30 +94,48 @@ struct Seg {
   int32_t ntiles;
 };
 
-struct KArgs {
+// One attention problem of a launch: its query and output rows, and the
+// segments [seg0, seg_end) of the launch's table.  Problems are ordered by
+// key tiles, most first.
+struct Prob {
   const uint16_t *q;
-  int64_t qts, qhs;
-  const int32_t *q_rows;
-  int32_t q_row0, lq;
   uint16_t *o;
-  int64_t ots, ohs;
-  const int32_t *o_rows;
-  int32_t o_row0;
+  const int32_t *q_rows, *o_rows;
   const int8_t *q8;
   const float *qs;
   int64_t q8hs;
   int32_t qshs;
-  int32_t heads, nqt;
-  float c;  // softmax scale * log2(e)
-  int32_t nseg;
-  int32_t ntiles;  // sum of seg[].ntiles
-  // Items (head, query tile) [0, full) run whole, one per workgroup; the
-  // remaining ones run as nsplit key ranges each, whose partial results
-  // (per workgroup: [kBM][D] normalised O, then [kBM] log2-sum-exp) go to ws.
-  int32_t full, nsplit;
-  float *ws;
-  Seg seg[kMaxSeg];
+  int32_t q_row0, o_row0, lq, nqt;
+  int32_t seg0, seg_end;
+  int32_t ntiles;  // key tiles of its segments
+  int32_t item0;   // items of the problems in front of it
+  int32_t nwhole;  // its items [0, nwhole) run whole
+  int32_t npart;   // key ranges of each of the others (see KArgs)
+  int32_t line0;   // line position of item nwhole
 };
+
+constexpr int kMaxProb = 16, kMaxBatchSeg = 24;
+
+struct KArgs {
+  int64_t qts, qhs, ots, ohs;
+  int32_t heads;
+  float c;  // softmax scale * log2(e)
+  int32_t nprob;
+  // An item is a (problem, head, query tile).  Items [0, full) run whole, one
+  // per workgroup.  The others (the last, partial round) are cut into npart
+  // equal key ranges each, which are laid end to end on a line; each of the
+  // `pieces` remaining workgroups takes the next `share` of them, which may
+  // begin in one item and end in another.  (A line cut at arbitrary key tiles
+  // took the same time, 157 against 159 us at 154 items of 135 key tiles, for
+  // more arithmetic here and in the merge.)  The part of an item that a
+  // workgroup does not hold whole goes to ws slot 2 w (its first item) or
+  // 2 w + 1 (its last): [kBM][D] normalised O, then [kBM] log2-sum-exp.
+  int32_t full, pieces, share, line;
+  float *ws;
+  Prob pr[kMaxProb];
+  Seg seg[kMaxBatchSeg];
+};
+static_assert(sizeof(KArgs) <= 4096, "kernel arguments");
 
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   bf16x2 v = {(__bf16)a, (__bf16)b};
@@ -132,6 +151,69 @@ __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0f70)
 __device__ __forceinline__ int xcd_logical_id(int b, int G) {
   const int xcd = b & 7, pos = b >> 3, per = G >> 3, rem = G & 7;
   return xcd < rem ? xcd * (per + 1) + pos : rem * (per + 1) + (xcd - rem) * per + pos;
+}
+
+// The kernel's arguments through a pointer that the compiler cannot follow, so
+// that the item loop reads them where it needs them: it would otherwise keep
+// them, and what derives from them and from the lane number, in registers
+// across the whole loop, which has none to spare.
+__device__ __forceinline__ const KArgs &kernel_args() {
+  auto p = (const __attribute__((address_space(4))) KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KArgs *)p;
+}
+__device__ __forceinline__ int lane_in_group() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+
+// The key tiles [ta, tb) of one item that a workgroup runs; slot < 0: all of
+// them, else where its partial result goes.
+struct Frag {
+  int p, h, qt, ta, tb, slot;
+};
+
+// A workgroup's part of the launch: one whole item, or its share of the line.
+struct Cursor {
+  int w, pos, hi;  // whole: w = -1 and pos the item (hi = pos + 1)
+};
+__device__ __forceinline__ Cursor cursor_begin(const KArgs &a, int b) {
+  // read what the first item needs in one round trip: the loads below depend on each other
+  asm volatile("" ::"s"(a.pr[0].nqt), "s"(a.pr[0].line0), "s"(a.pr[1].item0), "s"(a.seg[0].tokens), "s"(a.seg[1].tokens),
+               "s"(a.seg[2].tokens), "s"(a.seg[3].tokens));
+  if (b < a.full) return Cursor{-1, b, b + 1};
+  const int w = xcd_logical_id(b - a.full, a.pieces);
+  return Cursor{w, w * a.share, min((w + 1) * a.share, a.line)};
+}
+// The next item (or part of one) of a workgroup; false at its end.
+__device__ __forceinline__ bool cursor_next(const KArgs &a, Cursor &c, Frag &f) {
+  if (c.pos >= c.hi) return false;
+  int p = 0, item;
+  f.slot = -1;
+  if (c.w < 0) {
+    while (p + 1 < a.nprob && c.pos >= a.pr[p + 1].item0) ++p;
+    // head-major logical ids per XCD within the problem's whole items
+    item = xcd_logical_id(c.pos - a.pr[p].item0, a.pr[p].nwhole);
+    f.ta = 0;
+    f.tb = a.pr[p].ntiles;
+    c.pos = c.hi;
+  } else {
+    while (p + 1 < a.nprob && c.pos >= a.pr[p + 1].line0) ++p;
+    const int np = a.pr[p].npart, nt = a.pr[p].ntiles, off = c.pos - a.pr[p].line0;
+    const int it = uniform(off / np), q0 = off - it * np, q1 = min(np, q0 + c.hi - c.pos);
+    f.ta = uniform(nt * q0 / np);
+    f.tb = uniform(nt * q1 / np);
+    if (q0 > 0 || q1 < np) f.slot = 2 * c.w + (c.pos == c.w * a.share ? 0 : 1);
+    c.pos += q1 - q0;
+    item = a.pr[p].nwhole + it;
+  }
+  f.p = p;
+  f.h = uniform(item / a.pr[p].nqt);
+  f.qt = item - f.h * a.pr[p].nqt;
+  return true;
 }
 
 // Position of one head's tile stream: segment s, tile t of nt, with the
@@ -157,21 +239,20 @@ __device__ __forceinline__ void stream_set(Stream &S, const KArgs &a, int h, int
   S.ks = I8 ? G.ks + (int64_t)h * G.kshs : nullptr;
 }
 
-// Tile gt of the concatenated segments.
+// Tile gt of the concatenated segments from s on.
 template <bool I8>
-__device__ __forceinline__ void stream_seek(Stream &S, const KArgs &a, int h, int gt) {
-  int s = 0;
-  while (s + 1 < a.nseg && gt >= a.seg[s].ntiles) gt -= a.seg[s++].ntiles;
+__device__ __forceinline__ void stream_seek(Stream &S, const KArgs &a, int h, int s, int send, int gt) {
+  while (s + 1 < send && gt >= a.seg[s].ntiles) gt -= a.seg[s++].ntiles;
   stream_set<I8>(S, a, h, s);
   S.t = gt;
 }
 
-// Next tile; the last tile of the last segment repeats (loads of a repeated
-// tile are in-bounds and their results unused).
+// Next tile; the last tile of the last segment (send - 1) repeats (loads of a
+// repeated tile are in-bounds and their results unused).
 template <bool I8>
-__device__ __forceinline__ void stream_next(Stream &S, const KArgs &a, int h) {
+__device__ __forceinline__ void stream_next(Stream &S, const KArgs &a, int h, int send) {
   if (++S.t >= S.nt) {
-    if (S.s + 1 < a.nseg) {
+    if (S.s + 1 < send) {
       asm volatile("" ::: "memory");
       stream_set<I8>(S, a, h, S.s + 1);
     } else {
@@ -438,7 +519,7 @@ constexpr bool plan_valid(const SlotPlan &s, int nqk, int npv, int db, int nld, 
 }
 
 template <int D>
-__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_fwd_kernel(const KArgs a) {
+__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(1, 1))) attn_fwd_kernel(const KArgs args) {
   constexpr int KROW = 2 * D;  // bytes per key row in memory
   constexpr int KCPR = KROW / 16;       // 16-byte chunks per key row
   constexpr int KRS = KROW + 16;        // LDS key row stride: one pad chunk, an odd number of chunks
@@ -467,50 +548,15 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   __shared__ __attribute__((aligned(1024))) char smem[3 * KT + 3 * VT];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
-  // item L, whole or key-tile range [t_begin, t_begin + cnt) of part `part`
-  int L, part = -1, t_begin = 0, cnt = a.ntiles;
-  if ((int)blockIdx.x < a.full) {
-    L = xcd_logical_id(blockIdx.x, a.full);
-  } else {
-    const int tb = blockIdx.x - a.full, item = tb / a.nsplit;
-    L = a.full + item;
-    part = tb - item * a.nsplit;
-    t_begin = a.ntiles * part / a.nsplit;
-    cnt = a.ntiles * (part + 1) / a.nsplit - t_begin;
-  }
-  const int h = L / a.nqt;
-  const int qt = L - h * a.nqt;
-  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, g = lane >> 5;
+  Cursor cur = cursor_begin(args, blockIdx.x);
+  Frag fr;
+  while (cursor_next(kernel_args(), cur, fr)) {
+  const KArgs &a = kernel_args();
+  const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index (uniform)
-  const int q0 = qt * kBM + w * kQW;                        // first query row of this wave
-
-  // ---- query operands of both 32-row halves (B operands of S^T = K Q^T), pinned in AGPRs
-  i32x4 qv[2][QST];
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const int ql = q0 + hf * 32 + lr;
-    if (ql < a.lq) {
-      const int row = a.q_rows ? a.q_rows[ql] : a.q_row0 + ql;
-      const uint16_t *p = a.q + (int64_t)row * a.qts + (int64_t)h * a.qhs + g * 8;
-#pragma unroll
-      for (int st = 0; st < QST; ++st) {
-        const i32x4 raw = *(const i32x4 *)(p + st * 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t u = (uint32_t)raw[e];
-          qv[hf][st][e] =
-              (int)pack_bf16x2(__uint_as_float(u << 16) * a.c, __uint_as_float(u & 0xffff0000u) * a.c);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int st = 0; st < QST; ++st) qv[hf][st] = i32x4{0, 0, 0, 0};
-    }
-  }
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-    for (int st = 0; st < QST; ++st) qpin(hf * QST + st, qv[hf][st]);
+  const Prob &P = a.pr[fr.p];
+  const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
+  const int q0 = fr.qt * kBM + w * kQW;  // first query row of this wave
 
   // per-lane LDS read offsets from smem (bytes; k-step, key half, buffer and db parts are uniform/immediate)
   const uint32_t kro = lr * KRS + g * 16;
@@ -595,6 +641,45 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
     return m;
   };
 
+  // ---- prologue: K(0..2), V(0..1) resident; S = scores of sub-tile 0 (minus m)
+  Stream t0, t1, t2, t3;
+  stream_seek<false>(t0, a, h, P.seg0, send, fr.ta);
+  t1 = t0;
+  stream_next<false>(t1, a, h, send);
+  t2 = t1;
+  stream_next<false>(t2, a, h, send);
+  t3 = t2;
+  stream_next<false>(t3, a, h, send);
+  load_k(t0, 0);
+  load_k(t1, 1);
+  load_v(t0, 0);
+  // ---- query operands of both 32-row halves (B operands of S^T = K Q^T), pinned in AGPRs;
+  // all loads issued (behind the tile loads) before any is used, rows past the
+  // end re-read the last row and are zeroed
+  i32x4 qv[2][QST];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const int ql = min(q0 + hf * 32 + lr, P.lq - 1);
+    const int row = P.q_rows ? P.q_rows[ql] : P.q_row0 + ql;
+    const uint16_t *p = P.q + (int64_t)row * a.qts + (int64_t)h * a.qhs + g * 8;
+#pragma unroll
+    for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 16);
+  }
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const bool live = q0 + hf * 32 + lr < P.lq;
+#pragma unroll
+    for (int st = 0; st < QST; ++st) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t u = (uint32_t)qv[hf][st][e];
+        const uint32_t x = pack_bf16x2(__uint_as_float(u << 16) * a.c, __uint_as_float(u & 0xffff0000u) * a.c);
+        qv[hf][st][e] = live ? (int)x : 0;
+      }
+      qpin(hf * QST + st, qv[hf][st]);
+    }
+  }
+
   f32x16 o[2][DB];  // block hf * DB + db lives in AGPRs a[16 b, 16 b + 15]
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf)
@@ -609,18 +694,6 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   f32x16 negm[2];  // -mref in every element, the score accumulator start
   const f32x16 zero16 = {};
 
-  // ---- prologue: K(0..2), V(0..1) resident; S = scores of sub-tile 0 (minus m)
-  Stream t0, t1, t2, t3;
-  stream_seek<false>(t0, a, h, t_begin);
-  t1 = t0;
-  stream_next<false>(t1, a, h);
-  t2 = t1;
-  stream_next<false>(t2, a, h);
-  t3 = t2;
-  stream_next<false>(t3, a, h);
-  load_k(t0, 0);
-  load_k(t1, 1);
-  load_v(t0, 0);
   // valid keys of tiles j, j+1, j+2, j+3
   int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
   wait_vmem();
@@ -841,7 +914,7 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
     }
     lvd = lds0 + 3 * KT + b1 * VT;
     sv = sk;
-    stream_next<false>(sk, a, h);
+    stream_next<false>(sk, a, h, send);
     nv3 = tile_valid(sk);
   }
 
@@ -854,15 +927,15 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
     for (int db = 0; db < DB; ++db) opin(hf * DB + db, o[hf][db]);
-  if (part >= 0) {
-    // key range of a split item: normalised partial O and its log2-sum-exp
-    float *wo = a.ws + (int64_t)(blockIdx.x - a.full) * (kBM * D + kBM);
+  if (fr.slot >= 0) {
+    // part of an item: normalised partial O and its log2-sum-exp
+    float *wo = a.ws + (int64_t)fr.slot * (kBM * D + kBM);
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
       const float inv = 1.0f / lt;
       const int rl = w * kQW + hf * 32 + lr;  // row within the item
-      if (q0 + hf * 32 + lr < a.lq) {
+      if (q0 + hf * 32 + lr < P.lq) {
         float *op = wo + rl * D + 4 * g;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -873,25 +946,28 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
         if (g == 0) wo[kBM * D + rl] = mref[hf] + __log2f(lt);
       }
     }
-    return;
-  }
+  } else {
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-    const float inv = 1.0f / lt;
-    const int ql = q0 + hf * 32 + lr;
-    if (ql < a.lq) {
-      const int row = a.o_rows ? a.o_rows[ql] : a.o_row0 + ql;
-      uint16_t *op = a.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
+    for (int hf = 0; hf < 2; ++hf) {
+      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
+      const float inv = 1.0f / lt;
+      const int ql = q0 + hf * 32 + lr;
+      if (ql < P.lq) {
+        const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
+        uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
-                      (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
-          *(i32x2 *)(op + db * 32 + 8 * u) = pr;
-        }
+          for (int u = 0; u < 4; ++u) {
+            i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
+                        (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
+            *(i32x2 *)(op + db * 32 + 8 * u) = pr;
+          }
+      }
     }
+  }
+  // the next item's first tile loads overwrite tiles that other waves may still read
+  __syncthreads();
   }
 }
 
@@ -992,7 +1068,7 @@ __device__ __forceinline__ void pv_v(f32x16 &o, i32x4 v, i32x4 p) {
 }
 
 template <int D>
-__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_i8_kernel(const KArgs a) {
+__global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) attn_i8_kernel(const KArgs args) {
   constexpr int KROW = D;            // bytes per int8 key row
   constexpr int KCPR = KROW / 16;    // 16-byte chunks per key row
   constexpr int KRS = KROW + 16;     // LDS key row stride (one pad chunk)
@@ -1018,33 +1094,15 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   __shared__ __attribute__((aligned(1024))) char smem[TAB + kWaves * 64 * 32];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
-  int L, part = -1, t_begin = 0, cnt = a.ntiles;
-  if ((int)blockIdx.x < a.full) {
-    L = xcd_logical_id(blockIdx.x, a.full);
-  } else {
-    const int tb = blockIdx.x - a.full, item = tb / a.nsplit;
-    L = a.full + item;
-    part = tb - item * a.nsplit;
-    t_begin = a.ntiles * part / a.nsplit;
-    cnt = a.ntiles * (part + 1) / a.nsplit - t_begin;
-  }
-  const int h = L / a.nqt;
-  const int qt = L - h * a.nqt;
-  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, g = lane >> 5;
+  Cursor cur = cursor_begin(args, blockIdx.x);
+  Frag fr;
+  while (cursor_next(kernel_args(), cur, fr)) {
+  const KArgs &a = kernel_args();
+  const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q0 = qt * kBM + w * kQW;
-
-  // query operands of both 32-row halves (B operands of S^T = K Q^T)
-  i32x4 qv[2][QST];
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const int ql = q0 + hf * 32 + lr;
-    const int8_t *p = a.q8 + (int64_t)h * a.q8hs + (int64_t)ql * D + g * 16;
-#pragma unroll
-    for (int st = 0; st < QST; ++st) qv[hf][st] = ql < a.lq ? *(const i32x4 *)(p + st * 32) : i32x4{0, 0, 0, 0};
-  }
-  // softmax scale * log2(e) * query block scale (the wave's 64 rows lie in one 128-row block)
-  const float cq = a.c * a.qs[(int64_t)h * a.qshs + q0 / TMHD_QUANT_BLOCK] * (1.0f / kI8Slope);
+  const Prob &P = a.pr[fr.p];
+  const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
+  const int q0 = fr.qt * kBM + w * kQW;
 
   const uint32_t kro = lr * KRS + g * 16;
   const uint32_t vro = 3 * KT + lr * VRS + g * 16;
@@ -1057,18 +1115,12 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   auto vblk = [&](int i) { return min(w + i * kWaves, NVL - 1); };
   constexpr int NLD = KWL + VWL;
   static_assert(NLD <= 8, "eight offset words per lane");
-  {
-    uint32_t tab[8] = {};
+  auto koff_of = [&](int i) {
+    const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
+    return (uint32_t)(row * KROW + chunk * 16);
+  };
 #pragma unroll
-    for (int i = 0; i < KWL; ++i) {
-      const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
-      tab[i] = row * KROW + chunk * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < VWL; ++i) tab[KWL + i] = 0;  // set by write_vtab once the streams are known
-    *(i32x4 *)(smem + TAB + tid * 32) = i32x4{(int)tab[0], (int)tab[1], (int)tab[2], (int)tab[3]};
-    *(i32x4 *)(smem + TAB + tid * 32 + 16) = i32x4{(int)tab[4], (int)tab[5], (int)tab[6], (int)tab[7]};
-  }
+  for (int i = 0; i < KWL; ++i) *(uint32_t *)(smem + TAB + tid * 32 + i * 4) = koff_of(i);
   auto read_tab = [&](uint32_t (&t)[8]) {
     const i32x4 lo = *(const i32x4 *)(smem + TAB + tid * 32), hi = *(const i32x4 *)(smem + TAB + tid * 32 + 16);
 #pragma unroll
@@ -1105,10 +1157,10 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
     else
       load_lds16(vbase, t[n], vdst + vblk(n - KWL) * 1024);
   };
-  auto load_k = [&](const uint32_t (&t)[8], const Stream &S, int buf) {
+  auto load_k = [&](const Stream &S, int buf) {
     const char *base = S.kb + (int64_t)S.t * (kBN * KROW);
 #pragma unroll
-    for (int i = 0; i < KWL; ++i) load_lds16(base, t[i], lds0 + buf * KT + kblk(i) * 1024);
+    for (int i = 0; i < KWL; ++i) load_lds16(base, koff_of(i), lds0 + buf * KT + kblk(i) * 1024);
   };
   auto load_v = [&](const Stream &S, int buf) {
     const char *base = S.vb + S.t * (kBN * 2);
@@ -1152,6 +1204,37 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
     return m;
   };
 
+
+  // ---- prologue: K(0), K(1), V(0) resident; P of sub-tile 0
+  Stream t0, t1, t2, t3;
+  stream_seek<true>(t0, a, h, P.seg0, send, fr.ta);
+  t1 = t0;
+  stream_next<true>(t1, a, h, send);
+  t2 = t1;
+  stream_next<true>(t2, a, h, send);
+  t3 = t2;
+  stream_next<true>(t3, a, h, send);
+  load_k(t0, 0);
+  load_k(t1, 1);
+  load_v(t0, 0);
+  write_vtab(t1.vrs2);  // the loop's first value loads are of tile 1
+  // query operands of both 32-row halves (B operands of S^T = K Q^T); rows past the end re-read
+  // the last row and are zeroed
+  i32x4 qv[2][QST];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const int8_t *p = P.q8 + (int64_t)h * P.q8hs + (int64_t)min(q0 + hf * 32 + lr, P.lq - 1) * D + g * 16;
+#pragma unroll
+    for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 32);
+  }
+  // softmax scale * log2(e) * query block scale (the wave's 64 rows lie in one 128-row block)
+  const float cq = a.c * P.qs[(int64_t)h * P.qshs + q0 / TMHD_QUANT_BLOCK] * (1.0f / kI8Slope);
+
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf)
+    if (q0 + hf * 32 + lr >= P.lq)
+#pragma unroll
+      for (int st = 0; st < QST; ++st) qv[hf][st] = i32x4{0, 0, 0, 0};
 
   // Rare path, and the first sub-tile: the scores of a 32-key sub-tile from
   // LDS (K rows at kb) into sn, dequantised against the reference, keys at or
@@ -1211,24 +1294,6 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
       }
   };
 
-  // ---- prologue: K(0), K(1), V(0) resident; P of sub-tile 0
-  Stream t0, t1, t2, t3;
-  stream_seek<true>(t0, a, h, t_begin);
-  t1 = t0;
-  stream_next<true>(t1, a, h);
-  t2 = t1;
-  stream_next<true>(t2, a, h);
-  t3 = t2;
-  stream_next<true>(t3, a, h);
-  write_vtab(t1.vrs2);  // the loop's first value loads are of tile 1
-  __syncthreads();  // the offset table
-  {
-    uint32_t t[8];
-    read_tab(t);
-    load_k(t, t0, 0);
-    load_k(t, t1, 1);
-    load_v(t0, 0);
-  }
   int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
   float ks2 = load_ks(t2);
   float ks0 = load_ks(t0), ks1 = load_ks(t1);
@@ -1308,10 +1373,13 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
       for (int u = 0; u < 16; ++u)
         if (pl.c[u] == r) {
           const int hf = u >> 3, q = u & 7;
-          int pr = (int)pack_bf16x2(f(sn[hf][2 * q]), f(sn[hf][2 * q + 1]));
+          // the adds first, then the pack: the next unit's add does not follow the
+          // statement that pins its operand directly (a wait state each otherwise)
           ts[hf] += f(sn[hf][2 * q]);
           ts[hf] += f(sn[hf][2 * q + 1]);
-          asm volatile("" : "+v"(pr), "+v"(ts[hf]));
+          asm volatile("" : "+v"(ts[hf]));
+          int pr = (int)pack_bf16x2(f(sn[hf][2 * q]), f(sn[hf][2 * q + 1]));
+          asm volatile("" : "+v"(pr));
           pkn[hf][q >> 2][q & 3] = pr;
         }
       __builtin_amdgcn_sched_barrier(0);
@@ -1372,21 +1440,21 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
     lvd = lds0 + 3 * KT + (vb ^ 1) * VT;
     ks2 = load_ks(sk);
     sv = sk;
-    stream_next<true>(sk, a, h);
+    stream_next<true>(sk, a, h, send);
     nv3 = tile_valid(sk);
   }
 
   // ---- epilogue (as the kernel above)
   wait_vmem();
   drain_o();
-  if (part >= 0) {
-    float *wo = a.ws + (int64_t)(blockIdx.x - a.full) * (kBM * D + kBM);
+  if (fr.slot >= 0) {
+    float *wo = a.ws + (int64_t)fr.slot * (kBM * D + kBM);
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
       const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
       const float inv = 1.0f / lt;
       const int rl = w * kQW + hf * 32 + lr;
-      if (q0 + hf * 32 + lr < a.lq) {
+      if (q0 + hf * 32 + lr < P.lq) {
         float *op = wo + rl * D + 4 * g;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -1397,54 +1465,83 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
         if (g == 0) wo[kBM * D + rl] = mref[hf] + __log2f(lt);
       }
     }
-    return;
-  }
+  } else {
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-    const float inv = 1.0f / lt;
-    const int ql = q0 + hf * 32 + lr;
-    if (ql < a.lq) {
-      const int row = a.o_rows ? a.o_rows[ql] : a.o_row0 + ql;
-      uint16_t *op = a.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
+    for (int hf = 0; hf < 2; ++hf) {
+      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
+      const float inv = 1.0f / lt;
+      const int ql = q0 + hf * 32 + lr;
+      if (ql < P.lq) {
+        const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
+        uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
-                      (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
-          *(i32x2 *)(op + db * 32 + 8 * u) = pr;
-        }
+          for (int u = 0; u < 4; ++u) {
+            i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
+                        (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
+            *(i32x2 *)(op + db * 32 + 8 * u) = pr;
+          }
+      }
     }
+  }
+  // the next item's first tile loads overwrite tiles that other waves may still read
+  __syncthreads();
   }
 }
 
-// Merge of split items: O = sum_p 2^(lse_p - lse) O_p with lse = log2 sum_p
-// 2^lse_p (the partial O_p are normalised).  One thread per 4 columns of a
-// row; item i of the split ones owns workspace blocks [i * nsplit, (i+1) * nsplit).
+// Merge of the items that the shares cut: O = sum_p 2^(lse_p - lse) O_p with
+// lse = log2 sum_p 2^lse_p over the item's parts (the partial O_p are
+// normalised).  One thread per 4 columns of a row; items full, full + 1, ...
+// have kBM / RPB blocks each.  An item that one workgroup holds whole is left.
 template <int D>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const KArgs a) {
   constexpr int CG = D / 4, RPB = 256 / CG;  // column groups per row, rows per block
-  const int item = blockIdx.x / (kBM / RPB);
-  const int rl = (blockIdx.x - item * (kBM / RPB)) * RPB + threadIdx.x / CG;
+  const int item = a.full + blockIdx.x / (kBM / RPB);
+  int p = 0;
+  while (p + 1 < a.nprob && item >= a.pr[p + 1].item0) ++p;
+  const Prob &P = a.pr[p];
+  const int L = item - P.item0, h = L / P.nqt, qt = L - h * P.nqt;
+  const int rl = (blockIdx.x % (kBM / RPB)) * RPB + threadIdx.x / CG;
   const int cg = threadIdx.x % CG;
-  const int L = a.full + item, h = L / a.nqt, qt = L - h * a.nqt;
   const int ql = qt * kBM + rl;
-  if (ql >= a.lq) return;
+  if (ql >= P.lq) return;
+  // workgroups w0 .. w1 hold ranges [s, s + npart) of the line; the item is
+  // w0's last, unless it begins there, and the first of the others
+  const int s = P.line0 + (L - P.nwhole) * P.npart;
+  const int w0 = s / a.share, n = (s + P.npart - 1) / a.share - w0 + 1;
+  if (n < 2) return;
+  const int first = s > w0 * a.share ? 1 : 0;
   constexpr int64_t slot = kBM * D + kBM;
-  const float *base = a.ws + (int64_t)item * a.nsplit * slot;
-  float m = -INFINITY;
-  for (int p = 0; p < a.nsplit; ++p) m = fmaxf(m, base[p * slot + kBM * D + rl]);
-  float wsum = 0.0f;
+  // four parts at a time, their loads all issued before any is used
+  float m = -INFINITY, wsum = 0.0f;
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int p = 0; p < a.nsplit; ++p) {
-    const float wp = __builtin_amdgcn_exp2f(base[p * slot + kBM * D + rl] - m);
-    wsum += wp;
-    acc += wp * *(const f32x4 *)(base + p * slot + rl * D + 4 * cg);
+  for (int i = 0; i < n; i += 4) {
+    float lse[4];
+    f32x4 val[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = min(i + j, n - 1);
+      const float *b = a.ws + (int64_t)(2 * (w0 + r) + (r == 0 ? first : 0)) * slot;
+      lse[j] = b[kBM * D + rl];
+      val[j] = *(const f32x4 *)(b + rl * D + 4 * cg);
+    }
+    const float mn = fmaxf(m, fmaxf(fmaxf(lse[0], lse[1]), fmaxf(lse[2], lse[3])));
+    const float keep = __builtin_amdgcn_exp2f(m - mn);
+    wsum *= keep;
+    acc *= keep;
+    m = mn;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i + j < n) {
+        const float wp = __builtin_amdgcn_exp2f(lse[j] - m);
+        wsum += wp;
+        acc += wp * val[j];
+      }
   }
   const float inv = 1.0f / wsum;
-  const int row = a.o_rows ? a.o_rows[ql] : a.o_row0 + ql;
-  uint16_t *op = a.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * cg;
+  const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
+  uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * cg;
   *(i32x2 *)op = i32x2{(int)pack_bf16x2(acc[0] * inv, acc[1] * inv), (int)pack_bf16x2(acc[2] * inv, acc[3] * inv)};
 }
 
@@ -1452,45 +1549,74 @@ bool aligned(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
 int64_t split_slot_bytes(int D) { return (int64_t)kBM * (D + 1) * 4; }
 
-// Key ranges per remaining item: as many as fit the CUs the whole items leave
-// free in the last round, at most 8, each at least 4 tiles long.
-int choose_split(int items, int cus, int ntiles) {
-  if (cus <= 0) return 1;
-  const int rem = items % cus;
-  if (rem == 0) return 1;
-  int n = cus / rem;
-  n = n < 8 ? n : 8;
-  n = n < ntiles / 4 ? n : ntiles / 4;
-  return n > 1 ? n : 1;
+// Times behind the split rule, in microseconds, fitted to calls of 8 to 280
+// items (6 to 252 key tiles, both head dims and backends) timed at 1 to 15
+// ranges per item: the rule's choice is within 8% of the best of them.
+// A key tile of a workgroup, by how many run: more of them run at a lower
+// clock (the card's power limit), and two INT8-QK workgroups share a CU.
+double tile_us(bool i8, int D, int workgroups, int cus) {
+  if (i8 && workgroups > cus) return D == 128 ? 2.6 : 1.9;
+  const double one = D == 128 ? (i8 ? 1.22 : 1.38) : (i8 ? 1.0 : 1.1);
+  return one * (1.0 + 0.2 * workgroups / cus);
 }
+// What an item costs besides its tiles, and the merge: its launch, and a
+// partial slot's write and read (at head_dim 128).
+constexpr double kItemUs = 6.0, kMergeUs = 8.0, kMergeUsPerSlot = 0.02;
+constexpr int kMaxParts = 16;
 
-// The INT8-QK kernel's last round, over `slots` resident workgroups (two per
-// CU): the rem items it holds run as n key ranges each, n (at most 8, each
-// range at least 4 key tiles, rem * n within the workspace's max_parts)
-// chosen to make the round shortest, ceil(rem * n / slots) sub-rounds of 1 / n
-// of an item (the earliest n on ties).  A round that fills three quarters of
-// the slots, as at 768p (1,920 items on 512 slots: 384), runs as 4 ranges in 3
-// full sub-rounds, 0.75 of an item instead of 1; a round of at most half the
-// slots gets the choose_split ranges.
-int choose_split_i8(int items, int slots, int ntiles, int64_t max_parts) {
-  if (slots <= 0) return 1;
-  const int rem = items % slots;
-  if (rem == 0) return 1;
-  int best = 1;
-  int64_t best_rounds = 1, best_n = 1;  // the round lasts best_rounds / best_n items
-  for (int n = 2; n <= 8 && n <= ntiles / 4; ++n) {
-    if ((int64_t)rem * n > max_parts) break;
-    const int64_t rounds = ((int64_t)rem * n + slots - 1) / slots;
-    if (rounds * best_n < best_rounds * n) {
-      best = n;
-      best_rounds = rounds;
-      best_n = n;
-    }
+// Decides how the last, partial round of items runs: whole, or as key ranges
+// dealt evenly to workgroups (see KArgs).  `slots` workgroups are resident at
+// once.  n ranges per item of the longest problem (fewer of the others, of
+// about the same length) are shared out `share` to a workgroup; the n whose
+// estimated time is least, if it beats whole items.
+void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
+  const int cus = device_cus(), slots = (i8 ? 2 : 1) * cus;
+  const Prob &last = k.pr[k.nprob - 1];
+  const int items = last.item0 + last.nqt * k.heads;
+  k.full = items;
+  for (int p = 0; p < k.nprob; ++p) k.pr[p].nwhole = k.pr[p].nqt * k.heads;
+  if (cus <= 0 || !k.ws || items % slots == 0) return;
+  const int full = items - items % slots;
+  int nwhole[kMaxProb], rest[kMaxProb], longest = 0;  // longest: key tiles of the round's longest item
+  for (int p = 0; p < k.nprob; ++p) {
+    const int n = k.pr[p].nwhole, whole = full - k.pr[p].item0;
+    nwhole[p] = whole < 0 ? 0 : whole < n ? whole : n;
+    rest[p] = n - nwhole[p];
+    if (rest[p] && k.pr[p].ntiles > longest) longest = k.pr[p].ntiles;
   }
-  return best;
+  auto parts = [&](int p, int n) {
+    const int q = (int)(((int64_t)2 * n * k.pr[p].ntiles + longest) / (2 * (int64_t)longest));
+    return q < 1 ? 1 : q;
+  };
+  double best = 0.97 * (longest * tile_us(i8, D, items - full, cus) + kItemUs);
+  int best_n = 0;
+  for (int n = 2; n <= kMaxParts && 2 * n <= longest; ++n) {
+    int64_t line = 0;
+    for (int p = 0; p < k.nprob; ++p) line += (int64_t)rest[p] * parts(p, n);
+    const int64_t share = (line + slots - 1) / slots, pieces = (line + share - 1) / share;
+    if (line > 0x3fffffff || 2 * pieces * split_slot_bytes(D) > ws_bytes) continue;
+    const int64_t begun = n % share == 0 ? 1 : share / n + 2;  // items a workgroup touches
+    const int64_t cut = pieces + (n % share == 0 ? 0 : items - full);
+    const double us = (double)share * longest / n * tile_us(i8, D, (int)pieces, cus) + kItemUs * (1 + 0.7 * (double)(begun - 1)) +
+                      kMergeUs + D / 128.0 * kMergeUsPerSlot * (double)cut;
+    if (us < best) best = us, best_n = n;
+  }
+  if (!best_n) return;
+  k.full = full;
+  k.line = 0;
+  for (int p = 0; p < k.nprob; ++p) {
+    k.pr[p].nwhole = nwhole[p];
+    k.pr[p].npart = parts(p, best_n);
+    k.pr[p].line0 = k.line;
+    k.line += rest[p] * k.pr[p].npart;
+  }
+  k.share = (k.line + slots - 1) / slots;
+  k.pieces = (k.line + k.share - 1) / k.share;
 }
 
-int build_kargs(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, KArgs *k) {
+// Checks one call's arguments and fills its problem and segments (tables
+// starting at P and S).
+int build_problem(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, Prob *P, Seg *seg) {
   if (!args) return set_error(TMHD_ERR_INVALID, "attention: null args");
   const int D = args->head_dim;
   if (D != 64 && D != 128) return set_error(TMHD_ERR_UNSUPPORTED, "attention: head_dim %d (64 or 128)", D);
@@ -1505,31 +1631,24 @@ int build_kargs(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, KA
   const int nqt = (args->lq + kBM - 1) / kBM;
   if (args->split_workspace && (!aligned(args->split_workspace, 16) || args->split_workspace_bytes < 0))
     return set_error(TMHD_ERR_INVALID, "attention: split workspace must be 16-byte aligned");
-  *k = KArgs{};
-  k->q = (const uint16_t *)args->q;
-  k->qts = args->q_token_stride;
-  k->qhs = args->q_head_stride;
-  k->q_rows = args->q_rows;
-  k->q_row0 = args->q_row0;
-  k->lq = args->lq;
-  k->o = (uint16_t *)args->o;
-  k->ots = args->o_token_stride;
-  k->ohs = args->o_head_stride;
-  k->o_rows = args->o_rows;
-  k->o_row0 = args->o_row0;
-  k->heads = args->heads;
-  k->nqt = nqt;
-  k->c = args->scale * kLog2e;
-  k->nseg = args->n_segments;
+  *P = Prob{};
+  P->q = (const uint16_t *)args->q;
+  P->q_rows = args->q_rows;
+  P->q_row0 = args->q_row0;
+  P->lq = args->lq;
+  P->o = (uint16_t *)args->o;
+  P->o_rows = args->o_rows;
+  P->o_row0 = args->o_row0;
+  P->nqt = nqt;
   if (i8) {
     if (!qq || !qq->q_i8 || !qq->q_scale || !aligned(qq->q_i8, 16) || qq->q_head_stride % 16)
       return set_error(TMHD_ERR_INVALID, "attention i8: bad quantized query buffers");
     if (qq->q_head_stride < (int64_t)nqt * kBM * D || qq->q_scale_head_stride < nqt * (kBM / TMHD_QUANT_BLOCK))
       return set_error(TMHD_ERR_INVALID, "attention i8: quantized query capacity below round_up(lq, 256)");
-    k->q8 = qq->q_i8;
-    k->qs = qq->q_scale;
-    k->q8hs = qq->q_head_stride;
-    k->qshs = qq->q_scale_head_stride;
+    P->q8 = qq->q_i8;
+    P->qs = qq->q_scale;
+    P->q8hs = qq->q_head_stride;
+    P->qshs = qq->q_scale_head_stride;
   }
   for (int i = 0; i < args->n_segments; ++i) {
     const tmhd_kv_segment &sg = args->seg[i];
@@ -1543,7 +1662,8 @@ int build_kargs(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, KA
       return set_error(TMHD_ERR_INVALID,
                        "attention: segment %d is not a slot (tokens %d, vt_row_stride %d, strides %lld/%lld)", i,
                        sg.tokens, sg.vt_row_stride, (long long)sg.k_head_stride, (long long)sg.vt_head_stride);
-    Seg &S = k->seg[i];
+    Seg &S = seg[i];
+    S = Seg{};
     S.k = (const uint16_t *)sg.k;
     S.vt = (const uint16_t *)sg.vt;
     S.khs = sg.k_head_stride;
@@ -1551,7 +1671,7 @@ int build_kargs(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, KA
     S.vrs = sg.vt_row_stride;
     S.tokens = sg.tokens;
     S.ntiles = (int)(cap / kBN);
-    k->ntiles += S.ntiles;
+    P->ntiles += S.ntiles;
     if (i8) {
       if (!qq->k_i8[i] || !qq->k_scale[i] || !aligned(qq->k_i8[i], 16) || qq->k_head_stride[i] < cap * D ||
           qq->k_head_stride[i] % 16 || qq->k_scale_head_stride[i] < (cap + TMHD_QUANT_BLOCK - 1) / TMHD_QUANT_BLOCK)
@@ -1565,52 +1685,84 @@ int build_kargs(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, KA
   return TMHD_OK;
 }
 
+// One launch of the problems in k (their segments set), and its merge.
 template <bool I8>
-int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, void *stream) {
-  KArgs k;
-  int st = build_kargs(args, qq, I8, &k);
-  if (st) return st;
-  if (args->lq == 0) return TMHD_OK;
-  const int64_t items = (int64_t)k.nqt * k.heads;
-  if (items > 0x3fffffff) return set_error(TMHD_ERR_UNSUPPORTED, "attention: grid too large");
-  // split the items of the last, partial round into key ranges when a workspace is given
-  k.full = (int)items;
-  k.nsplit = 1;
-  int rem = 0;
-  if (args->split_workspace) {
-    // workgroups resident at once: one per CU (BF16), two per CU (INT8-QK)
-    const int slots = (I8 ? 2 : 1) * device_cus();
-    const int n = I8 ? choose_split_i8((int)items, slots, k.ntiles,
-                                       args->split_workspace_bytes / split_slot_bytes(args->head_dim))
-                     : choose_split((int)items, slots, k.ntiles);
-    rem = n > 1 ? (int)(items % slots) : 0;
-    if (n > 1 && args->split_workspace_bytes >= (int64_t)rem * n * split_slot_bytes(args->head_dim)) {
-      k.full = (int)items - rem;
-      k.nsplit = n;
-      k.ws = (float *)args->split_workspace;
-    } else {
-      rem = 0;
-    }
+int launch_group(KArgs &k, int nseg, int D, void *ws, int64_t ws_bytes, hipStream_t s, const char *what) {
+  if (k.nprob == 0) return TMHD_OK;
+  (void)nseg;
+  std::stable_sort(k.pr, k.pr + k.nprob, [](const Prob &x, const Prob &y) { return x.ntiles > y.ntiles; });
+  int64_t items = 0;
+  for (int p = 0; p < k.nprob; ++p) {
+    k.pr[p].item0 = (int)items;
+    items += (int64_t)k.pr[p].nqt * k.heads;
+    if (items > 0x3fffffff) return set_error(TMHD_ERR_UNSUPPORTED, "attention: grid too large");
   }
-  const unsigned grid = (unsigned)(k.full + (int64_t)rem * k.nsplit);
-  hipStream_t s = (hipStream_t)stream;
-  if (I8 && args->head_dim == 128)
+  k.ws = (float *)ws;
+  plan_split(k, I8, D, ws_bytes);
+  const unsigned grid = (unsigned)(k.full + k.pieces);
+  if (I8 && D == 128)
     hipLaunchKernelGGL((attn_i8_kernel<128>), dim3(grid), dim3(kWaves * 64), 0, s, k);
   else if (I8)
     hipLaunchKernelGGL((attn_i8_kernel<64>), dim3(grid), dim3(kWaves * 64), 0, s, k);
-  else if (args->head_dim == 128)
+  else if (D == 128)
     hipLaunchKernelGGL((attn_fwd_kernel<128>), dim3(grid), dim3(kWaves * 64), 0, s, k);
   else
     hipLaunchKernelGGL((attn_fwd_kernel<64>), dim3(grid), dim3(kWaves * 64), 0, s, k);
-  const char *what = I8 ? "tmhd_attn_fwd_i8qk" : "tmhd_attn_fwd_bf16";
-  int st2 = check_launch(what);
-  if (st2 || rem == 0) return st2;
-  const unsigned mgrid = (unsigned)rem * (kBM / (256 / (args->head_dim / 4)));
-  if (args->head_dim == 128)
+  const int st = check_launch(what);
+  if (st || !k.pieces) return st;
+  const unsigned mgrid = (unsigned)(items - k.full) * (kBM / (256 / (D / 4)));
+  if (D == 128)
     hipLaunchKernelGGL((attn_merge_kernel<128>), dim3(mgrid), dim3(256), 0, s, k);
   else
     hipLaunchKernelGGL((attn_merge_kernel<64>), dim3(mgrid), dim3(256), 0, s, k);
   return check_launch(what);
+}
+
+// n calls with the same heads, head_dim, scale and strides, in as few launches
+// as their segments fit.  The first call's split workspace serves every launch.
+template <bool I8>
+int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, int n, void *stream) {
+  const char *what = I8 ? "tmhd_attn_fwd_i8qk" : "tmhd_attn_fwd_bf16";
+  if (n < 0 || (n > 0 && !args)) return set_error(TMHD_ERR_INVALID, "attention: null args");
+  KArgs k;
+  int nseg = 0;
+  auto reset = [&]() {
+    k = KArgs{};
+    k.qts = args->q_token_stride, k.qhs = args->q_head_stride;
+    k.ots = args->o_token_stride, k.ohs = args->o_head_stride;
+    k.heads = args->heads;
+    k.c = args->scale * kLog2e;
+    nseg = 0;
+  };
+  // every call is checked before the first launch
+  for (int i = 0; i < n; ++i) {
+    Prob P;
+    Seg seg[kMaxSeg];
+    if (int st = build_problem(args + i, I8 && qq ? qq + i : nullptr, I8, &P, seg)) return st;
+    if (args[i].heads != args->heads || args[i].head_dim != args->head_dim || args[i].scale != args->scale ||
+        args[i].q_token_stride != args->q_token_stride || args[i].q_head_stride != args->q_head_stride ||
+        args[i].o_token_stride != args->o_token_stride || args[i].o_head_stride != args->o_head_stride)
+      return set_error(TMHD_ERR_INVALID, "attention: the calls of a batch must share heads, head_dim, scale and strides");
+  }
+  if (n == 0) return TMHD_OK;
+  reset();
+  for (int i = 0; i < n; ++i) {
+    if (args[i].lq == 0) continue;
+    if (k.nprob == kMaxProb || nseg + args[i].n_segments > kMaxBatchSeg) {
+      if (int st = launch_group<I8>(k, nseg, args->head_dim, args->split_workspace, args->split_workspace_bytes,
+                                    (hipStream_t)stream, what))
+        return st;
+      reset();
+    }
+    Prob &P = k.pr[k.nprob];
+    if (int st = build_problem(args + i, I8 && qq ? qq + i : nullptr, I8, &P, k.seg + nseg)) return st;
+    P.seg0 = nseg;
+    nseg += args[i].n_segments;
+    P.seg_end = nseg;
+    ++k.nprob;
+  }
+  return launch_group<I8>(k, nseg, args->head_dim, args->split_workspace, args->split_workspace_bytes,
+                          (hipStream_t)stream, what);
 }
 
 // Device address of `scratch` on the current device, looked up once per
@@ -1647,10 +1799,11 @@ extern "C" int tmhd_attn_fwd_bf16_noalloc(const tmhd_attn_args *args, void *stre
   if (args->split_workspace)
     return set_error(TMHD_ERR_INVALID, "%s: split_workspace must be NULL (the library's static scratch is used)",
                      what);
-  KArgs k;
-  if (int st = build_kargs(args, nullptr, false, &k)) return st;
-  // any call's split needs at most one slot per CU of the device
-  const int64_t need = (int64_t)device_cus() * split_slot_bytes(args->head_dim);
+  Prob P;
+  Seg seg[kMaxSeg];
+  if (int st = build_problem(args, nullptr, false, &P, seg)) return st;
+  // any call's split needs at most two slots per CU of the device
+  const int64_t need = 2 * (int64_t)device_cus() * split_slot_bytes(args->head_dim);
   if (need > (int64_t)sizeof(scratch))
     return set_error(TMHD_ERR_UNSUPPORTED, "%s: %lld bytes of split scratch on this device exceed the static %lld",
                      what, (long long)need, (long long)sizeof(scratch));
@@ -1659,20 +1812,19 @@ extern "C" int tmhd_attn_fwd_bf16_noalloc(const tmhd_attn_args *args, void *stre
   tmhd_attn_args a = *args;
   a.split_workspace = ws;
   a.split_workspace_bytes = (int64_t)sizeof(scratch);
-  return launch_attn<false>(&a, nullptr, stream);
+  return launch_attn<false>(&a, nullptr, 1, stream);
 }
 
 extern "C" int64_t tmhd_attn_split_workspace_bytes(int32_t head_dim) {
   if (head_dim != 64 && head_dim != 128) return 0;
-  // the INT8-QK kernel runs two workgroups per CU, and its split round can
-  // take up to three sub-rounds of them
-  return 3 * 2 * (int64_t)tmhd::device_cus() * tmhd::split_slot_bytes(head_dim);
+  // two slots per resident workgroup; the INT8-QK kernel runs two per CU
+  return 2 * 2 * (int64_t)tmhd::device_cus() * tmhd::split_slot_bytes(head_dim);
 }
 
 extern "C" int tmhd_attn_fwd_bf16(const tmhd_attn_args *args, void *stream) {
-  return tmhd::launch_attn<false>(args, nullptr, stream);
+  return tmhd::launch_attn<false>(args, nullptr, 1, stream);
 }
 
 extern "C" int tmhd_attn_fwd_i8qk(const tmhd_attn_args *args, const tmhd_qk_quant *quant, void *stream) {
-  return tmhd::launch_attn<true>(args, quant, stream);
+  return tmhd::launch_attn<true>(args, quant, 1, stream);
 }
