@@ -1828,3 +1828,12 @@ extern "C" int tmhd_attn_fwd_bf16(const tmhd_attn_args *args, void *stream) {
 extern "C" int tmhd_attn_fwd_i8qk(const tmhd_attn_args *args, const tmhd_qk_quant *quant, void *stream) {
   return tmhd::launch_attn<true>(args, quant, 1, stream);
 }
+
+extern "C" int tmhd_attn_fwd_bf16_batch(const tmhd_attn_args *args, int32_t n, void *stream) {
+  return tmhd::launch_attn<false>(args, nullptr, n, stream);
+}
+
+extern "C" int tmhd_attn_fwd_i8qk_batch(const tmhd_attn_args *args, const tmhd_qk_quant *quant, int32_t n,
+                                        void *stream) {
+  return tmhd::launch_attn<true>(args, quant, n, stream);
+}

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "tmhd.h"
+#include "tmhd_batch.h"
 
 namespace tmhd {
 

@@ -2,6 +2,8 @@
 // INT8 quantization of the INT8-QK attention path.
 #include <math.h>
 
+#include <algorithm>
+
 #include "tmhd_internal.h"
 
 namespace tmhd {
@@ -12,7 +14,9 @@ constexpr int kTile = 64;
 // ---------------------------------------------------------------------------
 // tmhd_kv_pack: one workgroup = 64 slot positions of one head, D threads.
 // Position p of the slot is: data row (p - dst) if dst <= p < dst + n,
-// zero if dst + n <= p < zero_to, untouched otherwise.
+// zero if dst + n <= p < zero_to, untouched otherwise.  A launch packs up to
+// kMaxRanges row ranges: the 64-position blocks from blk0 on are range i's (one
+// launch per range instead cost 5 to 9 us each for ranges of 77 to 1,337 rows).
 // WITH_K false: the key rows of data positions are left to the caller (the
 // staged norm + RoPE kernel writes them); zero positions are still cleared.
 // Thread (dc, g) owns the 16-byte column chunk dc (columns 8 dc .. 8 dc + 7) of
@@ -20,14 +24,34 @@ constexpr int kTile = 64;
 // key and value chunks, copies the keys, and transposes the 8 x 8 block of
 // values in registers into 8 transposed rows of 8 positions. A wave's loads
 // and stores are whole 128-byte lines; no LDS and no barrier.
+constexpr int kMaxRanges = 32;
+struct PackRange {
+  const int32_t *rows;
+  int32_t row0, n, dst, zero_to;
+  int32_t p_begin;  // slot position of its first block
+  int32_t blk0;     // its first block in the launch
+};
+struct PackArgs {
+  const uint16_t *k, *v;
+  int64_t ts, hs;
+  uint16_t *ks, *vts;
+  int64_t khs, vhs;
+  int32_t vrs, nranges;
+  PackRange r[kMaxRanges];
+};
+
 template <int D, bool WITH_K = true>
-__global__ void __launch_bounds__(D) kv_pack_kernel(const uint16_t *__restrict__ k, const uint16_t *__restrict__ v,
-                                                    int64_t ts, int64_t hs, const int32_t *__restrict__ rows,
-                                                    int32_t row0, int32_t n, uint16_t *__restrict__ ks,
-                                                    uint16_t *__restrict__ vts, int64_t khs, int64_t vhs, int32_t vrs,
-                                                    int32_t dst, int32_t zero_to, int32_t p_begin) {
+__global__ void __launch_bounds__(D) kv_pack_kernel(const PackArgs a) {
+  int ri = 0;
+  while (ri + 1 < a.nranges && (int)blockIdx.x >= a.r[ri + 1].blk0) ++ri;
+  const PackRange &R = a.r[ri];
+  const uint16_t *__restrict__ k = a.k, *__restrict__ v = a.v;
+  const int32_t *__restrict__ rows = R.rows;
+  uint16_t *__restrict__ ks = a.ks, *__restrict__ vts = a.vts;
+  const int64_t ts = a.ts, hs = a.hs, khs = a.khs, vhs = a.vhs;
+  const int32_t vrs = a.vrs, row0 = R.row0, n = R.n, dst = R.dst, zero_to = R.zero_to;
   const int h = blockIdx.y;
-  const int p0 = p_begin + blockIdx.x * kTile;
+  const int p0 = R.p_begin + ((int)blockIdx.x - R.blk0) * kTile;
   const int dc = threadIdx.x >> 3, g = threadIdx.x & 7;
   int tok[8], kind[8];  // kind: 0 untouched, 1 data, 2 zero
   bool all = true, any = false;
@@ -99,18 +123,18 @@ __device__ __forceinline__ int64_t to_fixed(float x) {
   return (int64_t)__builtin_rintf(y);
 }
 
-// Key segments of one launch: workgroups [blk0[i], blk0[i + 1]) of the grid's
-// x dimension cover segment i (its own tokens, 256 per workgroup for the sums,
-// TMHD_QUANT_BLOCK for the blocks).
+// Limits of one smooth-quant launch: calls, and key segments over all of them.
+constexpr int kMaxCalls = 16, kMaxBatchSeg = 24;
+
+// Key segments whose sums a launch takes: workgroups [blk0[i], blk0[i + 1]) of
+// the grid's x dimension cover segment i, 256 of its tokens each.
 struct KeySegs {
-  const uint16_t *k[kMaxSeg];
-  int64_t khs[kMaxSeg];
-  int8_t *q8[kMaxSeg];
-  int64_t q8hs[kMaxSeg];
-  float *qs[kMaxSeg];
-  int32_t qshs[kMaxSeg];
-  int32_t tokens[kMaxSeg];
-  int32_t blk0[kMaxSeg + 1];
+  const uint16_t *k[kMaxBatchSeg];
+  int64_t khs[kMaxBatchSeg];
+  int64_t *part[kMaxBatchSeg];  // partial sums: block b of head h at part + h * part_hs + b * D
+  int64_t part_hs[kMaxBatchSeg];
+  int32_t tokens[kMaxBatchSeg];
+  int32_t blk0[kMaxBatchSeg + 1];
   int32_t n;
 };
 
@@ -124,9 +148,9 @@ __device__ __forceinline__ int key_seg(const KeySegs &a, int b) {
 // Thread (c, r) reads 16-byte chunk c (8 channels) of rows t0 + r, t0 + r + RPI, ...
 // (all its loads issued before any is used) and keeps 8 int64 partial sums;
 // partials are combined in LDS and added to ws[h][d] with one 64-bit atomic per
-// channel.  Values with |x| < 127 take the int32 conversion path; a chunk
+// channel, or (ATOMIC false) stored as the workgroup's partial sums.  Values with |x| < 127 take the int32 conversion path; a chunk
 // holding a larger value takes the int64 path (both give rint(x * 2^24) exactly).
-template <int D>
+template <int D, bool ATOMIC>
 __global__ void __launch_bounds__(256) k_sum_kernel(const KeySegs a, int64_t *__restrict__ ws) {
   constexpr int CPR = D / 8;      // 16-byte chunks per row
   constexpr int RPI = 256 / CPR;  // rows per pass
@@ -173,30 +197,70 @@ __global__ void __launch_bounds__(256) k_sum_kernel(const KeySegs a, int64_t *__
   if (tid < D) {
     long long sum = 0;
     for (int i = 0; i < RPI; ++i) sum += part[i][tid];
-    atomicAdd((unsigned long long *)(ws + h * D + tid), (unsigned long long)sum);
+    if constexpr (ATOMIC)
+      atomicAdd((unsigned long long *)(ws + h * D + tid), (unsigned long long)sum);
+    else
+      a.part[sg][h * a.part_hs[sg] + (int64_t)(blockIdx.x - a.blk0[sg]) * D + tid] = sum;
   }
 }
 
-// ws[i] = sum over the given per-segment key sums (0 when none are given)
-struct SumList {
-  const int64_t *p[kMaxSeg];
-  int32_t n;
+// The means of a batch of calls.  Segment i's sum is `given`, or the sum of its
+// nblk partial sums, which also goes to `out` if that is set (a later segment
+// may have it as `given`: both are read and written by the same thread).
+// Sums wrap, so their order does not matter.  One workgroup per head; group
+// r of its 512 / D takes partials r, r + 512 / D, ...  (Partial sums and this
+// kernel take the place of a zeroing launch, atomics, an initial sum and a
+// final division, and of one such chain for each segment whose sum is kept:
+// the 768p INT8-QK call with condition and padding rows spent 21 launches of 2
+// to 10 us on its quantization, and now spends 3.)
+struct MeanArgs {
+  const int64_t *given[kMaxBatchSeg];
+  const int64_t *part[kMaxBatchSeg];
+  int64_t part_hs[kMaxBatchSeg];
+  int64_t *out[kMaxBatchSeg];
+  int32_t nblk[kMaxBatchSeg];
+  int32_t call_seg0[kMaxCalls + 1];  // call c has segments [call_seg0[c], call_seg0[c + 1])
+  uint16_t *mean[kMaxCalls];
+  double count[kMaxCalls];           // keys of the call
+  int32_t ncalls;
 };
-__global__ void init_sum_kernel(int64_t *__restrict__ ws, const SumList l, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    unsigned long long acc = 0;  // wrapping sum: the same as the atomics' (associative modulo 2^64)
-    for (int s = 0; s < l.n; ++s) acc += (unsigned long long)l.p[s][i];
-    ws[i] = (int64_t)acc;
-  }
-}
-
-__global__ void k_mean_finalize_kernel(const int64_t *__restrict__ ws, uint16_t *__restrict__ mean, int n,
-                                       double count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    const double m = __ddiv_rn((double)ws[i], count * kMeanFix);
-    mean[i] = f32_to_bf16_bits((float)m);
+template <int D>
+__global__ void __launch_bounds__(512) k_mean_kernel(const MeanArgs a) {
+  constexpr int G = 512 / D;
+  __shared__ unsigned long long part[G][D];
+  const int h = blockIdx.x, d = threadIdx.x % D, r = threadIdx.x / D;
+  for (int c = 0; c < a.ncalls; ++c) {
+    unsigned long long acc = 0;
+    for (int s = a.call_seg0[c]; s < a.call_seg0[c + 1]; ++s) {
+      if (a.given[s]) {
+        if (r == 0) acc += (unsigned long long)a.given[s][h * D + d];
+        continue;
+      }
+      const int64_t *p = a.part[s] + h * a.part_hs[s] + d;
+      unsigned long long sum = 0;
+      int b = r;
+      for (; b + 7 * G < a.nblk[s]; b += 8 * G) {
+        int64_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = p[(int64_t)(b + i * G) * D];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum += (unsigned long long)x[i];
+      }
+      for (; b < a.nblk[s]; b += G) sum += (unsigned long long)p[(int64_t)b * D];
+      __syncthreads();  // the previous segment's reads
+      part[r][d] = sum;
+      __syncthreads();
+      if (r == 0) {
+#pragma unroll
+        for (int i = 1; i < G; ++i) sum += part[i][d];
+        if (a.out[s]) a.out[s][h * D + d] = (int64_t)sum;
+        acc += sum;
+      }
+    }
+    if (r == 0) {
+      const double m = __ddiv_rn((double)(int64_t)acc, a.count[c] * kMeanFix);
+      a.mean[c][h * D + d] = f32_to_bf16_bits((float)m);
+    }
   }
 }
 
@@ -273,88 +337,95 @@ __device__ __forceinline__ void quant_block(const uint16_t *__restrict__ src, in
   }
 }
 
-template <int D>
-__global__ void __launch_bounds__(256) block_quant_kernel(const uint16_t *__restrict__ src, int64_t sts, int64_t shs,
-                                                          const int32_t *__restrict__ rows, int32_t row0,
-                                                          const uint16_t *__restrict__ mean, int32_t nvalid,
-                                                          int32_t nwrite, int8_t *__restrict__ q8, int64_t q8hs,
-                                                          float *__restrict__ qscale, int32_t qshs) {
-  if (mean)
-    quant_block<D, true>(src, sts, shs, rows, row0, mean, nvalid, nwrite, q8, q8hs, qscale, qshs, blockIdx.y, blockIdx.x);
-  else
-    quant_block<D, false>(src, sts, shs, rows, row0, mean, nvalid, nwrite, q8, q8hs, qscale, qshs, blockIdx.y,
-                          blockIdx.x);
-}
+// Every key segment's and every call's query blocks of a batch in one launch:
+// workgroups from blk0[i] on are entry i's.
+struct QuantEntry {
+  const uint16_t *src;
+  int64_t sts, shs;
+  const int32_t *rows;   // queries: their row list, or row0
+  const uint16_t *mean;  // keys: [H][D]; queries: nullptr
+  int8_t *q8;
+  int64_t q8hs;
+  float *qs;
+  int32_t qshs, row0, nvalid, nwrite, blk0;
+};
+struct QuantArgs {
+  int32_t n;
+  QuantEntry e[kMaxBatchSeg + kMaxCalls];
+};
+static_assert(sizeof(QuantArgs) <= 4096, "kernel arguments");
 
-// Every key segment's blocks in one launch (slot rows: token stride D); rows up
-// to the 64-token tile padding are written.
 template <int D>
-__global__ void __launch_bounds__(256) key_block_quant_kernel(const KeySegs a, const uint16_t *__restrict__ mean) {
-  const int sg = key_seg(a, blockIdx.x);
-  const int nwrite = (a.tokens[sg] + kTile - 1) / kTile * kTile;
-  quant_block<D, true>(a.k[sg], D, a.khs[sg], nullptr, 0, mean, a.tokens[sg], nwrite, a.q8[sg], a.q8hs[sg], a.qs[sg],
-                       a.qshs[sg], blockIdx.y, blockIdx.x - a.blk0[sg]);
+__global__ void __launch_bounds__(256) block_quant_kernel(const QuantArgs a) {
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.e[i + 1].blk0) ++i;
+  const QuantEntry &E = a.e[i];
+  const int blk = blockIdx.x - E.blk0;
+  if (E.mean)
+    quant_block<D, true>(E.src, E.sts, E.shs, nullptr, 0, E.mean, E.nvalid, E.nwrite, E.q8, E.q8hs, E.qs, E.qshs,
+                         blockIdx.y, blk);
+  else
+    quant_block<D, false>(E.src, E.sts, E.shs, E.rows, E.row0, nullptr, E.nvalid, E.nwrite, E.q8, E.q8hs, E.qs, E.qshs,
+                          blockIdx.y, blk);
 }
 
 bool aligned(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
+// Calls [0, n) of a batch (within the launch limits): key sums, means, then
+// every key and query block.  sum_out: per call kMaxSeg pointers, or nullptr.
 template <int D>
-int launch_block_quant(const uint16_t *src, int64_t sts, int64_t shs, const int32_t *rows, int32_t row0,
-                       const uint16_t *mean, int32_t nvalid, int32_t nwrite, int8_t *q8, int64_t q8hs, float *qs,
-                       int32_t qshs, int heads, hipStream_t s) {
-  const int nblk = (nwrite + TMHD_QUANT_BLOCK - 1) / TMHD_QUANT_BLOCK;
-  if (nblk == 0) return TMHD_OK;
-  hipLaunchKernelGGL(block_quant_kernel<D>, dim3(nblk, heads), dim3(256), 0, s, src, sts, shs, rows, row0, mean,
-                     nvalid, nwrite, q8, q8hs, qs, qshs);
-  return check_launch("block_quant");
-}
-
-template <int D>
-int smooth_quant(const tmhd_attn_args *a, const tmhd_qk_quant *qq, hipStream_t s) {
+int smooth_quant(const tmhd_attn_args *a, const tmhd_qk_quant *qq, int64_t *const *sum_out, int n, hipStream_t s) {
   const int H = a->heads;
-  int64_t total = 0;
-  for (int i = 0; i < a->n_segments; ++i) total += a->seg[i].tokens;
-  // 1. exact key sums, 2. bf16 mean
-  // one segment table for the key passes; workgroup ranges per pass
-  KeySegs ks{}, sums{};
-  SumList given{};
-  ks.n = a->n_segments;
-  for (int i = 0; i < a->n_segments; ++i) {
-    const tmhd_kv_segment &sg = a->seg[i];
-    ks.k[i] = (const uint16_t *)sg.k;
-    ks.khs[i] = sg.k_head_stride;
-    ks.q8[i] = qq->k_i8[i];
-    ks.q8hs[i] = qq->k_head_stride[i];
-    ks.qs[i] = qq->k_scale[i];
-    ks.qshs[i] = qq->k_scale_head_stride[i];
-    ks.tokens[i] = sg.tokens;
-    if (qq->k_sum[i]) {  // exact sums given by the caller (tmhd_k_fixed_sum)
-      given.p[given.n++] = qq->k_sum[i];
-    } else {
-      sums.k[sums.n] = ks.k[i];
-      sums.khs[sums.n] = ks.khs[i];
-      sums.tokens[sums.n++] = sg.tokens;
+  KeySegs ks{};
+  MeanArgs mean{};
+  QuantArgs quant{};
+  int nseg = 0, qblocks = 0;
+  mean.ncalls = n;
+  for (int c = 0; c < n; ++c) {
+    mean.call_seg0[c] = nseg;
+    mean.mean[c] = qq[c].k_mean;
+    for (int i = 0; i < a[c].n_segments; ++i, ++nseg) {
+      const tmhd_kv_segment &sg = a[c].seg[i];
+      mean.count[c] += (double)sg.tokens;
+      mean.given[nseg] = qq[c].k_sum[i];
+      if (!qq[c].k_sum[i]) {
+        // the quantized keys' own rows hold the partial sums until they are written:
+        // D int64 per 256 tokens in the cap * D bytes of a head
+        int64_t *part = (int64_t *)qq[c].k_i8[i];
+        const int64_t part_hs = qq[c].k_head_stride[i] / 8;
+        mean.part[nseg] = ks.part[ks.n] = part;
+        mean.part_hs[nseg] = ks.part_hs[ks.n] = part_hs;
+        mean.nblk[nseg] = (sg.tokens + 255) / 256;
+        mean.out[nseg] = sum_out ? sum_out[c * kMaxSeg + i] : nullptr;
+        ks.k[ks.n] = (const uint16_t *)sg.k;
+        ks.khs[ks.n] = sg.k_head_stride;
+        ks.tokens[ks.n] = sg.tokens;
+        ks.blk0[ks.n + 1] = ks.blk0[ks.n] + mean.nblk[nseg];
+        ++ks.n;
+      }
+      // rows up to the 64-token tile padding are written
+      QuantEntry &e = quant.e[quant.n++];
+      const int nwrite = (sg.tokens + kTile - 1) / kTile * kTile;
+      e = QuantEntry{(const uint16_t *)sg.k, D, sg.k_head_stride, nullptr, qq[c].k_mean, qq[c].k_i8[i],
+                     qq[c].k_head_stride[i], qq[c].k_scale[i], qq[c].k_scale_head_stride[i], 0, sg.tokens, nwrite,
+                     qblocks};
+      qblocks += (nwrite + TMHD_QUANT_BLOCK - 1) / TMHD_QUANT_BLOCK;
     }
+    // queries: rows up to the 256-row workgroup padding are written
+    const int qcap = (a[c].lq + 255) / 256 * 256;
+    if (qcap == 0) continue;
+    quant.e[quant.n++] = QuantEntry{(const uint16_t *)a[c].q, a[c].q_token_stride, a[c].q_head_stride, a[c].q_rows,
+                                    nullptr, qq[c].q_i8, qq[c].q_head_stride, qq[c].q_scale,
+                                    qq[c].q_scale_head_stride, a[c].q_row0, a[c].lq, qcap, qblocks};
+    qblocks += qcap / TMHD_QUANT_BLOCK;
   }
-  auto ranges = [](KeySegs &t, int per) {
-    t.blk0[0] = 0;
-    for (int i = 0; i < t.n; ++i) t.blk0[i + 1] = t.blk0[i] + (t.tokens[i] + per - 1) / per;
-    return t.blk0[t.n];
-  };
-  hipLaunchKernelGGL(init_sum_kernel, dim3((H * D + 255) / 256), dim3(256), 0, s, qq->mean_workspace, given, H * D);
-  if (sums.n) hipLaunchKernelGGL(k_sum_kernel<D>, dim3(ranges(sums, 256), H), dim3(256), 0, s, sums, qq->mean_workspace);
-  hipLaunchKernelGGL(k_mean_finalize_kernel, dim3((H * D + 255) / 256), dim3(256), 0, s, qq->mean_workspace,
-                     qq->k_mean, H * D, (double)total);
+  mean.call_seg0[n] = nseg;
+  if (ks.n)
+    hipLaunchKernelGGL((k_sum_kernel<D, false>), dim3(ks.blk0[ks.n], H), dim3(256), 0, s, ks, (int64_t *)nullptr);
+  hipLaunchKernelGGL(k_mean_kernel<D>, dim3(H), dim3(512), 0, s, mean);
   if (int st = check_launch("smooth-K mean")) return st;
-  // 3. keys, every segment in one launch (rows up to the 64-token tile padding are written)
-  const int nblk = ranges(ks, TMHD_QUANT_BLOCK);
-  hipLaunchKernelGGL(key_block_quant_kernel<D>, dim3(nblk, H), dim3(256), 0, s, ks, (const uint16_t *)qq->k_mean);
-  if (int st = check_launch("block_quant keys")) return st;
-  // 4. queries (rows up to the 256-row workgroup padding are written)
-  const int qcap = (a->lq + 255) / 256 * 256;
-  return launch_block_quant<D>((const uint16_t *)a->q, a->q_token_stride, a->q_head_stride, a->q_rows, a->q_row0,
-                               nullptr, a->lq, qcap, qq->q_i8, qq->q_head_stride, qq->q_scale,
-                               qq->q_scale_head_stride, H, s);
+  hipLaunchKernelGGL(block_quant_kernel<D>, dim3(qblocks, H), dim3(256), 0, s, quant);
+  return check_launch("block_quant");
 }
 
 }  // namespace
@@ -362,43 +433,77 @@ int smooth_quant(const tmhd_attn_args *a, const tmhd_qk_quant *qq, hipStream_t s
 
 namespace tmhd {
 
+int kv_pack_ranges(const void *k, const void *v, int64_t token_stride, int64_t head_stride,
+                   const tmhd_pack_range *ranges, int32_t nranges, void *k_slot, void *vt_slot, int64_t k_head_stride,
+                   int64_t vt_head_stride, int32_t vt_row_stride, int32_t heads, int32_t head_dim, void *stream,
+                   bool with_k, bool check_only) {
+  if (head_dim != 64 && head_dim != 128) return set_error(TMHD_ERR_UNSUPPORTED, "kv_pack: head_dim %d", head_dim);
+  if (nranges < 0 || (nranges > 0 && !ranges)) return set_error(TMHD_ERR_INVALID, "kv_pack: %d ranges", nranges);
+  bool data = false;
+  for (int i = 0; i < nranges; ++i) {
+    const tmhd_pack_range &r = ranges[i];
+    if (r.n < 0 || r.dst < 0 || heads <= 0)
+      return set_error(TMHD_ERR_INVALID, "kv_pack: n %d dst %d heads %d", r.n, r.dst, heads);
+    const int64_t end = std::max((int64_t)r.dst + r.n, (int64_t)r.zero_to);
+    const int64_t p_begin = r.dst / kTile * kTile;
+    const int64_t p_end = (end + kTile - 1) / kTile * kTile;
+    if (p_end > vt_row_stride || vt_row_stride % kTile || (int64_t)vt_row_stride * head_dim > vt_head_stride ||
+        p_end * head_dim > k_head_stride)
+      return set_error(TMHD_ERR_INVALID, "kv_pack: positions [%lld, %lld) exceed the slot (cap %d)",
+                       (long long)p_begin, (long long)p_end, vt_row_stride);
+    data = data || r.n > 0;
+  }
+  if ((data && (!k || !v)) || !k_slot || !vt_slot || !aligned(k_slot, 16) || !aligned(vt_slot, 16) ||
+      (data && (!aligned(k, 16) || !aligned(v, 16))) || token_stride % 8 || head_stride % 8 || k_head_stride % 8 ||
+      vt_head_stride % 8)
+    return set_error(TMHD_ERR_INVALID, "kv_pack: pointers and strides must be 16-byte aligned");
+  if (check_only) return TMHD_OK;
+  PackArgs a{(const uint16_t *)k, (const uint16_t *)v, token_stride, head_stride, (uint16_t *)k_slot,
+             (uint16_t *)vt_slot, k_head_stride, vt_head_stride, vt_row_stride, 0, {}};
+  for (int i = 0, blocks = 0; i < nranges; ++i) {
+    const tmhd_pack_range &r = ranges[i];
+    const int p_begin = r.dst / kTile * kTile, end = std::max(r.dst + r.n, r.zero_to);
+    const int nblk = ((end + kTile - 1) / kTile * kTile - p_begin) / kTile;
+    if (nblk > 0) {
+      a.r[a.nranges++] = PackRange{r.rows, r.row0, r.n, r.dst, r.zero_to, p_begin, blocks};
+      blocks += nblk;
+    }
+    if (blocks == 0 || (a.nranges < kMaxRanges && i + 1 < nranges)) continue;
+    const dim3 grid(blocks, heads);
+    hipStream_t s = (hipStream_t)stream;
+    if (head_dim == 128 && with_k)
+      hipLaunchKernelGGL((kv_pack_kernel<128, true>), grid, dim3(128), 0, s, a);
+    else if (head_dim == 128)
+      hipLaunchKernelGGL((kv_pack_kernel<128, false>), grid, dim3(128), 0, s, a);
+    else if (with_k)
+      hipLaunchKernelGGL((kv_pack_kernel<64, true>), grid, dim3(64), 0, s, a);
+    else
+      hipLaunchKernelGGL((kv_pack_kernel<64, false>), grid, dim3(64), 0, s, a);
+    if (int st = check_launch("tmhd_kv_pack")) return st;
+    a.nranges = 0;
+    blocks = 0;
+  }
+  return TMHD_OK;
+}
+
 int kv_pack(const void *k, const void *v, int64_t token_stride, int64_t head_stride, const int32_t *rows,
             int32_t row0, int32_t n, void *k_slot, void *vt_slot, int64_t k_head_stride, int64_t vt_head_stride,
             int32_t vt_row_stride, int32_t dst, int32_t zero_to, int32_t heads, int32_t head_dim, void *stream,
             bool with_k, bool check_only) {
-  if (head_dim != 64 && head_dim != 128) return set_error(TMHD_ERR_UNSUPPORTED, "kv_pack: head_dim %d", head_dim);
-  if (n < 0 || dst < 0 || heads <= 0) return set_error(TMHD_ERR_INVALID, "kv_pack: n %d dst %d heads %d", n, dst, heads);
-  const int end = max(dst + n, zero_to);
-  const int p_begin = dst / kTile * kTile;
-  const int p_end = (end + kTile - 1) / kTile * kTile;
-  if (p_end > vt_row_stride || vt_row_stride % kTile || (int64_t)vt_row_stride * head_dim > vt_head_stride ||
-      (int64_t)p_end * head_dim > k_head_stride)
-    return set_error(TMHD_ERR_INVALID, "kv_pack: positions [%d, %d) exceed the slot (cap %d)", p_begin, p_end,
-                     vt_row_stride);
-  if ((n > 0 && (!k || !v)) || !k_slot || !vt_slot || !aligned(k_slot, 16) || !aligned(vt_slot, 16) ||
-      (n > 0 && (!aligned(k, 16) || !aligned(v, 16))) || token_stride % 8 || head_stride % 8 || k_head_stride % 8 ||
-      vt_head_stride % 8)
-    return set_error(TMHD_ERR_INVALID, "kv_pack: pointers and strides must be 16-byte aligned");
-  if (check_only || p_end == p_begin) return TMHD_OK;
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((p_end - p_begin) / kTile, heads);
-#define TMHD_PACK(DIM, WK)                                                                                      \
-  hipLaunchKernelGGL((kv_pack_kernel<DIM, WK>), grid, dim3(DIM), 0, s, (const uint16_t *)k, (const uint16_t *)v, \
-                     token_stride, head_stride, rows, row0, n, (uint16_t *)k_slot, (uint16_t *)vt_slot,          \
-                     k_head_stride, vt_head_stride, vt_row_stride, dst, zero_to, p_begin)
-  if (head_dim == 128 && with_k)
-    TMHD_PACK(128, true);
-  else if (head_dim == 128)
-    TMHD_PACK(128, false);
-  else if (with_k)
-    TMHD_PACK(64, true);
-  else
-    TMHD_PACK(64, false);
-#undef TMHD_PACK
-  return check_launch("tmhd_kv_pack");
+  const tmhd_pack_range r{rows, row0, n, dst, zero_to};
+  return kv_pack_ranges(k, v, token_stride, head_stride, &r, 1, k_slot, vt_slot, k_head_stride, vt_head_stride,
+                        vt_row_stride, heads, head_dim, stream, with_k, check_only);
 }
 
 }  // namespace tmhd
+
+extern "C" int tmhd_kv_pack_ranges(const void *k, const void *v, int64_t token_stride, int64_t head_stride,
+                                   const tmhd_pack_range *ranges, int32_t n_ranges, void *k_slot, void *vt_slot,
+                                   int64_t k_head_stride, int64_t vt_head_stride, int32_t vt_row_stride,
+                                   int32_t heads, int32_t head_dim, void *stream) {
+  return tmhd::kv_pack_ranges(k, v, token_stride, head_stride, ranges, n_ranges, k_slot, vt_slot, k_head_stride,
+                              vt_head_stride, vt_row_stride, heads, head_dim, stream, true, false);
+}
 
 extern "C" int tmhd_kv_pack(const void *k, const void *v, int64_t token_stride, int64_t head_stride,
                             const int32_t *rows, int32_t row0, int32_t n, void *k_slot, void *vt_slot,
@@ -408,9 +513,11 @@ extern "C" int tmhd_kv_pack(const void *k, const void *v, int64_t token_stride, 
                        vt_row_stride, dst, zero_to, heads, head_dim, stream, true, false);
 }
 
-extern "C" int tmhd_qk_smooth_quant(const tmhd_attn_args *args, const tmhd_qk_quant *quant, void *stream) {
-  using namespace tmhd;
-  if (!args || !quant) return set_error(TMHD_ERR_INVALID, "smooth_quant: null arguments");
+namespace tmhd {
+namespace {
+
+// Checks one call of the smooth quantization.
+int check_smooth_quant(const tmhd_attn_args *args, const tmhd_qk_quant *quant) {
   const int D = args->head_dim;
   if (D != 64 && D != 128) return set_error(TMHD_ERR_UNSUPPORTED, "smooth_quant: head_dim %d", D);
   if (args->n_segments < 1 || args->n_segments > kMaxSeg || args->heads <= 0 || args->lq < 0)
@@ -437,8 +544,45 @@ extern "C" int tmhd_qk_smooth_quant(const tmhd_attn_args *args, const tmhd_qk_qu
         quant->k_scale_head_stride[i] < (sg.tokens + TMHD_QUANT_BLOCK - 1) / TMHD_QUANT_BLOCK)
       return set_error(TMHD_ERR_INVALID, "smooth_quant: segment %d quantized key buffers too small", i);
   }
+  return TMHD_OK;
+}
+
+int smooth_quant_batch(const tmhd_attn_args *args, const tmhd_qk_quant *quant, int64_t *const *sum_out, int32_t n,
+                       void *stream) {
+  if (n < 0 || (n > 0 && (!args || !quant))) return set_error(TMHD_ERR_INVALID, "smooth_quant: null arguments");
+  // every call is checked before the first launch
+  for (int i = 0; i < n; ++i) {
+    if (int st = check_smooth_quant(args + i, quant + i)) return st;
+    if (args[i].heads != args->heads || args[i].head_dim != args->head_dim)
+      return set_error(TMHD_ERR_INVALID, "smooth_quant: the calls of a batch must share heads and head_dim");
+    for (int j = 0; sum_out && j < args[i].n_segments; ++j)
+      if (sum_out[i * kMaxSeg + j] && !aligned(sum_out[i * kMaxSeg + j], 8))
+        return set_error(TMHD_ERR_INVALID, "smooth_quant: segment %d key sums must be 8-byte aligned", j);
+  }
   hipStream_t s = (hipStream_t)stream;
-  return D == 128 ? smooth_quant<128>(args, quant, s) : smooth_quant<64>(args, quant, s);
+  for (int i = 0; i < n;) {
+    int m = 0, segs = 0;
+    while (i + m < n && m < kMaxCalls && segs + args[i + m].n_segments <= kMaxBatchSeg) segs += args[i + m++].n_segments;
+    int64_t *const *so = sum_out ? sum_out + i * kMaxSeg : nullptr;
+    if (int st = args->head_dim == 128 ? smooth_quant<128>(args + i, quant + i, so, m, s)
+                                       : smooth_quant<64>(args + i, quant + i, so, m, s))
+      return st;
+    i += m;
+  }
+  return TMHD_OK;
+}
+
+}  // namespace
+}  // namespace tmhd
+
+extern "C" int tmhd_qk_smooth_quant(const tmhd_attn_args *args, const tmhd_qk_quant *quant, void *stream) {
+  if (!args || !quant) return tmhd::set_error(TMHD_ERR_INVALID, "smooth_quant: null arguments");
+  return tmhd::smooth_quant_batch(args, quant, nullptr, 1, stream);
+}
+
+extern "C" int tmhd_qk_smooth_quant_batch(const tmhd_attn_args *args, const tmhd_qk_quant *quant,
+                                          int64_t *const *k_sum_out, int32_t n, void *stream) {
+  return tmhd::smooth_quant_batch(args, quant, k_sum_out, n, stream);
 }
 
 extern "C" int tmhd_k_fixed_sum(const void *k, int64_t k_head_stride, int32_t tokens, int32_t heads, int32_t head_dim,
@@ -460,8 +604,8 @@ extern "C" int tmhd_k_fixed_sum(const void *k, int64_t k_head_stride, int32_t to
   t.blk0[1] = (tokens + 255) / 256;
   hipLaunchKernelGGL(zero_i64_kernel, dim3((heads * head_dim + 255) / 256), dim3(256), 0, s, sum, heads * head_dim);
   if (head_dim == 128)
-    hipLaunchKernelGGL(k_sum_kernel<128>, dim3(t.blk0[1], heads), dim3(256), 0, s, t, sum);
+    hipLaunchKernelGGL((k_sum_kernel<128, true>), dim3(t.blk0[1], heads), dim3(256), 0, s, t, sum);
   else
-    hipLaunchKernelGGL(k_sum_kernel<64>, dim3(t.blk0[1], heads), dim3(256), 0, s, t, sum);
+    hipLaunchKernelGGL((k_sum_kernel<64, true>), dim3(t.blk0[1], heads), dim3(256), 0, s, t, sum);
   return check_launch("tmhd_k_fixed_sum");
 }

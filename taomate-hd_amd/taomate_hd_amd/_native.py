@@ -1,4 +1,4 @@
-"""ctypes binding of libtmhd.so (the C ABI declared in include/tmhd.h).
+"""ctypes binding of libtmhd.so (the C ABI declared in include/tmhd.h and tmhd_batch.h).
 
 The library is the only compute path of this package: every operator raises
 if it is not built or no GPU is present.  There is no CPU fallback.
@@ -72,6 +72,16 @@ class QKQuant(ctypes.Structure):
         ("k_mean", c_void_p),
         ("mean_workspace", c_void_p),
         ("k_sum", c_void_p * MAX_SEGMENTS),
+    ]
+
+
+class PackRange(ctypes.Structure):
+    _fields_ = [
+        ("rows", c_void_p),
+        ("row0", c_int32),
+        ("n", c_int32),
+        ("dst", c_int32),
+        ("zero_to", c_int32),
     ]
 
 
@@ -189,7 +199,23 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     ),
 }
 
-EXPORTED_SYMBOLS = tuple(_SIGNATURES)
+# include/tmhd_batch.h
+_BATCH_SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
+    "tmhd_attn_fwd_bf16_batch": (c_int, [POINTER(AttnArgs), c_int32, c_void_p]),
+    "tmhd_attn_fwd_i8qk_batch": (c_int, [POINTER(AttnArgs), POINTER(QKQuant), c_int32, c_void_p]),
+    "tmhd_qk_smooth_quant_batch": (
+        c_int, [POINTER(AttnArgs), POINTER(QKQuant), POINTER(c_void_p), c_int32, c_void_p],
+    ),
+    "tmhd_kv_pack_ranges": (
+        c_int,
+        [
+            c_void_p, c_void_p, c_int64, c_int64, POINTER(PackRange), c_int32,
+            c_void_p, c_void_p, c_int64, c_int64, c_int32, c_int32, c_int32, c_void_p,
+        ],
+    ),
+}
+
+EXPORTED_SYMBOLS = tuple(_SIGNATURES)  # of include/tmhd.h
 
 _lock = threading.Lock()
 _lib: ctypes.CDLL | None = None
@@ -208,7 +234,7 @@ def load() -> ctypes.CDLL:
                     "(hipcc --offload-arch=gfx950) before using the HIP operators"
                 )
             lib = ctypes.CDLL(str(LIB_PATH))
-            for name, (restype, argtypes) in _SIGNATURES.items():
+            for name, (restype, argtypes) in (*_SIGNATURES.items(), *_BATCH_SIGNATURES.items()):
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes
@@ -246,7 +272,12 @@ def require_same_gpu(torch: Any, device: Any, **tensors: Any) -> None:
 
 
 def stream_ptr(torch: Any, device: Any) -> int:
-    return int(torch.cuda.current_stream(device=device).cuda_stream)
+    """Handle of the current stream on ``device`` (read directly: a Stream object
+    costs 2 us, and a hook call asks several times)."""
+    index = getattr(device, "index", None)
+    if index is None:
+        index = torch.device(device).index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(tensor: Any) -> int:

@@ -11,6 +11,8 @@ ref attention_hook.py:335-371, inference/sage_value_padding.py:79-97).
 
 from __future__ import annotations
 
+import ctypes
+from dataclasses import dataclass
 from typing import Any, Sequence
 
 from . import _native
@@ -47,47 +49,66 @@ class QKQuantWorkspace:
         return buf
 
     def quant_struct(self, *, heads: int, head_dim: int, lq: int, tokens: Sequence[int], device: Any) -> tuple[Any, dict[str, Any]]:
+        structs, views = self.quant_structs(heads=heads, head_dim=head_dim, calls=[(lq, tokens)], device=device,
+                                            with_views=True)
+        return structs[0], views[0]
+
+    def quant_structs(self, *, heads: int, head_dim: int, calls: Sequence[tuple[int, Sequence[int]]], device: Any,
+                      with_views: bool = False) -> tuple[Any, list[dict[str, Any]]]:
+        """The operands of ``calls`` (query rows, segment tokens) side by side in
+        this stream's buffers: an array of structs, and with ``with_views`` a
+        dict of tensors per call."""
         torch = self._torch
         key = (str(device), _native.stream_ptr(torch, device))
         store = self._buffers.setdefault(key, {})
-        qcap = round_up(max(lq, 1), _native.QUERY_TILE)
-        caps = [round_up(t, KV_TILE) for t in tokens]
-        nblk = [round_up(c, _native.QUANT_BLOCK) // _native.QUANT_BLOCK for c in caps]
-        # 256-byte aligned carve-out offsets inside one int8 buffer and one fp32 buffer
-        k_off, total = [], 0
-        for c in caps:
-            k_off.append(total)
-            total += round_up(heads * c * head_dim, 256)
-        s_off, stotal = [], 0
-        for b in nblk:
-            s_off.append(stotal)
-            stotal += round_up(heads * b, 64)
-        q_i8 = self._grow(store, "q_i8", heads * qcap * head_dim, torch.int8, device)
-        q_scale = self._grow(store, "q_scale", heads * (qcap // _native.QUANT_BLOCK), torch.float32, device)
-        k_i8 = self._grow(store, "k_i8", total, torch.int8, device)
-        k_scale = self._grow(store, "k_scale", stotal, torch.float32, device)
-        k_mean = self._grow(store, "k_mean", heads * head_dim, torch.bfloat16, device)
-        ws = self._grow(store, "mean_ws", heads * head_dim, torch.int64, device)
-        qq = _native.QKQuant()
-        qq.q_i8 = _native.ptr(q_i8)
-        qq.q_scale = _native.ptr(q_scale)
-        qq.q_head_stride = qcap * head_dim
-        qq.q_scale_head_stride = qcap // _native.QUANT_BLOCK
-        for i, c in enumerate(caps):
-            qq.k_i8[i] = _native.ptr(k_i8) + k_off[i]
-            qq.k_scale[i] = _native.ptr(k_scale) + 4 * s_off[i]
-            qq.k_head_stride[i] = c * head_dim
-            qq.k_scale_head_stride[i] = nblk[i]
-        qq.k_mean = _native.ptr(k_mean)
-        qq.mean_workspace = _native.ptr(ws)
-        views = {
-            "q_i8": q_i8[: heads * qcap * head_dim].view(heads, qcap, head_dim),
-            "q_scale": q_scale[: heads * (qcap // _native.QUANT_BLOCK)].view(heads, -1),
-            "k_mean": k_mean[: heads * head_dim].view(heads, head_dim),
-            "k_i8": [k_i8[o : o + heads * c * head_dim].view(heads, c, head_dim) for o, c in zip(k_off, caps)],
-            "k_scale": [k_scale[o : o + heads * b].view(heads, b) for o, b in zip(s_off, nblk)],
-        }
-        return qq, views
+        # 256-byte aligned carve-out offsets inside the int8 and fp32 buffers
+        plan, q_total, qs_total, k_total, ks_total = [], 0, 0, 0, 0
+        for lq, tokens in calls:
+            qcap = round_up(max(lq, 1), _native.QUERY_TILE)
+            segs = []
+            for t in tokens:
+                cap = round_up(t, KV_TILE)
+                nblk = round_up(cap, _native.QUANT_BLOCK) // _native.QUANT_BLOCK
+                segs.append((cap, nblk, k_total, ks_total))
+                k_total += round_up(heads * cap * head_dim, 256)
+                ks_total += round_up(heads * nblk, 64)
+            plan.append((qcap, q_total, qs_total, segs))
+            q_total += heads * qcap * head_dim
+            qs_total += round_up(heads * (qcap // _native.QUANT_BLOCK), 64)
+        n = len(plan)
+        width = heads * head_dim
+        q_i8 = self._grow(store, "q_i8", q_total, torch.int8, device)
+        q_scale = self._grow(store, "q_scale", qs_total, torch.float32, device)
+        k_i8 = self._grow(store, "k_i8", k_total, torch.int8, device)
+        k_scale = self._grow(store, "k_scale", ks_total, torch.float32, device)
+        k_mean = self._grow(store, "k_mean", n * width, torch.bfloat16, device)
+        ws = self._grow(store, "mean_ws", width, torch.int64, device)
+        q_at, qs_at, k_at, ks_at, mean_at = (_native.ptr(t) for t in (q_i8, q_scale, k_i8, k_scale, k_mean))
+        ws_at = _native.ptr(ws)
+        structs = (_native.QKQuant * n)()
+        views = []
+        for i, (qcap, q_off, qs_off, segs) in enumerate(plan):
+            qq = structs[i]
+            qq.q_i8 = q_at + q_off
+            qq.q_scale = qs_at + 4 * qs_off
+            qq.q_head_stride = qcap * head_dim
+            qq.q_scale_head_stride = qcap // _native.QUANT_BLOCK
+            for j, (cap, nblk, k_off, s_off) in enumerate(segs):
+                qq.k_i8[j] = k_at + k_off
+                qq.k_scale[j] = ks_at + 4 * s_off
+                qq.k_head_stride[j] = cap * head_dim
+                qq.k_scale_head_stride[j] = nblk
+            qq.k_mean = mean_at + 2 * i * width
+            qq.mean_workspace = ws_at
+            if with_views:
+                views.append({
+                    "q_i8": q_i8[q_off : q_off + heads * qcap * head_dim].view(heads, qcap, head_dim),
+                    "q_scale": q_scale[qs_off : qs_off + heads * (qcap // _native.QUANT_BLOCK)].view(heads, -1),
+                    "k_mean": k_mean[i * width : (i + 1) * width].view(heads, head_dim),
+                    "k_i8": [k_i8[o : o + heads * c * head_dim].view(heads, c, head_dim) for c, _, o, _ in segs],
+                    "k_scale": [k_scale[o : o + heads * b].view(heads, b) for _, b, _, o in segs],
+                })
+        return structs, views
 
 
 _SPLIT_WORKSPACES: dict[tuple[Any, ...], Any] = {}
@@ -141,21 +162,21 @@ def _row_list(torch: Any, rows: Any, device: Any, limit: int, name: str, checked
     return rows.to(torch.int32).contiguous()
 
 
-def _key_sum(torch: Any, lib: Any, view: SlotView, stream: int) -> int:
-    """Device address of the exact fixed-point key sums of a slot view (the
-    smooth-K mean's term for that segment), memoised on the slot per (row0,
-    tokens, stream): a cached block's keys are summed once, not on every call.
-    The slot drops the memo whenever it is written."""
-    slot = view.slot
-    key = (int(view.row0), int(view.tokens), int(stream))
-    hit = slot.key_sums.get(key)
-    if hit is None:
-        seg = view.to_segment()
-        hit = torch.empty((slot.heads, slot.head_dim), dtype=torch.int64, device=slot.device)
-        _native.check(lib.tmhd_k_fixed_sum(seg.k, seg.k_head_stride, seg.tokens, slot.heads, slot.head_dim,
-                                           _native.ptr(hit), stream), "tmhd_k_fixed_sum")
-        slot.key_sums[key] = hit
-    return _native.ptr(hit)
+def _key_sums(torch: Any, segments: Sequence[SlotView], stream: int, qq: Any, out: Any, base: int) -> None:
+    """Where the exact fixed-point key sums of each segment (the smooth-K mean's
+    terms) are or go, memoised on its slot per (row0, tokens, stream): a cached
+    block's keys are summed once, not on every call.  The slot drops the memo
+    whenever it is written."""
+    for j, view in enumerate(segments):
+        slot = view.slot
+        key = (int(view.row0), int(view.tokens), int(stream))
+        hit = slot.key_sums.get(key)
+        if hit is None:
+            hit = torch.empty((slot.heads, slot.head_dim), dtype=torch.int64, device=slot.device)
+            slot.key_sums[key] = hit
+            out[base + j] = _native.ptr(hit)  # summed by this batch
+        else:
+            qq.k_sum[j] = _native.ptr(hit)
 
 
 def _coalesce_segments(torch: Any, segments: list[SlotView], limit: int) -> list[SlotView]:
@@ -208,20 +229,46 @@ def segment_attention(
     Row lists are device tensors; their range is checked (one sync) unless
     ``rows_checked`` says the caller built them in range.
     """
-    if backend not in BACKENDS:
-        raise ValueError(f"unknown attention backend {backend!r}")
+    outs, views = segment_attention_batch(
+        torch,
+        [AttentionCall(query, segments, q_rows=q_rows, q_row0=q_row0, lq=lq, out=out, o_rows=o_rows, o_row0=o_row0,
+                       rows_checked=rows_checked)],
+        scale=scale, backend=backend, workspace=workspace, split=split, return_quant=return_quant, timer=timer,
+    )
+    return (outs[0], views[0]) if return_quant and backend == "i8qk" else outs[0]
+
+
+@dataclass
+class AttentionCall:
+    """One call of ``segment_attention_batch``: the arguments of
+    ``segment_attention`` that belong to a single call."""
+
+    query: Any
+    segments: Sequence[SlotView]
+    q_rows: Any | None = None
+    q_row0: int = 0
+    lq: int | None = None
+    out: Any | None = None
+    o_rows: Any | None = None
+    o_row0: int = 0
+    rows_checked: bool = False
+
+
+def _call_args(torch: Any, call: AttentionCall, args: Any, scale: float, keep: list[Any]) -> tuple[Any, list[SlotView]]:
+    """Check one call and fill its C arguments; returns its output and segments."""
+    query, out, q_rows, o_rows, lq = call.query, call.out, call.q_rows, call.o_rows, call.lq
+    q_row0, o_row0 = int(call.q_row0), int(call.o_row0)
     _validate_tokens_major(torch, query, "query")
-    heads, head_dim = int(query.shape[1]), int(query.shape[2])
-    keep: list[Any] = []
+    rows_in, heads, head_dim = query.shape
     if q_rows is not None:
-        q_rows = _row_list(torch, q_rows, query.device, int(query.shape[0]), "q_rows", rows_checked)
+        q_rows = _row_list(torch, q_rows, query.device, rows_in, "q_rows", call.rows_checked)
         keep.append(q_rows)
         n = int(q_rows.numel())
         if lq is not None and int(lq) != n:
             raise ValueError("lq differs from the query row list")
         lq = n
     elif lq is None:
-        lq = int(query.shape[0]) - int(q_row0)
+        lq = rows_in - q_row0
     lq = int(lq)
     if out is None:
         out = torch.empty((lq, heads, head_dim), dtype=torch.bfloat16, device=query.device)
@@ -230,15 +277,15 @@ def segment_attention(
     if tuple(out.shape[1:]) != (heads, head_dim):
         raise ValueError("out heads/dim differ from query")
     if o_rows is not None:
-        o_rows = _row_list(torch, o_rows, out.device, int(out.shape[0]), "o_rows", rows_checked)
+        o_rows = _row_list(torch, o_rows, out.device, int(out.shape[0]), "o_rows", call.rows_checked)
         keep.append(o_rows)
         if int(o_rows.numel()) != lq:
             raise ValueError("output row list length differs from the query rows")
-    elif not (0 <= int(o_row0) and int(o_row0) + lq <= int(out.shape[0])):
-        raise ValueError(f"output rows [{o_row0}, {int(o_row0) + lq}) outside out ({int(out.shape[0])} rows)")
-    if q_rows is None and not (0 <= int(q_row0) and int(q_row0) + lq <= int(query.shape[0])):
-        raise ValueError(f"query rows [{q_row0}, {int(q_row0) + lq}) outside query ({int(query.shape[0])} rows)")
-    segments = [s for s in segments if s.tokens > 0]
+    elif not (0 <= o_row0 and o_row0 + lq <= int(out.shape[0])):
+        raise ValueError(f"output rows [{o_row0}, {o_row0 + lq}) outside out ({int(out.shape[0])} rows)")
+    if q_rows is None and not (0 <= q_row0 and q_row0 + lq <= rows_in):
+        raise ValueError(f"query rows [{q_row0}, {q_row0 + lq}) outside query ({rows_in} rows)")
+    segments = [s for s in call.segments if s.tokens > 0]
     if not segments:
         raise ValueError("attention needs at least one key/value token")
     for s in segments:
@@ -246,48 +293,82 @@ def segment_attention(
             raise ValueError("segment heads/dim/device differ from the query")
     if len(segments) > _native.MAX_SEGMENTS:
         segments = _coalesce_segments(torch, segments, _native.MAX_SEGMENTS)
-    args = _native.AttnArgs()
+        keep.append(segments)
     args.q = _native.ptr(query)
     args.q_token_stride = query.stride(0)
     args.q_head_stride = query.stride(1)
     args.q_rows = _native.ptr(q_rows) if q_rows is not None and lq else None
-    args.q_row0 = int(q_row0)
+    args.q_row0 = q_row0
     args.lq = lq
     args.o = _native.ptr(out)
     args.o_token_stride = out.stride(0)
     args.o_head_stride = out.stride(1)
     args.o_rows = _native.ptr(o_rows) if o_rows is not None and lq else None
-    args.o_row0 = int(o_row0)
+    args.o_row0 = o_row0
     args.heads = heads
     args.head_dim = head_dim
-    args.scale = float(scale)
+    args.scale = scale
     args.n_segments = len(segments)
     for i, s in enumerate(segments):
-        args.seg[i] = s.to_segment()
+        s.fill_segment(args.seg[i])
+    return out, segments
+
+
+def segment_attention_batch(
+    torch: Any,
+    calls: Sequence[AttentionCall],
+    *,
+    scale: float,
+    backend: str = "bf16",
+    workspace: QKQuantWorkspace | None = None,
+    split: bool = True,
+    return_quant: bool = False,
+    timer: ComponentTimer | None = None,
+) -> tuple[list[Any], list[dict[str, Any]]]:
+    """Independent ``segment_attention`` calls in one kernel launch (see
+    ``tmhd_attn_fwd_bf16_batch``): a hook call's condition, media and padding
+    attention, or a packed sequence's documents, none of which alone fills the
+    GPU's last round of workgroups.  The calls share heads, head_dim and the
+    query and output strides; their output rows must not overlap.  Returns
+    their outputs, and with ``return_quant`` the INT8-QK operand views."""
+    if backend not in BACKENDS:
+        raise ValueError(f"unknown attention backend {backend!r}")
+    if not calls:
+        return [], []
+    keep: list[Any] = []  # row lists and merged slots, alive until the launches are queued
+    args = (_native.AttnArgs * len(calls))()
+    outs, segments = [], []
+    for i, call in enumerate(calls):
+        out, segs = _call_args(torch, call, args[i], float(scale), keep)
+        outs.append(out)
+        segments.append(segs)
+    device, heads, head_dim = calls[0].query.device, args[0].heads, args[0].head_dim
+    if any(call.query.device != device or out.device != device for call, out in zip(calls, outs)):
+        raise ValueError("the queries and outputs of a batch must share one GPU")
     lib = _native.load()
-    stream = _native.stream_ptr(torch, query.device)
-    if split and lq:
-        ws = split_workspace(torch, query.device, head_dim)
-        args.split_workspace = _native.ptr(ws)
-        args.split_workspace_bytes = int(ws.numel())
+    stream = _native.stream_ptr(torch, device)
+    if split and any(a.lq for a in args):
+        ws = split_workspace(torch, device, head_dim)
+        args[0].split_workspace = _native.ptr(ws)
+        args[0].split_workspace_bytes = int(ws.numel())
     if backend == "bf16":
         with maybe_region(timer, "attention"):
-            status = lib.tmhd_attn_fwd_bf16(args, stream)
+            status = lib.tmhd_attn_fwd_bf16_batch(args, len(calls), stream)
         _native.check(status, "tmhd_attn_fwd_bf16")
-        return out
+        return outs, []
     if workspace is None:
         workspace = QKQuantWorkspace(torch)
-    qq, views = workspace.quant_struct(
-        heads=heads, head_dim=head_dim, lq=lq, tokens=[s.tokens for s in segments], device=query.device
+    quants, views = workspace.quant_structs(
+        heads=heads, head_dim=head_dim, calls=[(a.lq, [s.tokens for s in segs]) for a, segs in zip(args, segments)],
+        device=device, with_views=return_quant,
     )
     with maybe_region(timer, "qk_quant"):
-        for i, seg in enumerate(segments):
-            qq.k_sum[i] = _key_sum(torch, lib, seg, stream)
-        status = lib.tmhd_qk_smooth_quant(args, qq, stream)
+        sums = (ctypes.c_void_p * (_native.MAX_SEGMENTS * len(calls)))()
+        for i, segs in enumerate(segments):
+            _key_sums(torch, segs, stream, quants[i], sums, i * _native.MAX_SEGMENTS)
+        status = lib.tmhd_qk_smooth_quant_batch(args, quants, sums, len(calls), stream)
     _native.check(status, "tmhd_qk_smooth_quant")
     with maybe_region(timer, "attention"):
-        status = lib.tmhd_attn_fwd_i8qk(args, qq, stream)
+        status = lib.tmhd_attn_fwd_i8qk_batch(args, quants, len(calls), stream)
     _native.check(status, "tmhd_attn_fwd_i8qk")
-    if return_quant:
-        return out, views
-    return out
+    return outs, views

@@ -17,8 +17,8 @@ part into a dense buffer per call (``_materialize_dense_kv_parts``, :56-97)
 and runs SDPA or SageAttention.  Here the history is read in place from the
 cache's slots, the chunk's own K/V rows are packed once into a slot (for a
 commit, that slot *is* the staged block), and one HIP kernel launch computes
-each attention over the segment table.  Query rows are read and output rows
-written in place through contiguous ranges or row lists.
+every attention of the call over its segments.  Query rows are read and output
+rows written in place through contiguous ranges or row lists.
 
 Backends: ``"sdpa"`` -> BF16 kernel (serial mode); ``"sage_attn"`` -> INT8-QK
 kernel (accelerated mode: smooth-K, per-128-block INT8 Q/K, bf16 P.V).
@@ -30,11 +30,11 @@ from enum import Enum
 from typing import Any, Callable
 
 from . import _native, condition
-from .attention import QKQuantWorkspace, segment_attention
+from .attention import AttentionCall, QKQuantWorkspace, segment_attention, segment_attention_batch
 from .kvcache import HeadMajorRingKVCache
 from .profiling import ComponentTimer, maybe_region
 from .rope import fused_qkv_qk_norm_rope_stage_
-from .slots import SlotPool, SlotView
+from .slots import KV_TILE, PackRows, SlotPool, SlotView, round_up
 
 ATTENTION_BACKENDS = ("sdpa", "sage_attn")
 
@@ -84,6 +84,13 @@ class _Rows:
         self.index = None
         if self.count and not self.contiguous:
             self.index = torch.tensor(absolute, dtype=torch.int32, device=device)
+
+    @classmethod
+    def range(cls, start: int, stop: int) -> "_Rows":
+        """The rows ``start .. stop``."""
+        rows = cls.__new__(cls)
+        rows.count, rows.start, rows.contiguous, rows.index = stop - start, start, True, None
+        return rows
 
     def query_kwargs(self) -> dict[str, Any]:
         if self.index is not None:
@@ -255,19 +262,19 @@ class StreamingAttentionHook:
             self._scratch = SlotPool(torch, heads=int(heads), head_dim=int(head_dim), device=device)
         return self._scratch
 
-    def _attend(self, torch: Any, query: Any, q_rows: _Rows, views: list[SlotView], out: Any, scale: float) -> None:
+    def _attend(self, torch: Any, query: Any, emits: list[tuple[Any, ...]], out: Any, scale: float) -> None:
+        """Every attention of a hook call (``emits``: rows, views, ...) as one batch."""
         backend = "bf16" if self.attention_backend == "sdpa" else "i8qk"
         if backend == "i8qk" and self._quant_ws is None:
             self._quant_ws = QKQuantWorkspace(torch)
-        segment_attention(
-            torch, query, views, scale=scale, backend=backend, out=out, workspace=self._quant_ws,
-            timer=self.timer, **q_rows.query_kwargs(), **q_rows.out_kwargs(),
-        )
-        self.kernel_calls += 1
+        calls = [AttentionCall(query, views, out=out, **rows.query_kwargs(), **rows.out_kwargs())
+                 for rows, views, *_ in emits]
+        segment_attention_batch(torch, calls, scale=scale, backend=backend, workspace=self._quant_ws, timer=self.timer)
+        self.kernel_calls += len(emits)
         if backend == "i8qk":
-            self.sage_attn_calls += 1
-            self.sage_attn_query_tokens += q_rows.count
-            self.sage_attn_key_tokens += sum(v.tokens for v in views)
+            self.sage_attn_calls += len(emits)
+            self.sage_attn_query_tokens += sum(rows.count for rows, *_ in emits)
+            self.sage_attn_key_tokens += sum(v.tokens for _, views, *_ in emits for v in views)
 
     def _document_rows(self, torch: Any, index: int, start: int, stop: int, commit_mask: Any) -> tuple[_Rows, _Rows]:
         rows = self._live_document_rows.get(index)
@@ -370,17 +377,17 @@ class StreamingAttentionHook:
                 if at != prestaged[1] or key.stride(1) != int(key.shape[2]):
                     prestaged = None
 
+        packs: list[tuple[_Rows, SlotView]] = []  # rows to pack and the view they get
+
         def scratch_pack(rows: _Rows) -> SlotView:
             nonlocal prestaged
             if prestaged is not None and rows.index is None and (rows.start, rows.count) == prestaged[2:]:
                 view = prestaged[0].view()
                 prestaged = None  # one use
                 return view
-            slot = pool.acquire(rows.count)
-            acquired.append(slot)
-            with maybe_region(self.timer, "pack"):
-                slot.pack(key, value, **rows.pack_kwargs())
-            return slot.view()
+            at = packs[-1][1].row0 + round_up(packs[-1][1].tokens, KV_TILE) if packs else 0
+            packs.append((rows, SlotView(None, rows.count, at)))  # its slot follows once every pack is known
+            return packs[-1][1]
 
         # ---- staging first: the staged slot doubles as a K/V segment
         if self.mode is HookMode.CLEAN_COMMIT:
@@ -401,14 +408,15 @@ class StreamingAttentionHook:
 
         compact = self._compact_output(layer_name, query)
         out = torch.empty_like(query) if compact is None else None
+        emits: list[tuple[Any, ...]] = []  # (rows, views, document, start, stop, kind) of each attention
         try:
             history = self.cache.history_views(layer_name)
             for index, (start, stop) in enumerate(zip(boundaries, boundaries[1:])):
                 if start == stop:
                     continue
                 if index not in live_documents:
-                    doc = _Rows(torch, list(range(start, stop)), query.device)
-                    self._emit(torch, compact, out, query, doc, [scratch_pack(doc)], scale, index, start, stop, "document")
+                    doc = _Rows.range(start, stop)
+                    emits.append((doc, [scratch_pack(doc)], index, start, stop, "document"))
                     continue
                 condition_rows, media_rows = self._document_rows(torch, index, start, stop, commit_mask)
                 condition_view = scratch_pack(condition_rows) if condition_rows.count else None
@@ -444,8 +452,7 @@ class StreamingAttentionHook:
                         if out is not None:
                             self._zero_rows(torch, out, condition_rows)
                     else:
-                        self._emit(torch, compact, out, query, condition_rows, [condition_view], scale, index,
-                                   start, stop, "condition")
+                        emits.append((condition_rows, [condition_view], index, start, stop, "condition"))
                 if media_rows.count:
                     plan = [
                         *([condition_view] if condition_view is not None else []),
@@ -453,16 +460,28 @@ class StreamingAttentionHook:
                         *([previous_view] if previous_view is not None else []),
                         current_view,
                     ]
-                    self._emit(torch, compact, out, query, media_rows, plan, scale, index, start, stop, "media")
+                    emits.append((media_rows, plan, index, start, stop, "media"))
+            if packs:
+                slot = pool.acquire(packs[-1][1].row0 + packs[-1][1].tokens)
+                acquired.append(slot)
+                for _, view in packs:
+                    view.slot = slot
+                ranges: list[PackRows] = []
+                with maybe_region(self.timer, "pack"):
+                    for rows, view in packs:
+                        slot.pack(key, value, dst=view.row0, batch=ranges, **rows.pack_kwargs())
+                    slot.pack_ranges(key, value, ranges, rows_checked=True)
+            if compact is None:
+                self._attend(torch, query, emits, out, scale)
+            else:
+                for emit in emits:
+                    self._emit_compact(torch, compact, query, *emit, scale)
         finally:
             for slot in acquired:
                 pool.release(slot)
         return out if compact is None else compact.output
 
-    def _emit(self, torch, compact, out, query, rows: _Rows, views, scale, index, start, stop, kind) -> None:
-        if compact is None:
-            self._attend(torch, query, rows, views, out, scale)
-            return
+    def _emit_compact(self, torch, compact, query, rows: _Rows, views, index, start, stop, kind, scale) -> None:
         # compact condition-cache writer: compute into a dense buffer first
         dense = torch.empty((rows.count, int(query.shape[1]), int(query.shape[2])), dtype=query.dtype,
                             device=query.device)

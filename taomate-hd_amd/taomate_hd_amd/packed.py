@@ -7,10 +7,10 @@ or FlashAttention-3.  Same arguments, validation and errors; the output is
 ``[tokens, heads, head_dim]`` bf16 in document order (empty documents add no
 rows, as the reference's concatenation does).
 
-Each non-empty document's K/V rows are packed once into one slot of a pooled
-head-major buffer (at a 64-row-aligned offset, tile tail zeroed); one BF16
-kernel launch per document then reads its query rows in place and writes its
-output rows in place, with no per-document concatenation.
+The non-empty documents' K/V rows are packed by one launch into one slot of a
+pooled head-major buffer (each at a 64-row-aligned offset, tile tail zeroed);
+one BF16 launch (per 16 documents) then reads their query rows in place and
+writes their output rows in place, with no per-document concatenation.
 """
 
 from __future__ import annotations
@@ -18,8 +18,8 @@ from __future__ import annotations
 from typing import Any
 
 from . import _native
-from .attention import segment_attention
-from .slots import KV_TILE, SlotPool, SlotView, round_up
+from .attention import AttentionCall, segment_attention_batch
+from .slots import KV_TILE, PackRows, SlotPool, SlotView, round_up
 
 _POOLS: dict[tuple[str, int, int, int], SlotPool] = {}
 
@@ -72,12 +72,14 @@ def packed_sdpa(q: Any, k: Any, v: Any, *, cu_seqlens: Any, cu_seqlens_host: tup
     pool = _pool(torch, q.device, heads, head_dim)
     slot = pool.acquire(total)
     try:
-        for (start, stop), dst in zip(docs, offsets):
-            slot.pack(k, v, row0=start, count=stop - start, dst=dst)
+        slot.pack_ranges(k, v, [PackRows(row0=start, count=stop - start, dst=dst) for (start, stop), dst in zip(docs, offsets)])
         out = torch.empty((int(q.shape[0]), heads, head_dim), dtype=torch.bfloat16, device=q.device)
-        for (start, stop), dst in zip(docs, offsets):
-            segment_attention(torch, q, [SlotView(slot, stop - start, dst)], scale=float(scale), backend="bf16",
-                              q_row0=start, lq=stop - start, out=out, o_row0=start)
+        segment_attention_batch(
+            torch,
+            [AttentionCall(q, [SlotView(slot, stop - start, dst)], q_row0=start, lq=stop - start, out=out, o_row0=start)
+             for (start, stop), dst in zip(docs, offsets)],
+            scale=float(scale), backend="bf16",
+        )
     finally:
         pool.release(slot)
     return out

@@ -17,7 +17,7 @@ for the INT8-QK smooth-K mean); attention reads them in place.
 from __future__ import annotations
 
 from dataclasses import dataclass
-from typing import Any
+from typing import Any, NamedTuple, Sequence
 
 from . import _native
 
@@ -59,18 +59,29 @@ class SlotView:
     tokens: int
     row0: int = 0
 
-    def to_segment(self) -> _native.KVSegment:
+    def fill_segment(self, segment: _native.KVSegment) -> _native.KVSegment:
         s = self.slot
-        if self.row0 % KV_TILE or self.row0 + round_up(self.tokens, KV_TILE) > s.capacity:
-            raise ValueError(f"slot view rows [{self.row0}, {self.row0 + self.tokens}) are not a tile-aligned part of the slot")
-        return _native.KVSegment(
-            k=_native.ptr(s.k) + 2 * self.row0 * s.head_dim,
-            vt=_native.ptr(s.vt) + 2 * self.row0,
-            k_head_stride=s.capacity * s.head_dim,
-            vt_head_stride=s.capacity * s.head_dim,
-            vt_row_stride=s.capacity,
-            tokens=int(self.tokens),
-        )
+        row0, tokens = int(self.row0), int(self.tokens)
+        if row0 % KV_TILE or row0 + round_up(tokens, KV_TILE) > s.capacity:
+            raise ValueError(f"slot view rows [{row0}, {row0 + tokens}) are not a tile-aligned part of the slot")
+        segment.k = _native.ptr(s.k) + 2 * row0 * s.head_dim
+        segment.vt = _native.ptr(s.vt) + 2 * row0
+        segment.k_head_stride = segment.vt_head_stride = s.capacity * s.head_dim
+        segment.vt_row_stride = s.capacity
+        segment.tokens = tokens
+        return segment
+
+    def to_segment(self) -> _native.KVSegment:
+        return self.fill_segment(_native.KVSegment())
+
+
+class PackRows(NamedTuple):
+    """One range of ``KVSlot.pack_ranges``: the arguments of ``KVSlot.pack``."""
+
+    rows: Any | None = None
+    row0: int = 0
+    count: int | None = None
+    dst: int = 0
 
 
 class KVSlot:
@@ -87,6 +98,8 @@ class KVSlot:
         self.k = torch.empty((self.heads, self.capacity, self.head_dim), dtype=torch.bfloat16, device=self.device)
         self.vt = torch.empty((self.heads, self.head_dim, self.capacity), dtype=torch.bfloat16, device=self.device)
         self.tokens = 0
+        # handle of the stream whose allocation pool the memory came from
+        self.allocated_on = _native.stream_ptr(torch, self.device) if self.k.is_cuda else 0
         # handle of the stream a pool last took this slot back on
         self.released_on: int | None = None
         # exact fixed-point key sums of views of this slot, (row0, tokens, stream) ->
@@ -104,7 +117,7 @@ class KVSlot:
         return SlotView(self, count)
 
     def pack(self, key: Any, value: Any, *, rows: Any | None = None, row0: int = 0, count: int | None = None,
-             dst: int = 0, rows_checked: bool = False) -> None:
+             dst: int = 0, rows_checked: bool = False, batch: list[PackRows] | None = None) -> None:
         """Copy token-major rows of ``key``/``value`` ([T, H, D] bf16) into the slot.
 
         ``rows`` is an int32/int64 GPU index tensor; without it rows
@@ -112,7 +125,17 @@ class KVSlot:
         ``dst ..`` (``dst`` a multiple of 64) and the slot rows after them up to
         the next multiple of 64 are zeroed; ``tokens`` becomes the end row.
         The range of ``rows`` is checked (one sync) unless ``rows_checked``.
+        With ``batch`` the range is only appended to that list, for a
+        ``pack_ranges`` of all of them.
         """
+        ranges = [] if batch is None else batch
+        ranges.append(PackRows(rows, row0, count, dst))
+        if batch is None:
+            self.pack_ranges(key, value, ranges, rows_checked=rows_checked)
+
+    def pack_ranges(self, key: Any, value: Any, ranges: Sequence[PackRows], *, rows_checked: bool = False) -> None:
+        """``pack`` of several row ranges in one launch; they must not share a
+        64-row tile of the slot.  ``tokens`` becomes the end row of the last."""
         torch = self._torch
         for name, t in (("key", key), ("value", value)):
             _native.require_device_tensor(torch, t, name)
@@ -122,30 +145,39 @@ class KVSlot:
             raise ValueError("key and value must share shape and strides")
         if tuple(key.shape[1:]) != (self.heads, self.head_dim):
             raise ValueError(f"K/V heads x dim {tuple(key.shape[1:])} differ from slot {(self.heads, self.head_dim)}")
-        rows_ptr = None
-        if rows is not None:
-            from .attention import _row_list
+        total = int(key.shape[0])
+        table = (_native.PackRange * len(ranges))()
+        keep: list[Any] = []
+        end = self.tokens
+        for r, item in zip(table, ranges):
+            if item.rows is not None:
+                from .attention import _row_list
 
-            rows = _row_list(torch, rows, key.device, int(key.shape[0]), "rows", rows_checked)
-            n = int(rows.numel())
-            rows_ptr = _native.ptr(rows) if n else None
-        else:
-            n = int(key.shape[0]) - int(row0) if count is None else int(count)
-            if int(row0) < 0 or n < 0 or int(row0) + n > int(key.shape[0]):
-                raise ValueError(f"rows [{row0}, {int(row0) + n}) outside the {int(key.shape[0])} K/V rows")
-        dst = int(dst)
-        if dst < 0 or dst % KV_TILE or dst + n > self.capacity:
-            raise ValueError(f"{n} rows at slot row {dst} do not fit the slot capacity {self.capacity} (tile-aligned)")
+                rows = _row_list(torch, item.rows, key.device, total, "rows", rows_checked)
+                keep.append(rows)
+                n = int(rows.numel())
+                r.rows = _native.ptr(rows) if n else None
+                r.row0 = 0
+            else:
+                n = total - int(item.row0) if item.count is None else int(item.count)
+                if int(item.row0) < 0 or n < 0 or int(item.row0) + n > total:
+                    raise ValueError(f"rows [{item.row0}, {int(item.row0) + n}) outside the {total} K/V rows")
+                r.rows = None
+                r.row0 = int(item.row0)
+            dst = int(item.dst)
+            if dst < 0 or dst % KV_TILE or dst + n > self.capacity:
+                raise ValueError(f"{n} rows at slot row {dst} do not fit the slot capacity {self.capacity} (tile-aligned)")
+            r.n, r.dst, r.zero_to = n, dst, dst + round_up(n, KV_TILE)
+            end = dst + n
         self.key_sums.clear()
-        lib = _native.load()
-        status = lib.tmhd_kv_pack(
-            _native.ptr(key), _native.ptr(value), key.stride(0), key.stride(1), rows_ptr, int(row0), n,
-            _native.ptr(self.k), _native.ptr(self.vt), self.capacity * self.head_dim,
-            self.capacity * self.head_dim, self.capacity, dst, dst + round_up(n, KV_TILE), self.heads,
-            self.head_dim, _native.stream_ptr(torch, key.device),
+        stride = self.capacity * self.head_dim
+        status = _native.load().tmhd_kv_pack_ranges(
+            _native.ptr(key), _native.ptr(value), key.stride(0), key.stride(1), table, len(ranges),
+            _native.ptr(self.k), _native.ptr(self.vt), stride, stride, self.capacity, self.heads, self.head_dim,
+            _native.stream_ptr(torch, key.device),
         )
         _native.check(status, "tmhd_kv_pack")
-        self.tokens = dst + n
+        self.tokens = end
 
     def token_major(self, tokens: int | None = None, order: Any | None = None) -> tuple[Any, Any]:
         """Materialise ``[tokens, H, D]`` key/value copies (compatibility path)."""
@@ -210,12 +242,13 @@ class SlotPool:
         torch = self._torch
         if torch.device(self.device).type != "cuda":
             return 0
-        return int(torch.cuda.current_stream(device=self.device).cuda_stream)
+        return _native.stream_ptr(torch, self.device)
 
     def release(self, slot: KVSlot) -> None:
         slot.tokens = 0
         torch = self._torch
-        if slot.k.is_cuda:
+        # (the stream of its allocation needs no record)
+        if slot.k.is_cuda and _native.stream_ptr(torch, slot.k.device) != slot.allocated_on:
             stream = torch.cuda.current_stream(device=slot.k.device)
             slot.k.record_stream(stream)
             slot.vt.record_stream(stream)

@@ -59,3 +59,85 @@ def test_shared_out_ranges_match_whole_items(torch_mod, dev, backend, heads, dim
         want = oatt.attention_fp64(q[:, hs], k[:, hs], v[:, hs], dim ** -0.5)
         mx, mean = err_stats(b[:, hs], want)
         assert mx <= 2e-2 and mean <= 1e-3, (mx, mean)
+
+
+@pytest.mark.parametrize("backend", ["bf16", "i8qk"])
+@pytest.mark.parametrize(
+    "heads,dim,docs,shared",
+    [
+        (14, 128, [300, 1, 64, 65, 513], True),  # a shared segment in front of every document's own
+        (3, 64, [33, 257, 256, 0, 700], False),  # a call without queries
+        (2, 128, list(range(1, 20)), True),  # more calls and segments than one launch takes (16, 24)
+    ],
+)
+def test_batch_matches_single_calls(torch_mod, dev, backend, heads, dim, docs, shared):
+    """A batch gives what its calls give alone: for INT8-QK the same operands bit
+    for bit (with the key sums taken in the batch), and outputs that differ only
+    by where the ranges of the last round are cut; one call reads its rows
+    through a row list."""
+    torch = torch_mod
+    from taomate_hd_amd import KVSlot, segment_attention
+    from taomate_hd_amd.attention import AttentionCall, QKQuantWorkspace, segment_attention_batch
+    from taomate_hd_amd.slots import PackRows, SlotView, round_up
+
+    lengths = [max(n, 1) for n in docs]  # keys of each document; docs: its queries
+    total = sum(lengths)
+    q = to_dev(randn_bf16((total, heads, dim), 150), dev)
+    k = to_dev(randn_bf16((total, heads, dim), 151, offset=key_offset(heads, dim, 153)), dev)
+    v = to_dev(randn_bf16((total, heads, dim), 152), dev)
+    slot = KVSlot(torch, heads=heads, head_dim=dim, capacity=sum(round_up(n, 64) for n in lengths), device=dev)
+    alone = KVSlot(torch, heads=heads, head_dim=dim, capacity=slot.capacity, device=dev)
+    for s in (slot, alone):
+        s.k.fill_(9.0)
+        s.vt.fill_(9.0)
+    at, row, ranges, starts = 0, 0, [], []
+    for n in lengths:
+        starts.append((row, at))
+        rows = torch.arange(row, row + n, device=dev) if n % 2 else None
+        ranges.append(PackRows(rows, row, n, at))
+        alone.pack(k, v, row0=row, count=n, dst=at)
+        row, at = row + n, at + round_up(n, 64)
+    slot.pack_ranges(k, v, ranges)
+    torch.cuda.synchronize()
+    assert torch.equal(slot.k.view(torch.int16), alone.k.view(torch.int16))
+    assert torch.equal(slot.vt.view(torch.int16), alone.vt.view(torch.int16))
+    assert slot.tokens == alone.tokens
+    first = SlotView(slot, lengths[0], 0)
+
+    def views(i):
+        own = SlotView(slot, lengths[i], starts[i][1])
+        return [first, own] if shared and i else [own]
+
+    out = torch.full_like(q, 7.0)
+    calls = []
+    for i, n in enumerate(docs):
+        rows = dict(q_row0=starts[i][0], lq=n, o_row0=starts[i][0])
+        if i == 1:
+            index = torch.arange(starts[i][0], starts[i][0] + n, device=dev, dtype=torch.int32)
+            rows = dict(q_rows=index, o_rows=index)
+        calls.append(AttentionCall(q, views(i), out=out, **rows))
+    outs, quants = segment_attention_batch(torch, calls, scale=dim ** -0.5, backend=backend,
+                                           workspace=QKQuantWorkspace(torch), return_quant=True)
+    assert all(o is out for o in outs)
+    torch.cuda.synchronize()
+    for i, n in enumerate(docs):
+        ref = torch.full_like(q, 7.0)
+        got = segment_attention(torch, q, [SlotView(alone, x.tokens, x.row0) for x in views(i)], scale=dim ** -0.5,
+                                backend=backend, q_row0=starts[i][0], lq=n, out=ref, o_row0=starts[i][0],
+                                workspace=QKQuantWorkspace(torch), return_quant=backend == "i8qk")
+        torch.cuda.synchronize()
+        rows = slice(starts[i][0], starts[i][0] + n)
+        if backend == "i8qk":
+            want = got[1]
+            nq = round_up(n, 256)
+            assert torch.equal(quants[i]["k_mean"].view(torch.int16), want["k_mean"].view(torch.int16)), i
+            assert torch.equal(quants[i]["q_i8"][:, :nq], want["q_i8"][:, :nq]), i
+            assert torch.equal(quants[i]["q_scale"][:, : nq // 128], want["q_scale"][:, : nq // 128]), i
+            for a, b in zip(quants[i]["k_i8"] + quants[i]["k_scale"], want["k_i8"] + want["k_scale"]):
+                assert torch.equal(a, b), i
+        if n:
+            # outputs below 4 in magnitude: one bf16 step is at most 1.6e-2
+            mx, mean = err_stats(bf16.from_torch(out[rows]), bf16.from_torch(ref[rows]))
+            assert mx <= 1.6e-2 and mean <= 2e-4, (i, mx, mean)
+        else:
+            assert torch.equal(out[rows], ref[rows])
