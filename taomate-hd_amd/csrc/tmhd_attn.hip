@@ -110,7 +110,8 @@ struct Prob {
   int32_t ntiles;  // key tiles of its segments
   int32_t item0;   // items of the problems in front of it
   int32_t nwhole;  // its items [0, nwhole) run whole
-  int32_t npart;   // key ranges of each of the others (see KArgs)
+  int32_t npart;   // line units of each of the others (see KArgs): its key ranges, or
+  int32_t cut;     // (cut 0) what it weighs as a whole
   int32_t line0;   // line position of item nwhole
 };
 
@@ -125,12 +126,18 @@ struct KArgs {
   // per workgroup.  The others (the last, partial round) are cut into npart
   // equal key ranges each, which are laid end to end on a line; each of the
   // `pieces` remaining workgroups takes the next `share` of them, which may
-  // begin in one item and end in another.  (A line cut at arbitrary key tiles
-  // took the same time, 157 against 159 us at 154 items of 135 key tiles, for
-  // more arithmetic here and in the merge.)  The part of an item that a
-  // workgroup does not hold whole goes to ws slot 2 w (its first item) or
-  // 2 w + 1 (its last): [kBM][D] normalised O, then [kBM] log2-sum-exp.
+  // begin in one item and end in another.
+  // The items of a problem much shorter than the longest are not cut; such an
+  // item takes the units of its length and overhead, rounded up, and runs where
+  // its first unit falls (counted by its tiles alone, the share that held eight
+  // items of 6 tiles outlasted the others, 197 against 180 us for the call).
+  // (A line cut at arbitrary key tiles took the same time, 157 against 159 us
+  // at 154 items of 135 key tiles, for more arithmetic here and in the merge.)
+  // The part of an item that a workgroup does not hold whole goes to ws slot
+  // 2 w (its first item) or 2 w + 1 (its last): normalised O ([kBM][D] values,
+  // see write_item), then [kBM] log2-sum-exp.
   int32_t full, pieces, share, line;
+  int32_t o16;  // output rows 16-byte aligned
   float *ws;
   Prob pr[kMaxProb];
   Seg seg[kMaxBatchSeg];
@@ -190,6 +197,7 @@ __device__ __forceinline__ Cursor cursor_begin(const KArgs &a, int b) {
 }
 // The next item (or part of one) of a workgroup; false at its end.
 __device__ __forceinline__ bool cursor_next(const KArgs &a, Cursor &c, Frag &f) {
+  for (;;) {
   if (c.pos >= c.hi) return false;
   int p = 0, item;
   f.slot = -1;
@@ -204,16 +212,24 @@ __device__ __forceinline__ bool cursor_next(const KArgs &a, Cursor &c, Frag &f) 
     while (p + 1 < a.nprob && c.pos >= a.pr[p + 1].line0) ++p;
     const int np = a.pr[p].npart, nt = a.pr[p].ntiles, off = c.pos - a.pr[p].line0;
     const int it = uniform(off / np), q0 = off - it * np, q1 = min(np, q0 + c.hi - c.pos);
-    f.ta = uniform(nt * q0 / np);
-    f.tb = uniform(nt * q1 / np);
-    if (q0 > 0 || q1 < np) f.slot = 2 * c.w + (c.pos == c.w * a.share ? 0 : 1);
+    const int at = c.pos;
     c.pos += q1 - q0;
+    f.ta = 0;
+    f.tb = nt;
+    if (a.pr[p].cut) {
+      f.ta = uniform(nt * q0 / np);
+      f.tb = uniform(nt * q1 / np);
+      if (q0 > 0 || q1 < np) f.slot = 2 * c.w + (at == c.w * a.share ? 0 : 1);
+    } else if (q0 > 0) {
+      continue;
+    }
     item = a.pr[p].nwhole + it;
   }
   f.p = p;
   f.h = uniform(item / a.pr[p].nqt);
   f.qt = item - f.h * a.pr[p].nqt;
   return true;
+  }
 }
 
 // Position of one head's tile stream: segment s, tile t of nt, with the
@@ -433,6 +449,92 @@ __device__ __forceinline__ void load_lds16(const void *base, uint32_t off, uint3
   asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds_addr) : "memory");
 }
 
+// Physical 16-byte chunk of chunk c of staged row r (rows of 2 D bytes): the
+// rows that share the 512 bytes of the 128 banks sit next to each other, the
+// others are spread over the chunks.  A staging write (8 bytes per lane, one
+// chunk of 32 rows) and a read (16 bytes per lane, whole rows) then meet every
+// bank once.
+template <int D>
+__device__ __forceinline__ int stage_chunk(int r, int c) {
+  constexpr int CPR = D / 8, RPL = 256 / D;
+  return c ^ ((r / RPL) & (CPR - 1));
+}
+
+// Writes ROWS staged output rows (at `stage`, in LDS) of rows ql0, ql0 + 1, ...
+// of head h, token-major: whole rows, 16 bytes per lane.  THREADS lanes, of
+// which this one is number t.
+template <int D, int ROWS, int THREADS>
+__device__ __forceinline__ void write_rows(const char *stage, const KArgs &a, const Prob &P, int h, int ql0, int t) {
+  constexpr int CPR = D / 8, RPI = THREADS / CPR;
+#pragma unroll
+  for (int it = 0; it < ROWS / RPI; ++it) {
+    const int r = it * RPI + t / CPR, c = t % CPR, ql = ql0 + r;
+    const i32x4 v = *(const i32x4 *)(stage + r * (2 * D) + stage_chunk<D>(r, c) * 16);
+    if (ql < P.lq) {
+      const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
+      uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + c * 8;
+      if (a.o16) {
+        *(i32x4 *)op = v;
+      } else {  // rows aligned to 8 bytes only
+        *(i32x2 *)op = i32x2{v[0], v[1]};
+        *(i32x2 *)(op + 4) = i32x2{v[2], v[3]};
+      }
+    }
+  }
+}
+
+// One item's result from the registers of its four waves: o[hf][db] of a lane
+// holds columns db * 32 + 8 u + 4 g + (0..3) (u = 0..3) of row hf * 32 + lr.  Whole
+// items go through LDS (`smem`, free of tile reads and loads by now; each wave
+// its own rows) and out as whole rows: a round of items of one key tile takes
+// 13.0 us (BF16, head_dim 128; INT8-QK 16.3), against 14.5 (18.7) with the rows
+// stored straight from the registers, 16 bytes of 32 rows at a time; the output
+// alone is 3.3 us of memory time.  Parts go to their slot in register order, 1
+// KiB per store, which the merge reads back.
+template <int D>
+__device__ __forceinline__ void write_item(f32x16 (&o)[2][D / 32], const float (&lsum)[2], const float (&mref)[2],
+                                           const KArgs &a, const Prob &P, const Frag &fr, int w, int lane, char *smem) {
+  constexpr int DB = D / 32;
+  const int lr = lane & 31, g = lane >> 5, q0 = fr.qt * kBM + w * kQW;
+  if (fr.slot >= 0) {
+    float *wo = a.ws + (int64_t)fr.slot * (kBM * D + kBM);
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
+      const float inv = 1.0f / lt;
+      if (q0 + hf * 32 + lr < P.lq) {
+        float *op = wo + (w * 2 + hf) * (32 * D) + lane * 4;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            *(f32x4 *)(op + (db * 4 + u) * 256) = f32x4{o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv,
+                                                        o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv};
+        if (g == 0) wo[kBM * D + w * kQW + hf * 32 + lr] = mref[hf] + __log2f(lt);
+      }
+    }
+    return;
+  }
+  char *stage = smem + w * (kQW * 2 * D);
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
+    const float inv = 1.0f / lt;
+    const int r = hf * 32 + lr;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        *(i32x2 *)(stage + r * (2 * D) + stage_chunk<D>(r, db * 4 + u) * 16 + 8 * g) =
+            i32x2{(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
+                  (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
+  }
+  // a wave reads what its other lanes wrote: LDS serves a wave in order
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  write_rows<D, kQW, 64>(stage, a, P, fr.h, q0, lane);
+}
+
 // Work plan of one sub-tile, fixed at compile time.  The sub-tile issues
 // 2 * ns MFMAs (two per slot, one per query half); region r is the code in
 // front of MFMA r.  Issuing an MFMA holds the wave for about 16 of the MFMA's
@@ -546,6 +648,7 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   // fall on 16 distinct bank groups and every operand read is one base
   // register plus an immediate offset.
   __shared__ __attribute__((aligned(1024))) char smem[3 * KT + 3 * VT];
+  static_assert(kBM * 2 * D <= (int)sizeof(smem), "the item's output rows are staged in it");
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
   Cursor cur = cursor_begin(args, blockIdx.x);
@@ -927,46 +1030,9 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
     for (int db = 0; db < DB; ++db) opin(hf * DB + db, o[hf][db]);
-  if (fr.slot >= 0) {
-    // part of an item: normalised partial O and its log2-sum-exp
-    float *wo = a.ws + (int64_t)fr.slot * (kBM * D + kBM);
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-      const float inv = 1.0f / lt;
-      const int rl = w * kQW + hf * 32 + lr;  // row within the item
-      if (q0 + hf * 32 + lr < P.lq) {
-        float *op = wo + rl * D + 4 * g;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            *(f32x4 *)(op + db * 32 + 8 * u) = f32x4{o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv,
-                                                     o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv};
-        if (g == 0) wo[kBM * D + rl] = mref[hf] + __log2f(lt);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-      const float inv = 1.0f / lt;
-      const int ql = q0 + hf * 32 + lr;
-      if (ql < P.lq) {
-        const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
-        uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
-                        (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
-            *(i32x2 *)(op + db * 32 + 8 * u) = pr;
-          }
-      }
-    }
-  }
-  // the next item's first tile loads overwrite tiles that other waves may still read
+  __syncthreads();  // every wave's tile reads and loads are done
+  write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
+  // the next item's first tile loads overwrite rows that other waves may still read
   __syncthreads();
   }
 }
@@ -1092,6 +1158,7 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   // then each lane's tile-load source offsets (8 words per lane)
   constexpr int TAB = 3 * KT + 2 * VT;
   __shared__ __attribute__((aligned(1024))) char smem[TAB + kWaves * 64 * 32];
+  static_assert(kBM * 2 * D <= (int)sizeof(smem), "the item's output rows are staged in it (over the offsets)");
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
 
   Cursor cur = cursor_begin(args, blockIdx.x);
@@ -1447,102 +1514,75 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   // ---- epilogue (as the kernel above)
   wait_vmem();
   drain_o();
-  if (fr.slot >= 0) {
-    float *wo = a.ws + (int64_t)fr.slot * (kBM * D + kBM);
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-      const float inv = 1.0f / lt;
-      const int rl = w * kQW + hf * 32 + lr;
-      if (q0 + hf * 32 + lr < P.lq) {
-        float *op = wo + rl * D + 4 * g;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            *(f32x4 *)(op + db * 32 + 8 * u) = f32x4{o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv,
-                                                     o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv};
-        if (g == 0) wo[kBM * D + rl] = mref[hf] + __log2f(lt);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
-      const float inv = 1.0f / lt;
-      const int ql = q0 + hf * 32 + lr;
-      if (ql < P.lq) {
-        const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
-        uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * g;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            i32x2 pr = {(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
-                        (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
-            *(i32x2 *)(op + db * 32 + 8 * u) = pr;
-          }
-      }
-    }
-  }
-  // the next item's first tile loads overwrite tiles that other waves may still read
+  __syncthreads();  // every wave's tile reads and loads are done
+  write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
+  // the next item's first tile loads overwrite rows that other waves may still read
   __syncthreads();
   }
 }
 
 // Merge of the items that the shares cut: O = sum_p 2^(lse_p - lse) O_p with
 // lse = log2 sum_p 2^lse_p over the item's parts (the partial O_p are
-// normalised).  One thread per 4 columns of a row; items full, full + 1, ...
-// have kBM / RPB blocks each.  An item that one workgroup holds whole is left.
+// normalised, in the attention kernel's register order).  A workgroup takes 32
+// rows of an item, a wave a quarter of their columns; items full, full + 1, ...
+// have kBM / 32 workgroups each.  An item that one workgroup holds whole is
+// left.
 template <int D>
 __global__ void __launch_bounds__(256) attn_merge_kernel(const KArgs a) {
-  constexpr int CG = D / 4, RPB = 256 / CG;  // column groups per row, rows per block
-  const int item = a.full + blockIdx.x / (kBM / RPB);
+  constexpr int NC = D / 32;  // 16-byte chunks per lane and part
+  __shared__ __attribute__((aligned(1024))) char stage[32 * 2 * D];
+  const int item = a.full + blockIdx.x / (kBM / 32), rb = blockIdx.x % (kBM / 32);
   int p = 0;
   while (p + 1 < a.nprob && item >= a.pr[p + 1].item0) ++p;
   const Prob &P = a.pr[p];
   const int L = item - P.item0, h = L / P.nqt, qt = L - h * P.nqt;
-  const int rl = (blockIdx.x % (kBM / RPB)) * RPB + threadIdx.x / CG;
-  const int cg = threadIdx.x % CG;
-  const int ql = qt * kBM + rl;
-  if (ql >= P.lq) return;
+  if (qt * kBM + rb * 32 >= P.lq) return;
   // workgroups w0 .. w1 hold ranges [s, s + npart) of the line; the item is
   // w0's last, unless it begins there, and the first of the others
   const int s = P.line0 + (L - P.nwhole) * P.npart;
   const int w0 = s / a.share, n = (s + P.npart - 1) / a.share - w0 + 1;
-  if (n < 2) return;
+  if (n < 2 || !P.cut) return;
   const int first = s > w0 * a.share ? 1 : 0;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 31, g = lane >> 5;
+  const bool live = qt * kBM + rb * 32 + lr < P.lq;  // dead rows have no part
   constexpr int64_t slot = kBM * D + kBM;
   // four parts at a time, their loads all issued before any is used
   float m = -INFINITY, wsum = 0.0f;
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 acc[NC] = {};
   for (int i = 0; i < n; i += 4) {
     float lse[4];
-    f32x4 val[4];
+    f32x4 val[4][NC];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int r = min(i + j, n - 1);
       const float *b = a.ws + (int64_t)(2 * (w0 + r) + (r == 0 ? first : 0)) * slot;
-      lse[j] = b[kBM * D + rl];
-      val[j] = *(const f32x4 *)(b + rl * D + 4 * cg);
+      lse[j] = live ? b[kBM * D + rb * 32 + lr] : 0.0f;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        val[j][c] = live ? *(const f32x4 *)(b + rb * (32 * D) + (wv * NC + c) * 256 + lane * 4) : f32x4{};
     }
     const float mn = fmaxf(m, fmaxf(fmaxf(lse[0], lse[1]), fmaxf(lse[2], lse[3])));
     const float keep = __builtin_amdgcn_exp2f(m - mn);
     wsum *= keep;
-    acc *= keep;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) acc[c] *= keep;
     m = mn;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (i + j < n) {
         const float wp = __builtin_amdgcn_exp2f(lse[j] - m);
         wsum += wp;
-        acc += wp * val[j];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] += wp * val[j][c];
       }
   }
   const float inv = 1.0f / wsum;
-  const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
-  uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)h * a.ohs + 4 * cg;
-  *(i32x2 *)op = i32x2{(int)pack_bf16x2(acc[0] * inv, acc[1] * inv), (int)pack_bf16x2(acc[2] * inv, acc[3] * inv)};
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    *(i32x2 *)(stage + lr * (2 * D) + stage_chunk<D>(lr, wv * NC + c) * 16 + 8 * g) =
+        i32x2{(int)pack_bf16x2(acc[c][0] * inv, acc[c][1] * inv), (int)pack_bf16x2(acc[c][2] * inv, acc[c][3] * inv)};
+  __syncthreads();
+  write_rows<D, 32, 256>(stage, a, P, h, qt * kBM + rb * 32, threadIdx.x);
 }
 
 bool aligned(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
@@ -1559,10 +1599,11 @@ double tile_us(bool i8, int D, int workgroups, int cus) {
   const double one = D == 128 ? (i8 ? 1.22 : 1.38) : (i8 ? 1.0 : 1.1);
   return one * (1.0 + 0.2 * workgroups / cus);
 }
-// What an item costs besides its tiles, and the merge: its launch, and a
+// What an item costs besides its tiles (5 rounds of 256 items of 1 to 64 key
+// tiles, extrapolated to none), and the merge: its launch, and a
 // partial slot's write and read (at head_dim 128).
-constexpr double kItemUs = 6.0, kMergeUs = 8.0, kMergeUsPerSlot = 0.02;
-constexpr int kMaxParts = 16;
+constexpr double kItemUs = 10.0, kItemUs64 = 6.0, kMergeUs = 8.0, kMergeUsPerSlot = 0.02;
+constexpr int kMaxParts = 16, kItemTiles = 8;  // kItemTiles: kItemUs in tiles
 
 // Decides how the last, partial round of items runs: whole, or as key ranges
 // dealt evenly to workgroups (see KArgs).  `slots` workgroups are resident at
@@ -1584,21 +1625,27 @@ void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
     rest[p] = n - nwhole[p];
     if (rest[p] && k.pr[p].ntiles > longest) longest = k.pr[p].ntiles;
   }
-  auto parts = [&](int p, int n) {
-    const int q = (int)(((int64_t)2 * n * k.pr[p].ntiles + longest) / (2 * (int64_t)longest));
+  // line units of an item of problem p when the longest is cut into n ranges,
+  // and whether it is cut
+  auto units = [&](int p, int n, bool &cut) {
+    int q = (int)(((int64_t)2 * n * k.pr[p].ntiles + longest) / (2 * (int64_t)longest));
+    cut = q > 1;
+    if (!cut) q = (int)(((int64_t)n * (k.pr[p].ntiles + kItemTiles) + longest - 1) / longest);
     return q < 1 ? 1 : q;
   };
-  double best = 0.97 * (longest * tile_us(i8, D, items - full, cus) + kItemUs);
+  const double item = D == 128 ? kItemUs : kItemUs64;
+  double best = 0.93 * (longest * tile_us(i8, D, items - full, cus) + item);
   int best_n = 0;
   for (int n = 2; n <= kMaxParts && 2 * n <= longest; ++n) {
     int64_t line = 0;
-    for (int p = 0; p < k.nprob; ++p) line += (int64_t)rest[p] * parts(p, n);
+    bool cut;
+    for (int p = 0; p < k.nprob; ++p) line += (int64_t)rest[p] * units(p, n, cut);
     const int64_t share = (line + slots - 1) / slots, pieces = (line + share - 1) / share;
     if (line > 0x3fffffff || 2 * pieces * split_slot_bytes(D) > ws_bytes) continue;
-    const int64_t begun = n % share == 0 ? 1 : share / n + 2;  // items a workgroup touches
-    const int64_t cut = pieces + (n % share == 0 ? 0 : items - full);
-    const double us = (double)share * longest / n * tile_us(i8, D, (int)pieces, cus) + kItemUs * (1 + 0.7 * (double)(begun - 1)) +
-                      kMergeUs + D / 128.0 * kMergeUsPerSlot * (double)cut;
+    const int64_t begun = n % share == 0 ? 1 : share / n + 2;  // long items a share touches
+    const int64_t slots_used = pieces + (n % share == 0 ? 0 : items - full);
+    const double us = (double)share * longest / n * tile_us(i8, D, (int)pieces, cus) +
+                      item * (1 + 0.7 * (double)(begun - 1)) + kMergeUs + D / 128.0 * kMergeUsPerSlot * (double)slots_used;
     if (us < best) best = us, best_n = n;
   }
   if (!best_n) return;
@@ -1606,7 +1653,9 @@ void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
   k.line = 0;
   for (int p = 0; p < k.nprob; ++p) {
     k.pr[p].nwhole = nwhole[p];
-    k.pr[p].npart = parts(p, best_n);
+    bool cut;
+    k.pr[p].npart = units(p, best_n, cut);
+    k.pr[p].cut = cut;
     k.pr[p].line0 = k.line;
     k.line += rest[p] * k.pr[p].npart;
   }
@@ -1710,7 +1759,7 @@ int launch_group(KArgs &k, int nseg, int D, void *ws, int64_t ws_bytes, hipStrea
     hipLaunchKernelGGL((attn_fwd_kernel<64>), dim3(grid), dim3(kWaves * 64), 0, s, k);
   const int st = check_launch(what);
   if (st || !k.pieces) return st;
-  const unsigned mgrid = (unsigned)(items - k.full) * (kBM / (256 / (D / 4)));
+  const unsigned mgrid = (unsigned)(items - k.full) * (kBM / 32);
   if (D == 128)
     hipLaunchKernelGGL((attn_merge_kernel<128>), dim3(mgrid), dim3(256), 0, s, k);
   else
@@ -1732,6 +1781,7 @@ int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, int n, void
     k.ots = args->o_token_stride, k.ohs = args->o_head_stride;
     k.heads = args->heads;
     k.c = args->scale * kLog2e;
+    k.o16 = 1;
     nseg = 0;
   };
   // every call is checked before the first launch
@@ -1759,6 +1809,7 @@ int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, int n, void
     P.seg0 = nseg;
     nseg += args[i].n_segments;
     P.seg_end = nseg;
+    k.o16 = k.o16 && aligned(P.o, 16) && k.ots % 8 == 0 && k.ohs % 8 == 0;
     ++k.nprob;
   }
   return launch_group<I8>(k, nseg, args->head_dim, args->split_workspace, args->split_workspace_bytes,

@@ -141,3 +141,26 @@ def test_batch_matches_single_calls(torch_mod, dev, backend, heads, dim, docs, s
             assert mx <= 1.6e-2 and mean <= 2e-4, (i, mx, mean)
         else:
             assert torch.equal(out[rows], ref[rows])
+
+
+@pytest.mark.parametrize("backend", ["bf16", "i8qk"])
+@pytest.mark.parametrize("dim,lq,n", [(128, 300, 200), (64, 70, 130), (128, 257, 2000)])
+def test_output_rows_aligned_to_8_bytes(torch_mod, dev, backend, dim, lq, n):
+    """Output rows that 16-byte stores do not fit (8-byte aligned base and
+    strides), whole items and cut ones (the last shape), with output rows in
+    reverse order: the values of the aligned output, nothing else touched."""
+    torch = torch_mod
+    from taomate_hd_amd import segment_attention
+
+    heads = 3
+    q = to_dev(randn_bf16((lq, heads, dim), 160), dev)
+    views = _slots(torch, dev, randn_bf16((n, heads, dim), 161), randn_bf16((n, heads, dim), 162), [n])
+    ref = segment_attention(torch, q, views, scale=dim ** -0.5, backend=backend)
+    base = torch.full((lq + 2, heads, dim + 12), 7.0, dtype=torch.bfloat16, device=dev)
+    out = base[:, :, 4 : 4 + dim]
+    order = torch.arange(lq, 0, -1, device=dev, dtype=torch.int32)
+    segment_attention(torch, q, views, scale=dim ** -0.5, backend=backend, out=out, o_rows=order)
+    torch.cuda.synchronize()
+    assert torch.equal(out[1 : lq + 1].flip(0).view(torch.int16), ref.view(torch.int16))
+    assert bool((base[:, :, :4] == 7.0).all()) and bool((base[:, :, 4 + dim :] == 7.0).all())
+    assert bool((base[0] == 7.0).all()) and bool((base[lq + 1] == 7.0).all())
