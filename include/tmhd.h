@@ -455,18 +455,17 @@ int tmhd_gemm_i8_i32(int32_t *out, const int8_t *a, const int8_t *b, int32_t m,
 
 /*
  * No counterpart in the reference (the caller-provided scratch of the two
- * GEMMs above).  When the 256 x 256 tiles leave a last round that fills at
- * most half of the CUs (or fill less than half in all), that round's tiles
- * are split along k into up to CUs / tiles parts of at least 256 bytes of k;
- * the parts' int32 partial tiles go to `workspace` and a second pass adds
- * them (exactly) and applies the same epilogue, so results are bit-identical
- * to the unsplit GEMM.  tmhd_gemm_split_workspace_bytes gives the bytes this
- * needs on the current device for the shape (0: no split); with a smaller or
- * null workspace the _ws calls run unsplit.  Partial tiles of calls that
- * overlap on one workspace race.  A last round of at most an eighth of the
- * CUs' tiles needs no workspace in these two GEMMs: it runs as 64 x 128
- * sub-tiles over the whole of k (bit-identical too), with or without one;
- * the SwiGLU GEMM below splits it along k.
+ * GEMMs above).  When the 256 x 256 tiles leave a last round that does not
+ * fill the CUs (or fill less than one in all), that round runs in the form
+ * estimated fastest: whole, as smaller tiles over the whole of k, or, where it
+ * fills at most half of the CUs, split along k into up to CUs / tiles parts of
+ * at least 256 bytes of k; the parts' int32 partial tiles go to `workspace`
+ * and a second pass adds them (exactly) and applies the same epilogue.
+ * Results are bit-identical in every form.  tmhd_gemm_split_workspace_bytes
+ * gives the bytes that the k split would need on the current device for the
+ * shape (0: none); with a smaller or null workspace the _ws calls do not use
+ * that form.  Partial tiles of calls that overlap on one workspace race.  The
+ * SwiGLU GEMM below has the same forms.
  */
 int64_t tmhd_gemm_split_workspace_bytes(int32_t m, int32_t n, int32_t k);
 int tmhd_gemm_w8a8_ws(void *out, const int8_t *a, const int8_t *b, const float *a_scale,

@@ -153,6 +153,8 @@ struct GArgs {
   // K split of the last, partial round (one-wave-per-SIMD kernel): tiles
   // [0, full) are whole; block t * nsplit + p of the split launch is k-range p
   // of tile full + t, whose int32 partial tile goes to ws (merged afterwards)
+  // (tile kernel: parts of the tiles from `full` on, or with full < 0 its own
+  // tiling of the whole matrix)
   int32_t full, nsplit;
   int32_t *ws;
 };
@@ -365,6 +367,9 @@ gemm_i8_kernel(const GArgs ga) {
 constexpr int HBM_ = 256, HBN = 256, HKD = 128, HWAVES = 4, HRING = 5;
 constexpr int HUNIT = 2 * 128 * HKD;  // bytes of one ring unit: 128 rows of A, then of B
 
+// s_waitcnt immediate that leaves n vector-memory operations in flight (and waits for nothing else)
+constexpr int vmcnt_imm(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
+
 __device__ __forceinline__ void hload_lds16(const void *base, uint32_t off, uint32_t lds_addr) {
   asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds_addr) : "memory");
 }
@@ -453,7 +458,7 @@ gemm_i8_wave128_kernel(const GArgs ga) {
   for (int u = 0; u < 4; ++u)
 #pragma unroll
     for (int n = 0; n < 8; ++n) load_one(u, n);
-  __builtin_amdgcn_s_waitcnt(0x0f70 | 16);  // vmcnt(16): units 2, 3 may stay in flight
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(16));  // units 2, 3 may stay in flight
   __syncthreads();
   i32x4 cur[16], nxt[16];
   // operand r of k-step q of k block d (ring position dm = d % HRING): r < 8
@@ -719,135 +724,223 @@ gemm_i8_wave128_kernel(const GArgs ga) {
 }
 
 // ---------------------------------------------------------------------------
-// The last, partial round of 256 x 256 tiles when it holds at most an eighth
-// of a round: each of its tiles runs as 8 sub-tiles of 64 (m) x 128 (n) over
-// the whole of k, one workgroup each, so the round fills the CUs with no
-// partial sums and no merge (the k split's int32 partials and their merge
-// cost about twice the time).  4 waves as 2 (m) x 2 (n) of 32 x 64 (8 blocks
-// of v_mfma_i32_16x16x64_i8).  k moves in blocks of 128 bytes, one ring unit
-// each (64 rows of A, then 128 rows of B, rows of 128 bytes with chunk c of
-// row r at c ^ ((r >> 1) & 7), as in the whole-tile kernel), 5 units deep;
-// block d's loads fetch unit d + 3.  The epilogue stores straight from
-// registers (the round is small) with the whole-tile kernel's arithmetic.
-constexpr int SBM = 64, SBN = 128, SRING = 5;
-constexpr int SUNIT = (SBM + SBN) * HKD;  // bytes of one ring unit
-constexpr int SLOADS = SUNIT / 1024 / 4;  // 1 KiB wave loads per wave per unit
-static_assert(SUNIT % 4096 == 0 && SRING * SUNIT <= 160 * 1024, "ring fits the LDS");
+// INT8 GEMM tiles smaller than 256 x 256: 2 MH rows x 2 NH columns, 4 waves as
+// 2 x 2 of MH x NH (blocks of v_mfma_i32_16x16x64_i8), for calls and last
+// rounds whose 256 x 256 tiles leave CUs idle or compute rows that are not
+// there.  k moves in blocks of 128 bytes, two ring units each (one per half of
+// the tile's rows and columns, rows of 128 bytes with chunk c of row r at
+// c ^ ((r >> 1) & 7), as in the whole-tile kernel), RING units deep.  In block d,
+// k-step 0 loads unit 2 d + RING - 1 into the slot of unit 2 d - 1 and reads
+// k-step 1's operands; behind the wait (units 2 d + 2 and 2 d + 3 landed) and
+// the barrier, k-step 1 loads unit 2 d + RING into the slot of unit 2 d and
+// reads block d + 1's first operands.  Reads and loads are dealt between the
+// MFMAs.  What bounds these tiles is the latency of their loads (weights come
+// from HBM once): a ring of 6 to 10 units, or two workgroups per CU, keeps
+// about 100 KiB per CU in flight.
+// The MFMAs are inline asm with the accumulators in VGPRs: for rings that allow
+// one workgroup per CU the compiler keeps the builtin's accumulators in AGPRs
+// and copies them around every MFMA (12 instructions each; 192 x 128 tiles on
+// 331 x 5,376 x 10,752: 43 against 32 us).
+// Tile choice and times: see pick_tile.
+//
+// GLU: the tile's columns are NH gate columns and their NH up columns (128
+// weight rows on), in the waves (wm, 0) and (wm, 1); each hands half of its
+// bf16 projection to the other through LDS and writes SwiGLU of the half it
+// keeps.
 
-template <bool RAW>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-gemm_i8_sub_kernel(const GArgs ga) {
+__device__ __forceinline__ void mfma_i8(i32x4 &acc, const i32x4 &b, const i32x4 &a) {
+  asm("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc) : "v"(b), "v"(a));
+}
+
+template <int MH, int NH, int RING, int WPE, bool RAW, bool GLU>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+gemm_i8_tile_kernel(const GArgs ga) {
 #pragma clang fp contract(off)
-  __shared__ __attribute__((aligned(1024))) char smem[SRING * SUNIT];
+  constexpr int BM = 2 * MH, BN = 2 * NH, UNIT = (MH + NH) * HKD;
+  constexpr int AL = MH / 32, NL = (MH + NH) / 32;  // 1 KiB loads per wave and unit: of A, in all
+  constexpr int MB = MH / 16, NB = NH / 16, NR = MB + NB, NM = MB * NB;
+  constexpr int RS = NM / NR > 0 ? NM / NR : 1, LS = NM / NL > 0 ? NM / NL : 1;  // MFMAs per operand read / load
+  static_assert(RING >= 5 && RING * UNIT <= 160 * 1024 && (RING - 3) * NL < 64, "ring fits the LDS and vmcnt");
+  static_assert(NM >= NR && NM >= NL, "reads and loads fit between a k-step's MFMAs");
+  static_assert(!GLU || (128 % NH == 0 && !RAW), "gate and up columns in blocks of 128");
+  __shared__ __attribute__((aligned(1024))) char smem[RING * UNIT];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = w >> 1, wn = w & 1;  // wave tile: a rows [wm*32, +32), b rows [wn*64, +64)
-  // item L: sub-tile L % 8 of tile full + L / 8; the 8 sub-tiles of a tile are
-  // consecutive logical ids, which run on one XCD (its L2 holds their panels)
+  const int wm = w >> 1, wn = w & 1;
   const int L = xcd_logical_id(blockIdx.x, gridDim.x);
-  const int sub = L & 7;
-  int tm, tn;
-  grouped_tile(ga.full + (L >> 3), ga.tm_count, ga.tn_count, tm, tn);
-  const int m0 = tm * HBM_ + (sub >> 1) * SBM, n0 = tn * HBN + (sub & 1) * SBN;
+  // first row; column tile (of BN columns, or BN / 2 outputs)
+  constexpr int PN = HBN / BN;  // column tiles of a 256 x 256 tile
+  int m0, ct;
+  if (ga.full >= 0) {
+    // part of 256 x 256 tile full + L / parts: consecutive ids, which run on one
+    // XCD (its L2 holds their panels)
+    constexpr int PARTS = (HBM_ / BM > 0 ? HBM_ / BM : 1) * PN;
+    const int sub = L % PARTS;
+    int tm, tn;
+    grouped_tile(ga.full + L / PARTS, ga.tm_count, ga.tn_count, tm, tn);
+    m0 = tm * HBM_ + sub / PN * BM;
+    ct = tn * PN + sub % PN;
+  } else {
+    // the row tiles that share a weight panel run next to each other
+    const int tmc = (ga.m + BM - 1) / BM;
+    ct = L / tmc;
+    m0 = (L - ct * tmc) * BM;
+  }
+  // weight rows of the waves' halves: n0 + h * NS ..
+  constexpr int NS = GLU ? 128 : NH;
+  const int n0 = GLU ? ct / PN * HBN + ct % PN * NH : ct * BN;
   if (m0 >= ga.m || n0 >= ga.n) return;  // the whole workgroup: no barrier is left waiting
   const int nd = ga.k / HKD;  // >= 1
-
-  // Loads: block b (0..23) of a unit is 8 rows x 128 bytes: b < 8 the A rows
-  // 8 b .., else the B rows 8 (b - 8) ..; wave w loads blocks w + 4 i.  Lane:
-  // row 8 blk + lane / 8, physical chunk lane % 8, logical chunk
-  // (lane % 8) ^ ((row >> 1) & 7), the same for all of the wave's blocks
-  // (their parity is w's).
+  // Wave w loads 8-row blocks w, w + 4, ... of each operand.  Lane: row 8 blk +
+  // lane / 8, physical chunk lane % 8, logical chunk (lane % 8) ^ ((row >> 1) & 7),
+  // the same for all of the wave's blocks (their parity is w's).
   const int lch = (lane & 7) ^ ((4 * (w & 1) + (lane >> 4)) & 7);
-  uint32_t soff[SLOADS];
+  uint32_t soff[2][NL];
 #pragma unroll
-  for (int i = 0; i < SLOADS; ++i) {
-    const int b = w + 4 * i;
-    if (b < SBM / 8)
-      soff[i] = (uint32_t)((int64_t)min(m0 + b * 8 + (lane >> 3), ga.m - 1) * ga.lda) + lch * 16;
-    else
-      soff[i] = (uint32_t)((int64_t)min(n0 + (b - SBM / 8) * 8 + (lane >> 3), ga.n - 1) * ga.ldb) + lch * 16;
-  }
-  // unit u (k block min(u, nd - 1): units past the last block repeat it, into
-  // a slot nobody reads) into ring slot u % SRING
-  auto load_unit = [&](int u) {
-    const int64_t k0 = (int64_t)min(u, nd - 1) * HKD;
-    const uint32_t dst = lds0 + (uint32_t)((u % SRING) * SUNIT);
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < SLOADS; ++i) {
-      const int b = w + 4 * i;
-      hload_lds16((b < SBM / 8 ? ga.a : ga.b) + k0, soff[i], dst + b * 1024);
+    for (int i = 0; i < NL; ++i) {
+      if (i < AL)
+        soff[h][i] = (uint32_t)((int64_t)min(m0 + h * MH + (w + 4 * i) * 8 + (lane >> 3), ga.m - 1) * ga.lda) + lch * 16;
+      else
+        soff[h][i] =
+            (uint32_t)((int64_t)min(n0 + h * NS + (w + 4 * (i - AL)) * 8 + (lane >> 3), ga.n - 1) * ga.ldb) + lch * 16;
     }
+  // load i of unit (k block j, half h) into ring slot `slot`; units past the
+  // last block repeat it, into a slot nobody reads
+  auto load_one = [&](int j, int h, int slot, int i) {
+    const uint32_t at = i < AL ? (w + 4 * i) * 1024 : MH * HKD + (w + 4 * (i - AL)) * 1024;
+    hload_lds16((i < AL ? ga.a : ga.b) + (int64_t)min(j, nd - 1) * HKD, soff[h][i], lds0 + (uint32_t)(slot * UNIT) + at);
   };
-  // operand reads: 16x16x64 lane (i, g4) holds 16 bytes of row i at logical
-  // chunk 4 q + g4 (k-step q of the block)
+  // operand reads: 16x16x64 lane (i, g4) holds 16 bytes of row i at logical chunk 4 q + g4
   const int li = lane & 15, lg = lane >> 4;
   uint32_t rdq[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) rdq[q] = (uint32_t)(li * HKD + (((4 * q + lg) ^ ((li >> 1) & 7)) * 16));
-  // operand r of k-step q of unit u: r < 2 A block r, else B block r - 2
-  auto read_op = [&](int u, int q, int r) -> i32x4 {
-    const uint32_t base = (uint32_t)((u % SRING) * SUNIT) + rdq[q];
-    if (r < 2) return *(const i32x4 *)(smem + base + (wm * 32 + 16 * r) * HKD);
-    return *(const i32x4 *)(smem + base + SBM * HKD + (wn * 64 + 16 * (r - 2)) * HKD);
+  // operand r of k-step q of the block whose units are in slots s0 and s1: r < MB A block r, else B block r - MB
+  auto read_op = [&](int s0, int s1, int q, int r) -> i32x4 {
+    if (r < MB) return *(const i32x4 *)(smem + (uint32_t)((wm ? s1 : s0) * UNIT) + rdq[q] + r * 16 * HKD);
+    return *(const i32x4 *)(smem + (uint32_t)((wn ? s1 : s0) * UNIT + MH * HKD) + rdq[q] + (r - MB) * 16 * HKD);
   };
-
-  i32x4 acc[4][2];  // [n block][m block], D[n][m]: lane (j, g4) holds n = 16 nb + 4 g4 + (0..3), m = 16 mb + j
+  i32x4 acc[NB][MB];  // D[n][m]: lane (j, g4) holds n = 16 nb + 4 g4 + (0..3), m = 16 mb + j
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
+    for (int j = 0; j < MB; ++j) acc[i][j] = i32x4{0, 0, 0, 0};
 
-  // prologue: units 0..2 in flight, unit 0 landed
-  load_unit(0);
-  load_unit(1);
-  load_unit(2);
-  __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * SLOADS));  // units 1, 2 may stay in flight
+  // prologue: units 0 .. RING - 2 in flight, units 0 and 1 landed
+#pragma unroll
+  for (int u = 0; u < RING - 1; ++u)
+#pragma unroll
+    for (int i = 0; i < NL; ++i) load_one(u >> 1, u & 1, u, i);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 3) * NL));
   __syncthreads();
-  i32x4 cur[6], nxt[6];
+  i32x4 cur[NR], nxt[NR];
 #pragma unroll
-  for (int r = 0; r < 6; ++r) cur[r] = read_op(0, 0, r);
-  // block d: k-step 0 loads unit d + 3 into the slot of unit d - 2 (every
-  // wave is past block d - 2: the barrier of block d - 1) and reads k-step 1's
-  // operands; k-step 1 waits for unit d + 1 (units d + 2 and d + 3 may stay in
-  // flight), passes the barrier and reads block d + 1's first operands.
+  for (int r = 0; r < NR; ++r) cur[r] = read_op(0, 1, 0, r);
+  auto step = [](int s, int by) { return s + by >= RING ? s + by - RING : s + by; };
+  int s0 = 0;  // slot of unit 2 d
   for (int d = 0; d < nd; ++d) {
-    load_unit(d + 3);
+    const int s1 = step(s0, 1), sp = step(s0, RING - 1), t0 = step(s0, 2), t1 = step(s0, 3);
 #pragma unroll
-    for (int r = 0; r < 6; ++r) nxt[r] = read_op(d, 1, r);
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb) acc[nb][mb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur[2 + nb], cur[mb], acc[nb][mb], 0, 0, 0);
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (2 * SLOADS));
+    for (int idx = 0; idx < NM; ++idx) {
+      if (idx % RS == 0 && idx / RS < NR) nxt[idx / RS] = read_op(s0, s1, 1, idx / RS);
+      if (idx % LS == 0 && idx / LS < NL) load_one(d + (RING - 1) / 2, (RING - 1) & 1, sp, idx / LS);
+      mfma_i8(acc[idx / MB][idx % MB], cur[MB + idx / MB], cur[idx % MB]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((RING - 4) * NL));
     __syncthreads();
-    if (d + 1 < nd)
+    // (after the last block: a stale slot, unused)
 #pragma unroll
-      for (int r = 0; r < 6; ++r) cur[r] = read_op(d + 1, 0, r);
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < 2; ++mb) acc[nb][mb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(nxt[2 + nb], nxt[mb], acc[nb][mb], 0, 0, 0);
+    for (int idx = 0; idx < NM; ++idx) {
+      if (idx % RS == 0 && idx / RS < NR) cur[idx / RS] = read_op(t0, t1, 0, idx / RS);
+      if (idx % LS == 0 && idx / LS < NL) load_one(d + RING / 2, RING & 1, s0, idx / LS);
+      mfma_i8(acc[idx / MB][idx % MB], nxt[MB + idx / MB], nxt[idx % MB]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s0 = t0;
   }
-  // every wave drains its loads before the workgroup ends
-  __builtin_amdgcn_s_waitcnt(0x0f70);
+  // every wave drains its loads before the workgroup ends; the accumulators'
+  // wait states before VALU code reads them
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) asm volatile("" : "+v"(acc[i][j]));
 
   // epilogue straight from registers: 4 consecutive n of one m per lane
+  float asv[MB];
+  if constexpr (!RAW) {
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const int n = n0 + wn * 64 + nb * 16 + 4 * lg;
+    for (int mb = 0; mb < MB; ++mb) asv[mb] = ga.as[min(m0 + wm * MH + mb * 16 + li, ga.m - 1)];
+  }
+  auto columns = [&](int nb, float (&bsv)[4], uint16_t (&bbv)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int nn = min(n0 + wn * NS + nb * 16 + 4 * lg + e, ga.n - 1);
+      bsv[e] = ga.bs[nn];
+      bbv[e] = ga.bias ? ga.bias[nn] : 0;
+    }
+  };
+  auto project = [&](const i32x4 &v, const float (&bsv)[4], const uint16_t (&bbv)[4], float as) {
+    float t[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = dequant_f32(v[e], bsv[e], as, ga.bias != nullptr, bbv[e]);
+    return i32x2{(int)pack_bf16_rne(t[0], t[1]), (int)pack_bf16_rne(t[2], t[3])};
+  };
+  if constexpr (GLU) {
+    // wave (wm, 0) keeps gate blocks [0, NB / 2) and hands over the rest, wave
+    // (wm, 1) keeps up blocks [NB / 2, NB); lane layouts agree
+    constexpr int HALF = NB / 2;
+    static_assert(4 * HALF * MB * 512 <= RING * UNIT, "the exchange fits the ring");
+    __syncthreads();  // every wave is done with the ring
+    i32x2 kept[HALF][MB];
+    char *mine = smem + w * (HALF * MB * 512) + lane * 8;
+    const char *theirs = smem + (w ^ 1) * (HALF * MB * 512) + lane * 8;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      float bsv[4];
+      uint16_t bbv[4];
+      columns(nb, bsv, bbv);
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const i32x2 v = project(acc[nb][mb], bsv, bbv, asv[mb]);
+        const int i = (nb % HALF) * MB + mb;
+        if ((nb >= HALF) == (wn == 1))
+          kept[nb % HALF][mb] = v;
+        else
+          *(i32x2 *)(mine + i * 512) = v;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int nb = 0; nb < HALF; ++nb) {
+      const int n = ct * NH + (wn * HALF + nb) * 16 + 4 * lg;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const i32x2 other = *(const i32x2 *)(theirs + (nb * MB + mb) * 512);
+        const i32x2 g = wn ? other : kept[nb][mb], u = wn ? kept[nb][mb] : other;
+        const int m = m0 + wm * MH + mb * 16 + li;
+        if (m < ga.m)
+          *(i32x2 *)((uint16_t *)ga.out + (int64_t)m * ga.ldo + n) =
+              i32x2{(int)swiglu_pair((uint32_t)g[0], (uint32_t)u[0]), (int)swiglu_pair((uint32_t)g[1], (uint32_t)u[1])};
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    const int n = n0 + wn * NH + nb * 16 + 4 * lg;
     if (n >= ga.n) continue;
     float bsv[4];
     uint16_t bbv[4];
+    if constexpr (!RAW) columns(nb, bsv, bbv);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int nn = min(n + e, ga.n - 1);
-      bsv[e] = RAW ? 0.0f : ga.bs[nn];
-      bbv[e] = (!RAW && ga.bias) ? ga.bias[nn] : 0;
-    }
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb) {
-      const int m = m0 + wm * 32 + mb * 16 + li;
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = m0 + wm * MH + mb * 16 + li;
       if (m >= ga.m) continue;
       if constexpr (RAW) {
         int32_t *op = (int32_t *)ga.out + (int64_t)m * ga.ldo + n;
@@ -856,18 +949,12 @@ gemm_i8_sub_kernel(const GArgs ga) {
         else
           for (int e = 0; e < 4 && n + e < ga.n; ++e) op[e] = acc[nb][mb][e];
       } else {
-        const float asm_ = ga.as[m];
-        uint16_t vals[4];
-        float tv[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tv[e] = dequant_f32(acc[nb][mb][e], bsv[e], asm_, ga.bias != nullptr, bbv[e]);
-        bf16_quad(tv, vals);
+        const i32x2 v = project(acc[nb][mb], bsv, bbv, asv[mb]);
         uint16_t *op = (uint16_t *)ga.out + (int64_t)m * ga.ldo + n;
         if (n + 3 < ga.n && ga.st_ok)
-          *(i32x2 *)op = i32x2{(int)((uint32_t)vals[0] | ((uint32_t)vals[1] << 16)),
-                               (int)((uint32_t)vals[2] | ((uint32_t)vals[3] << 16))};
+          *(i32x2 *)op = v;
         else
-          for (int e = 0; e < 4 && n + e < ga.n; ++e) op[e] = vals[e];
+          for (int e = 0; e < 4 && n + e < ga.n; ++e) op[e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
       }
     }
   }
@@ -947,9 +1034,9 @@ __global__ void __launch_bounds__(256) gemm_split_merge_kernel(const GArgs ga) {
   }
 }
 
-// K split of the last, partial round of 256 x 256 tiles (all tiles when they
-// fill less than half the CUs): its tiles' 128-byte k blocks are dealt to S
-// parts, S up to CUs / tiles and at least 2 blocks per part, so that the
+// The k split that a last, partial round of 256 x 256 tiles (all tiles when they
+// fill less than half the CUs) may take: its tiles' 128-byte k blocks are dealt
+// to S parts, S up to CUs / tiles and at least 2 blocks per part, so that the
 // round fills the CUs; the partials are merged by gemm_split_merge_kernel.
 void gemm_split_plan(int32_t m, int32_t n, int32_t k, int &tail, int &parts) {
   tail = 0, parts = 1;
@@ -964,6 +1051,113 @@ void gemm_split_plan(int32_t m, int32_t n, int32_t k, int &tail, int &parts) {
 }
 
 int64_t gemm_split_bytes(int tail, int parts) { return (int64_t)tail * parts * HBM_ * HBN * 4; }
+
+// How the last, partial round of 256 x 256 tiles runs (all tiles, when they do
+// not fill a round).
+enum Tail { kTailWhole, kTailSplit, kTail64x64, kTail64x128, kTail128, kTail192x128, kTail256x128 };
+
+// The tiles of gemm_i8_tile_kernel and, per 128-byte block of k, the
+// microseconds of a round of them: `one` + `fill` * (share of the CUs in use),
+// or `two` with a second workgroup on each CU.  From k = 5,120 and 5,376 at 16
+// to 2,048 rows and 5,376 to 13,824 columns; with them the choice among the
+// forms below is within 10% of the best one measured there.
+struct TileCost {
+  Tail tail;
+  int bm, bn, per_cu;
+  double one, fill, two;
+};
+constexpr TileCost kTiles[] = {
+    {kTail64x64, 64, 64, 2, 0.19, 0.02, 0.37},     {kTail64x128, 64, 128, 2, 0.24, 0.09, 0.62},
+    {kTail128, 128, 128, 1, 0.42, 0.14, 0.0},      {kTail192x128, 192, 128, 1, 0.58, 0.22, 0.0},
+    {kTail256x128, 256, 128, 1, 0.78, 0.26, 0.0},
+};
+constexpr double kTileFixedUs = 5.0;  // a launch of them: first loads, epilogue
+
+// Cheapest form for `tiles` 256 x 256 tiles (fewer than cus) of an m x n x k
+// product; `part`: they are the last round of more.  Measured, us (before:
+// whole tiles, the k split, and 64 x 128 tiles for a small last round):
+//   16 x 5,120 x 13,824: 64 x 64 tiles 14, 64 x 128 22, k split 34
+//   331 x 5,120 x 13,824: 192 x 128 tiles 40, k split 50, 64 x 128 55, 64 x 64 55
+//   331 x 5,376 x 10,752: 128 x 128 27, 64 x 128 31, 192 x 128 32, k split 48
+//   512 x 5,376 x 5,376: 128 x 128 24, 64 x 64 27, k split 38
+//   1,024 x 5,376 x 10,752 (168 tiles): whole 57, 192 x 128 74, 256 x 128 89
+// The k split remains for long k (8 tiles of 32,768: 24 against 72 us estimated).
+Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cus, int split_parts) {
+  const double nd = (double)(k / HKD);
+  Tail best = kTailWhole;
+  double us = nd * (0.95 + 0.45 * (double)tiles / cus) + 8.0;
+  if (split_parts > 1) {
+    // 12 us of launches and merge, and per tile the write and read of its partials
+    const double t = nd / split_parts * 1.35 + 12.0 + 0.165 * (double)tiles;
+    if (t < us) us = t, best = kTailSplit;
+  }
+  for (const TileCost &c : kTiles) {
+    if (part && HBM_ % c.bm) continue;  // parts of a 256 x 256 tile divide it
+    const int64_t wgs = part ? tiles * (HBM_ / c.bm) * (HBN / c.bn)
+                             : (int64_t)((m + c.bm - 1) / c.bm) * ((n + c.bn - 1) / c.bn);
+    const int64_t slots = (int64_t)cus * c.per_cu, rest = wgs % slots;
+    const double full = c.per_cu == 2 ? c.two : c.one + c.fill;
+    const double last = rest == 0 ? 0.0 : rest <= cus ? c.one + c.fill * (double)rest / cus : c.two;
+    const double t = kTileFixedUs + nd * ((double)(wgs / slots) * full + last);
+    if (t < us) us = t, best = c.tail;
+  }
+  return best;
+}
+
+template <int MH, int NH, int RING, int WPE, bool RAW, bool GLU>
+void launch_tiles(GArgs ga, int64_t tiles, bool part, hipStream_t s) {
+  const int64_t wgs = part ? tiles * (HBM_ / (2 * MH)) * (HBN / (2 * NH))
+                           : (int64_t)((ga.m + 2 * MH - 1) / (2 * MH)) * ((ga.n + 2 * NH - 1) / (2 * NH));
+  if (!part) ga.full = -1;
+  hipLaunchKernelGGL((gemm_i8_tile_kernel<MH, NH, RING, WPE, RAW, GLU>), dim3((unsigned)wgs), dim3(256), 0, s, ga);
+}
+
+// The GEMM (checked arguments, 32-bit row offsets, whole 128-byte k blocks) in
+// rounds of whole tiles and a last round as pick_tail says.  ga.full: all tiles.
+template <bool RAW, bool GLU>
+void launch_rounds(GArgs ga, void *ws, int64_t ws_bytes, hipStream_t s) {
+  const int64_t tiles = ga.full;
+  const int cus = device_cus();
+  const int64_t last = cus > 0 ? tiles % cus : 0;
+  Tail tail = kTailWhole;
+  int split_tiles = 0, parts = 1;
+  if (last > 0) {
+    gemm_split_plan(ga.m, ga.n, ga.k, split_tiles, parts);
+    const bool can_split = parts > 1 && ws && ((uintptr_t)ws % 16) == 0 && ws_bytes >= gemm_split_bytes(split_tiles, parts);
+    tail = pick_tail(last, last < tiles, ga.m, ga.n, ga.k, cus, can_split ? parts : 1);
+  }
+  if (tail != kTailWhole) ga.full = (int32_t)(tiles - last);
+  const bool part = ga.full > 0;
+  if (part)
+    hipLaunchKernelGGL((gemm_i8_wave128_kernel<RAW, false, GLU>), dim3((unsigned)ga.full), dim3(HWAVES * 64), 0, s, ga);
+  switch (tail) {
+    case kTailWhole:
+      break;
+    case kTailSplit:
+      ga.nsplit = parts;
+      ga.ws = (int32_t *)ws;
+      hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, true>), dim3((unsigned)(last * parts)), dim3(HWAVES * 64), 0, s, ga);
+      if constexpr (GLU)
+        hipLaunchKernelGGL(gemm_split_merge_glu_kernel, dim3((unsigned)(last * (HBM_ / 8))), dim3(256), 0, s, ga);
+      else
+        hipLaunchKernelGGL(gemm_split_merge_kernel<RAW>, dim3((unsigned)(last * (HBM_ / 4))), dim3(256), 0, s, ga);
+      break;
+    case kTail64x64:
+      launch_tiles<32, 32, 10, 2, RAW, GLU>(ga, last, part, s);
+      break;
+    case kTail64x128:
+      launch_tiles<32, 64, 6, 2, RAW, GLU>(ga, last, part, s);
+      break;
+    case kTail128:
+      launch_tiles<64, 64, 9, 1, RAW, GLU>(ga, last, part, s);
+      break;
+    case kTail192x128:
+      launch_tiles<96, 64, 7, 1, RAW, GLU>(ga, last, part, s);
+      break;
+    case kTail256x128:
+      launch_tiles<128, 64, 6, 1, RAW, GLU>(ga, last, part, s);
+  }
+}
 
 template <bool RAW>
 int launch_gemm(void *out, const int8_t *a, const int8_t *b, const float *as, const float *bs, const void *bias,
@@ -980,49 +1174,19 @@ int launch_gemm(void *out, const int8_t *a, const int8_t *b, const float *as, co
   GArgs ga{a, b, out, as, bs, (const uint16_t *)bias, m, n, k, lda, ldb, ldo, (m + GBM - 1) / GBM, (n + GBN - 1) / GBN,
            (int32_t)(((uintptr_t)bs % 16) == 0 && ((uintptr_t)bias % 8) == 0),
            (int32_t)(!RAW && ((uintptr_t)out % 16) == 0 && ldo % 8 == 0), (int32_t)tiles, 1, nullptr};
-  const int64_t grid = tiles;
   // the one-wave-per-SIMD kernel takes 32-bit row offsets and whole 128-byte
   // k blocks; other shapes (k an odd multiple of 64) run the 8-wave kernel
   const bool wide = (int64_t)(m - 1) * lda + k < ((int64_t)1 << 32) &&
                     (int64_t)(n - 1) * ldb + k < ((int64_t)1 << 32);
-  if (wide && k % HKD == 0) {
-    // a last round of at most an eighth of the CUs' tiles runs as 64 x 128
-    // sub-tiles over the whole of k (no workspace needed); a larger partial
-    // round, up to half the CUs, is split along k into the workspace
-    const int cus = device_cus();
-    const int64_t last = cus > 0 ? tiles % cus : 0;
-    if (last > 0 && 8 * last <= cus) {
-      ga.full = (int32_t)(tiles - last);
-      hipStream_t s = (hipStream_t)stream;
-      if (ga.full > 0)
-        hipLaunchKernelGGL((gemm_i8_wave128_kernel<RAW, false>), dim3((unsigned)ga.full), dim3(HWAVES * 64), 0, s, ga);
-      hipLaunchKernelGGL((gemm_i8_sub_kernel<RAW>), dim3((unsigned)(last * 8)), dim3(256), 0, s, ga);
-      return check_launch(what);
-    }
-    int tail = 0, parts = 1;
-    gemm_split_plan(m, n, k, tail, parts);
-    if (parts > 1 && ws && ((uintptr_t)ws % 16) == 0 && ws_bytes >= gemm_split_bytes(tail, parts)) {
-      ga.full = (int32_t)(tiles - tail);
-      ga.nsplit = parts;
-      ga.ws = (int32_t *)ws;
-    }
-    hipStream_t s = (hipStream_t)stream;
-    if (ga.full > 0)
-      hipLaunchKernelGGL((gemm_i8_wave128_kernel<RAW, false>), dim3((unsigned)ga.full), dim3(HWAVES * 64), 0, s, ga);
-    if (ga.nsplit > 1) {
-      hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, true>), dim3((unsigned)(tail * parts)), dim3(HWAVES * 64), 0,
-                         s, ga);
-      hipLaunchKernelGGL(gemm_split_merge_kernel<RAW>, dim3((unsigned)(tail * (HBM_ / 4))), dim3(256), 0, s, ga);
-    }
-  } else {
-    hipLaunchKernelGGL(gemm_i8_kernel<RAW>, dim3((unsigned)grid), dim3(GWAVES * 64), 0, (hipStream_t)stream, ga);
-  }
+  if (wide && k % HKD == 0)
+    launch_rounds<RAW, false>(ga, ws, ws_bytes, (hipStream_t)stream);
+  else
+    hipLaunchKernelGGL(gemm_i8_kernel<RAW>, dim3((unsigned)tiles), dim3(GWAVES * 64), 0, (hipStream_t)stream, ga);
   return check_launch(what);
 }
 
 // The GEMM with the SwiGLU epilogue: out[m][n / 2] from gate / up rows
-// interleaved in blocks of 128 (see the GLU kernel).  Only the one-wave-per-
-// SIMD kernel and its k-split carry the GLU epilogue.
+// interleaved in blocks of 128 (see the GLU kernels).
 int launch_gemm_glu(void *out, const int8_t *a, const int8_t *b, const float *as, const float *bs, const void *bias,
                     int32_t m, int32_t n, int32_t k, int64_t lda, int64_t ldb, int64_t ldo, void *ws,
                     int64_t ws_bytes, void *stream) {
@@ -1041,22 +1205,7 @@ int launch_gemm_glu(void *out, const int8_t *a, const int8_t *b, const float *as
   const int64_t tiles = (int64_t)((m + HBM_ - 1) / HBM_) * (n / HBN);
   GArgs ga{a, b, out, as, bs, (const uint16_t *)bias, m, n, k, lda, ldb, ldo, (m + HBM_ - 1) / HBM_, n / HBN,
            (int32_t)(((uintptr_t)bs % 16) == 0 && ((uintptr_t)bias % 8) == 0), 1, (int32_t)tiles, 1, nullptr};
-  int tail = 0, parts = 1;
-  gemm_split_plan(m, n, k, tail, parts);
-  if (parts > 1 && ws && ((uintptr_t)ws % 16) == 0 && ws_bytes >= gemm_split_bytes(tail, parts)) {
-    ga.full = (int32_t)(tiles - tail);
-    ga.nsplit = parts;
-    ga.ws = (int32_t *)ws;
-  }
-  hipStream_t s = (hipStream_t)stream;
-  if (ga.full > 0)
-    hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, false, true>), dim3((unsigned)ga.full), dim3(HWAVES * 64), 0, s,
-                       ga);
-  if (ga.nsplit > 1) {
-    hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, true>), dim3((unsigned)(tail * parts)), dim3(HWAVES * 64), 0, s,
-                       ga);
-    hipLaunchKernelGGL(gemm_split_merge_glu_kernel, dim3((unsigned)(tail * (HBM_ / 8))), dim3(256), 0, s, ga);
-  }
+  launch_rounds<false, true>(ga, ws, ws_bytes, (hipStream_t)stream);
   return check_launch(what);
 }
 
