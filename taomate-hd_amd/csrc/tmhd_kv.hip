@@ -5,25 +5,18 @@
 #include <algorithm>
 
 #include "tmhd_internal.h"
+#include "tmhd_pack.h"
 
 namespace tmhd {
 namespace {
 
-constexpr int kTile = 64;
+constexpr int kTile = kPackTile;
 
 // ---------------------------------------------------------------------------
-// tmhd_kv_pack: one workgroup = 64 slot positions of one head, D threads.
-// Position p of the slot is: data row (p - dst) if dst <= p < dst + n,
-// zero if dst + n <= p < zero_to, untouched otherwise.  A launch packs up to
-// kMaxRanges row ranges: the 64-position blocks from blk0 on are range i's (one
-// launch per range instead cost 5 to 9 us each for ranges of 77 to 1,337 rows).
-// WITH_K false: the key rows of data positions are left to the caller (the
-// staged norm + RoPE kernel writes them); zero positions are still cleared.
-// Thread (dc, g) owns the 16-byte column chunk dc (columns 8 dc .. 8 dc + 7) of
-// the 8 tokens stored at transposed positions 8 g .. 8 g + 7: it loads their 8
-// key and value chunks, copies the keys, and transposes the 8 x 8 block of
-// values in registers into 8 transposed rows of 8 positions. A wave's loads
-// and stores are whole 128-byte lines; no LDS and no barrier.
+// tmhd_kv_pack: one workgroup = 64 slot positions of one head, D threads (see
+// pack_block).  A launch packs up to kMaxRanges row ranges: the 64-position
+// blocks from blk0 on are range i's (one launch per range instead cost 5 to
+// 9 us each for ranges of 77 to 1,337 rows).
 constexpr int kMaxRanges = 32;
 struct PackRange {
   const int32_t *rows;
@@ -40,70 +33,13 @@ struct PackArgs {
   PackRange r[kMaxRanges];
 };
 
-template <int D, bool WITH_K = true>
+template <int D>
 __global__ void __launch_bounds__(D) kv_pack_kernel(const PackArgs a) {
   int ri = 0;
   while (ri + 1 < a.nranges && (int)blockIdx.x >= a.r[ri + 1].blk0) ++ri;
   const PackRange &R = a.r[ri];
-  const uint16_t *__restrict__ k = a.k, *__restrict__ v = a.v;
-  const int32_t *__restrict__ rows = R.rows;
-  uint16_t *__restrict__ ks = a.ks, *__restrict__ vts = a.vts;
-  const int64_t ts = a.ts, hs = a.hs, khs = a.khs, vhs = a.vhs;
-  const int32_t vrs = a.vrs, row0 = R.row0, n = R.n, dst = R.dst, zero_to = R.zero_to;
-  const int h = blockIdx.y;
-  const int p0 = R.p_begin + ((int)blockIdx.x - R.blk0) * kTile;
-  const int dc = threadIdx.x >> 3, g = threadIdx.x & 7;
-  int tok[8], kind[8];  // kind: 0 untouched, 1 data, 2 zero
-  bool all = true, any = false;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    tok[e] = vt_position(g * 8 + e);
-    const int p = p0 + tok[e];
-    kind[e] = (p >= dst && p < dst + n) ? 1 : (p >= dst + n && p < zero_to) ? 2 : 0;
-    all = all && kind[e] != 0;
-    any = any || kind[e] != 0;
-  }
-  i32x4 kv[8], vv[8];
-  if (n > 0) {
-    // every load issued before any is used: indices are clamped into the
-    // data rows and the values of other positions are dropped afterwards
-    int64_t src[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int i = min(max(p0 + tok[e] - dst, 0), n - 1);
-      src[e] = (int64_t)(rows ? rows[i] : row0 + i) * ts + (int64_t)h * hs + dc * 8;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if constexpr (WITH_K) kv[e] = *(const i32x4 *)(k + src[e]);
-      vv[e] = *(const i32x4 *)(v + src[e]);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (n == 0 || kind[e] != 1) kv[e] = vv[e] = i32x4{0, 0, 0, 0};
-  uint16_t *kout = ks + (int64_t)h * khs + dc * 8;
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (WITH_K ? kind[e] != 0 : kind[e] == 2) *(i32x4 *)(kout + (int64_t)(p0 + tok[e]) * D) = kv[e];
-  if (!any) return;
-  uint16_t *out = vts + (int64_t)h * vhs + (int64_t)(dc * 8) * vrs + p0 + g * 8;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    i32x4 w;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const uint32_t x = (uint32_t)vv[2 * m][j >> 1], y = (uint32_t)vv[2 * m + 1][j >> 1];
-      w[m] = (int)((j & 1) ? (x >> 16) | (y & 0xffff0000u) : (x & 0xffffu) | (y << 16));
-    }
-    if (all) {
-      *(i32x4 *)(out + (int64_t)j * vrs) = w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (kind[e] != 0) out[(int64_t)j * vrs + e] = (uint16_t)((uint32_t)w[e >> 1] >> (16 * (e & 1)));
-    }
-  }
+  pack_block<D, true>(a.k, a.v, a.ts, a.hs, R.rows, R.row0, R.n, a.ks, a.vts, a.khs, a.vhs, a.vrs, R.dst, R.zero_to,
+                        R.p_begin + ((int)blockIdx.x - R.blk0) * kTile, blockIdx.y, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -436,7 +372,7 @@ namespace tmhd {
 int kv_pack_ranges(const void *k, const void *v, int64_t token_stride, int64_t head_stride,
                    const tmhd_pack_range *ranges, int32_t nranges, void *k_slot, void *vt_slot, int64_t k_head_stride,
                    int64_t vt_head_stride, int32_t vt_row_stride, int32_t heads, int32_t head_dim, void *stream,
-                   bool with_k, bool check_only) {
+                   bool check_only) {
   if (head_dim != 64 && head_dim != 128) return set_error(TMHD_ERR_UNSUPPORTED, "kv_pack: head_dim %d", head_dim);
   if (nranges < 0 || (nranges > 0 && !ranges)) return set_error(TMHD_ERR_INVALID, "kv_pack: %d ranges", nranges);
   bool data = false;
@@ -471,14 +407,10 @@ int kv_pack_ranges(const void *k, const void *v, int64_t token_stride, int64_t h
     if (blocks == 0 || (a.nranges < kMaxRanges && i + 1 < nranges)) continue;
     const dim3 grid(blocks, heads);
     hipStream_t s = (hipStream_t)stream;
-    if (head_dim == 128 && with_k)
-      hipLaunchKernelGGL((kv_pack_kernel<128, true>), grid, dim3(128), 0, s, a);
-    else if (head_dim == 128)
-      hipLaunchKernelGGL((kv_pack_kernel<128, false>), grid, dim3(128), 0, s, a);
-    else if (with_k)
-      hipLaunchKernelGGL((kv_pack_kernel<64, true>), grid, dim3(64), 0, s, a);
+    if (head_dim == 128)
+      hipLaunchKernelGGL(kv_pack_kernel<128>, grid, dim3(128), 0, s, a);
     else
-      hipLaunchKernelGGL((kv_pack_kernel<64, false>), grid, dim3(64), 0, s, a);
+      hipLaunchKernelGGL(kv_pack_kernel<64>, grid, dim3(64), 0, s, a);
     if (int st = check_launch("tmhd_kv_pack")) return st;
     a.nranges = 0;
     blocks = 0;
@@ -489,10 +421,10 @@ int kv_pack_ranges(const void *k, const void *v, int64_t token_stride, int64_t h
 int kv_pack(const void *k, const void *v, int64_t token_stride, int64_t head_stride, const int32_t *rows,
             int32_t row0, int32_t n, void *k_slot, void *vt_slot, int64_t k_head_stride, int64_t vt_head_stride,
             int32_t vt_row_stride, int32_t dst, int32_t zero_to, int32_t heads, int32_t head_dim, void *stream,
-            bool with_k, bool check_only) {
+            bool check_only) {
   const tmhd_pack_range r{rows, row0, n, dst, zero_to};
   return kv_pack_ranges(k, v, token_stride, head_stride, &r, 1, k_slot, vt_slot, k_head_stride, vt_head_stride,
-                        vt_row_stride, heads, head_dim, stream, with_k, check_only);
+                        vt_row_stride, heads, head_dim, stream, check_only);
 }
 
 }  // namespace tmhd
@@ -502,7 +434,7 @@ extern "C" int tmhd_kv_pack_ranges(const void *k, const void *v, int64_t token_s
                                    int64_t k_head_stride, int64_t vt_head_stride, int32_t vt_row_stride,
                                    int32_t heads, int32_t head_dim, void *stream) {
   return tmhd::kv_pack_ranges(k, v, token_stride, head_stride, ranges, n_ranges, k_slot, vt_slot, k_head_stride,
-                              vt_head_stride, vt_row_stride, heads, head_dim, stream, true, false);
+                              vt_head_stride, vt_row_stride, heads, head_dim, stream, false);
 }
 
 extern "C" int tmhd_kv_pack(const void *k, const void *v, int64_t token_stride, int64_t head_stride,
@@ -510,7 +442,7 @@ extern "C" int tmhd_kv_pack(const void *k, const void *v, int64_t token_stride, 
                             int64_t k_head_stride, int64_t vt_head_stride, int32_t vt_row_stride, int32_t dst,
                             int32_t zero_to, int32_t heads, int32_t head_dim, void *stream) {
   return tmhd::kv_pack(k, v, token_stride, head_stride, rows, row0, n, k_slot, vt_slot, k_head_stride, vt_head_stride,
-                       vt_row_stride, dst, zero_to, heads, head_dim, stream, true, false);
+                       vt_row_stride, dst, zero_to, heads, head_dim, stream, false);
 }
 
 namespace tmhd {

@@ -28,6 +28,7 @@
 #include <math.h>
 
 #include "tmhd_internal.h"
+#include "tmhd_pack.h"
 
 namespace tmhd {
 namespace {
@@ -58,23 +59,79 @@ struct RopeArgs {
   uint16_t *kslot;
   int64_t kslot_hs;
   int32_t stage_row0, stage_n, stage_dst;
+  // and the workgroups from vblk0 on pack the range's V and clear the rows up to stage_zero_to
+  uint16_t *vslot;
+  int64_t vslot_hs;
+  int32_t vslot_rs, stage_zero_to, stage_p0;
   // SEND only: rows go to the Ulysses send buffer instead of back in place:
   // row (t, part p, head h) at ((dest * 3 + p) * tokens + t) * L + l (layout 0)
-  // or ((dest * tokens + t) * 3 + p) * L + l (layout 1), dest = h / L, l = h % L
+  // or ((dest * tokens + t) * 3 + p) * L + l (layout 1), dest = h / L, l = h % L;
+  // the workgroups from vblk0 on copy the V rows and clear the padded heads
   uint16_t *send;
   int32_t send_local, send_layout;
+  int32_t vblk0;  // STAGE / SEND: workgroups of the Q / K rows
 };
 
 constexpr int kRopeUnroll = 4;  // row groups per wave; one per lane of a quad in the inverse RMS pass
+
+// V and padding part of SEND: 4 tokens of one destination, 64 lanes each.
+template <int D>
+__device__ __forceinline__ void send_v(const RopeArgs &a, int b) {
+  constexpr int CPH = D / 8;  // 16-byte chunks per head row
+  const int tblocks = (a.tokens + 3) / 4, dest = b / tblocks, lane = threadIdx.x & 63;
+  const int t = (b - dest * tblocks) * 4 + (threadIdx.x >> 6);
+  if (t >= a.tokens) return;
+  const int row_chunks = a.send_local * CPH;
+  const int real = min(a.heads - dest * a.send_local, a.send_local) * CPH;  // <= 0: a rank of padding only
+  auto row = [&](int p) {
+    const int64_t r = a.send_layout == 0 ? (int64_t)(dest * 3 + p) * a.tokens + t : ((int64_t)dest * a.tokens + t) * 3 + p;
+    return (i32x4 *)(a.send + r * row_chunks * 8);
+  };
+  const uint16_t *in = a.src + (int64_t)t * a.src_stride + (int64_t)(2 * a.heads + dest * a.send_local) * D;
+  i32x4 *out = row(2);
+  for (int c = lane; c < row_chunks; c += 64) {
+    if (c < real) {
+      out[c] = *(const i32x4 *)(in + c * 8);
+    } else {
+      out[c] = i32x4{0, 0, 0, 0};
+      row(0)[c] = i32x4{0, 0, 0, 0};
+      row(1)[c] = i32x4{0, 0, 0, 0};
+    }
+  }
+}
 
 // TABLE: cos / sin of channel d at cos_sin[positions[t]][d % h] and [h + d % h]
 // (the merged-projection form); otherwise at cos[t][d] and sin[t][d].
 // NORM false: the rotation alone, applied to the input values (no RMSNorm).
 // STAGE: the K rows of the staged token range also go to the slot.
 // SEND: the rows go to the Ulysses send buffer (the source is left as it is).
+// STAGE and SEND take the V rows along in the same launch: a launch of their
+// own drained the chip twice and left a gap.  Calls of both kinds were, before
+// and after: send of 3,063 tokens, 40 heads of 128, to 4 ranks 45.3 and 40.1 us
+// (188 MB moved: 37 us at the rate of a large copy); W8A8 projection and stage
+// of 4,836 tokens, 28 heads of 128, 290 and 286 us.
 template <int D, bool TABLE, bool NORM = true, bool STAGE = false, bool SEND = false>
 __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const RopeArgs a) {
 #pragma clang fp contract(off)
+  if constexpr (STAGE || SEND) {
+    if ((int)blockIdx.x >= a.vblk0) {
+      const int b = blockIdx.x - a.vblk0;
+      if constexpr (SEND) {
+        send_v<D>(a, b);
+      } else {
+        // 256 / D heads of one 64-position block
+        constexpr int HPB = 256 / D;
+        const int hblocks = (a.heads + HPB - 1) / HPB, tile = b / hblocks;
+        const int h = (b - tile * hblocks) * HPB + threadIdx.x / D;
+        const uint16_t *v = a.src + (int64_t)2 * a.heads * D;
+        if (h < a.heads)
+          pack_block<D, false>(v, v, a.src_stride, D, nullptr, a.stage_row0, a.stage_n, a.kslot, a.vslot, a.kslot_hs,
+                               a.vslot_hs, a.vslot_rs, a.stage_dst, a.stage_zero_to, a.stage_p0 + tile * kPackTile, h,
+                               threadIdx.x % D);
+      }
+      return;
+    }
+  }
   constexpr int LPR = D / 8;     // lanes per row
   constexpr int RPW = 64 / LPR;  // rows per wave and group
   constexpr int U = kRopeUnroll;
@@ -233,12 +290,15 @@ int rope_rows_check(const RopeArgs &a, int head_dim, const char *what) {
   return TMHD_OK;
 }
 
-int launch_rope(const RopeArgs &a, int head_dim, bool table, void *stream, const char *what, bool norm = true,
-                bool stage = false, bool send = false) {
+// vblocks: workgroups of the V part (stage, send)
+int launch_rope(RopeArgs a, int head_dim, bool table, void *stream, const char *what, bool norm = true,
+                bool stage = false, bool send = false, int64_t vblocks = 0) {
   if (int st = rope_rows_check(a, head_dim, what)) return st;
   const int64_t rows = (int64_t)a.tokens * a.parts * a.heads;
   const int rows_per_block = 4 * kRopeUnroll * (64 / (head_dim / 8));
-  const dim3 grid((unsigned)((rows + rows_per_block - 1) / rows_per_block)), block(256);
+  const int64_t row_blocks = (rows + rows_per_block - 1) / rows_per_block;
+  const dim3 grid((unsigned)(row_blocks + vblocks)), block(256);
+  a.vblk0 = (int32_t)row_blocks;
   hipStream_t s = (hipStream_t)stream;
   if (send) {
     if (head_dim == 128)
@@ -339,7 +399,7 @@ extern "C" int tmhd_qkv_norm_rope_stage(void *qkv, int32_t tokens, int32_t heads
   // the slot arguments are those of tmhd_kv_pack over the K and V thirds (checked before any launch)
   if (int st = kv_pack(base + width, base + 2 * width, row_stride, head_dim, nullptr, stage_row0, stage_n, k_slot,
                        vt_slot, k_head_stride, vt_head_stride, vt_row_stride, dst, zero_to, heads, head_dim, stream,
-                       false, true))
+                       true))
     return st;
   if (tokens > 0) {
     a.kslot = (uint16_t *)k_slot;
@@ -347,10 +407,21 @@ extern "C" int tmhd_qkv_norm_rope_stage(void *qkv, int32_t tokens, int32_t heads
     a.stage_row0 = stage_row0;
     a.stage_n = stage_n;
     a.stage_dst = dst;
-    if (int st = launch_rope(a, head_dim, true, stream, what, true, stage_n > 0)) return st;
+    a.vslot = (uint16_t *)vt_slot;
+    a.vslot_hs = vt_head_stride;
+    a.vslot_rs = vt_row_stride;
+    a.stage_zero_to = zero_to;
+    a.stage_p0 = dst / kPackTile * kPackTile;
+    if (stage_n > 0) {
+      const int64_t end = dst + stage_n > zero_to ? dst + stage_n : zero_to, heads_per_block = 256 / head_dim;
+      const int64_t hblocks = (heads + heads_per_block - 1) / heads_per_block;
+      const int64_t vblocks = (end - a.stage_p0 + kPackTile - 1) / kPackTile * hblocks;
+      return launch_rope(a, head_dim, true, stream, what, true, true, false, vblocks);
+    }
+    if (int st = launch_rope(a, head_dim, true, stream, what)) return st;
   }
   return kv_pack(base + width, base + 2 * width, row_stride, head_dim, nullptr, stage_row0, stage_n, k_slot, vt_slot,
-                 k_head_stride, vt_head_stride, vt_row_stride, dst, zero_to, heads, head_dim, stream, false, false);
+                 k_head_stride, vt_head_stride, vt_row_stride, dst, zero_to, heads, head_dim, stream, false);
 }
 
 extern "C" int tmhd_qk_norm_rope(const void *value, int32_t tokens, int32_t heads, int32_t head_dim,
@@ -434,13 +505,12 @@ extern "C" int tmhd_ulysses_qkv_norm_rope_send(const void *qkv, int64_t row_stri
   if (int st = qkv_rope_args(&a, const_cast<void *>(qkv), tokens, heads, head_dim, row_stride, q_weight, k_weight,
                              cos_sin, cos_sin_stride, cos_sin_rows, rotary_dim, positions, eps, what))
     return st;
-  // V rows and the zero padding heads come from the plain send (checked before any launch)
-  if (int st = ulysses_send(qkv, row_stride, tokens, heads, head_dim, world, layout, out, 4, stream, true)) return st;
+  // checked as the plain send is
+  if (int st = ulysses_send(qkv, row_stride, tokens, heads, head_dim, world, layout, out, stream, true)) return st;
   if (tokens == 0) return TMHD_OK;
   a.dst = nullptr;
   a.send = (uint16_t *)out;
   a.send_local = (heads + world - 1) / world;
   a.send_layout = layout;
-  if (int st = launch_rope(a, head_dim, true, stream, what, true, false, true)) return st;
-  return ulysses_send(qkv, row_stride, tokens, heads, head_dim, world, layout, out, 4, stream, false);
+  return launch_rope(a, head_dim, true, stream, what, true, false, true, (int64_t)((tokens + 3) / 4) * world);
 }

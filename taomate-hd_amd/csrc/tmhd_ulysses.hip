@@ -33,7 +33,6 @@ struct SendArgs {
   int64_t src_stride;  // elements between tokens of the merged projection
   uint16_t *dst;
   int32_t tokens, heads, local, world, layout;
-  int32_t copy_parts;  // bit p: copy the real heads of part p (padded heads are always zeroed)
 };
 
 template <int D>
@@ -45,13 +44,12 @@ __global__ void __launch_bounds__(256) ulysses_send_kernel(const SendArgs a) {
   const int row_chunks = a.local * CPH;
   const int64_t row = a.layout == 0 ? (int64_t)dp * a.tokens + t : ((int64_t)dest * a.tokens + t) * 3 + p;
   i32x4 *out = (i32x4 *)(a.dst + row * row_chunks * 8);
-  const bool copy = (a.copy_parts >> p) & 1;
   const uint16_t *in = a.src + (int64_t)t * a.src_stride + ((int64_t)p * a.heads + (int64_t)dest * a.local) * D;
   const int real = min(a.heads - dest * a.local, a.local) * CPH;  // chunks of real heads in this row
   for (int c = threadIdx.x; c < row_chunks; c += 64) {
     if (c >= real)
       out[c] = i32x4{0, 0, 0, 0};
-    else if (copy)
+    else
       out[c] = *(const i32x4 *)(in + c * 8);
   }
 }
@@ -113,10 +111,10 @@ dim3 row_grid(int32_t tokens, int32_t y) {
 
 }  // namespace
 
-// Shared with the norm + RoPE send (tmhd_rope.hip): validates and launches
-// the plain send for the parts in copy_parts.
+// Shared with the norm + RoPE send (tmhd_rope.hip): validates and, unless
+// check_only, launches the plain send.
 int ulysses_send(const void *qkv, int64_t row_stride, int32_t tokens, int32_t heads, int32_t head_dim,
-                 int32_t world, int32_t layout, void *out, int32_t copy_parts, void *stream, bool check_only) {
+                 int32_t world, int32_t layout, void *out, void *stream, bool check_only) {
   const char *what = "tmhd_ulysses_qkv_send";
   if (int st = check_world(tokens, heads, head_dim, world, what)) return st;
   if (layout != 0 && layout != 1) return set_error(TMHD_ERR_INVALID, "%s: layout %d (0 or 1)", what, layout);
@@ -132,7 +130,7 @@ int ulysses_send(const void *qkv, int64_t row_stride, int32_t tokens, int32_t he
   const int64_t qb = ((int64_t)(tokens - 1) * row_stride + (int64_t)3 * heads * head_dim) * 2;
   if (o0 < q0 + qb && q0 < o0 + ob) return set_error(TMHD_ERR_INVALID, "%s: out overlaps qkv", what);
   if (check_only) return TMHD_OK;
-  SendArgs a{(const uint16_t *)qkv, row_stride, (uint16_t *)out, tokens, heads, local, world, layout, copy_parts};
+  SendArgs a{(const uint16_t *)qkv, row_stride, (uint16_t *)out, tokens, heads, local, world, layout};
   const dim3 grid = row_grid(tokens, 3 * world), block(64, kRowsPerBlock);
   hipStream_t s = (hipStream_t)stream;
   if (head_dim == 128)
@@ -146,7 +144,7 @@ int ulysses_send(const void *qkv, int64_t row_stride, int32_t tokens, int32_t he
 
 extern "C" int tmhd_ulysses_qkv_send(const void *qkv, int64_t row_stride, int32_t tokens, int32_t heads,
                                      int32_t head_dim, int32_t world, int32_t layout, void *out, void *stream) {
-  return tmhd::ulysses_send(qkv, row_stride, tokens, heads, head_dim, world, layout, out, 7, stream, false);
+  return tmhd::ulysses_send(qkv, row_stride, tokens, heads, head_dim, world, layout, out, stream, false);
 }
 
 extern "C" int tmhd_ulysses_qkv_receive(const void *recv, int32_t tokens, int32_t local_heads, int32_t head_dim,
