@@ -77,19 +77,21 @@ class _Rows:
     """A set of packed-sequence rows: a contiguous range or a device row list
     (built from in-range host rows, so its kernels skip the range check)."""
 
-    def __init__(self, torch: Any, absolute: list[int], device: Any) -> None:
-        self.count = len(absolute)
-        self.start = absolute[0] if absolute else 0
-        self.contiguous = bool(absolute) and absolute[-1] - absolute[0] + 1 == len(absolute)
+    def __init__(self, torch: Any, absolute: Any, device: Any) -> None:
+        """``absolute``: ascending int64 CPU tensor."""
+        self.count = int(absolute.numel())
+        self.start = int(absolute[0]) if self.count else 0
+        self.contiguous = self.count > 0 and int(absolute[-1]) - self.start + 1 == self.count
+        self.host = absolute
         self.index = None
         if self.count and not self.contiguous:
-            self.index = torch.tensor(absolute, dtype=torch.int32, device=device)
+            self.index = absolute.to(device=device, dtype=torch.int32)
 
     @classmethod
     def range(cls, start: int, stop: int) -> "_Rows":
         """The rows ``start .. stop``."""
         rows = cls.__new__(cls)
-        rows.count, rows.start, rows.contiguous, rows.index = stop - start, start, True, None
+        rows.count, rows.start, rows.contiguous, rows.index, rows.host = stop - start, start, True, None, None
         return rows
 
     def query_kwargs(self) -> dict[str, Any]:
@@ -107,10 +109,6 @@ class _Rows:
             return {"rows": self.index, "rows_checked": True}
         return {"row0": self.start, "count": self.count}
 
-    def host_rows(self) -> list[int]:
-        if self.index is None:
-            return list(range(self.start, self.start + self.count))
-        return self.index.cpu().tolist()
 
 
 class StreamingAttentionHook:
@@ -279,9 +277,8 @@ class StreamingAttentionHook:
     def _document_rows(self, torch: Any, index: int, start: int, stop: int, commit_mask: Any) -> tuple[_Rows, _Rows]:
         rows = self._live_document_rows.get(index)
         if rows is None:
-            mask = commit_mask[start:stop].detach().cpu().tolist()
-            condition = [start + i for i, m in enumerate(mask) if not m]
-            media = [start + i for i, m in enumerate(mask) if m]
+            mask = commit_mask[start:stop].detach().cpu()
+            condition, media = (m.nonzero().view(-1) + start for m in (mask.logical_not(), mask))
             rows = (_Rows(torch, condition, commit_mask.device), _Rows(torch, media, commit_mask.device))
             self._live_document_rows[index] = rows
         return rows
@@ -505,8 +502,7 @@ class StreamingAttentionHook:
         """True when the active commit staged exactly ``rows`` (cached per step)."""
         hit = self._staged_match.get(index)
         if hit is None:
-            staged = self.cache.staged_rows_host()
-            hit = staged is not None and sorted(staged) == rows.host_rows()
+            hit = self.cache.staged_rows_equal(rows.host)
             self._staged_match[index] = hit
         return hit
 
