@@ -654,386 +654,386 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   Cursor cur = cursor_begin(args, blockIdx.x);
   Frag fr;
   while (cursor_next(kernel_args(), cur, fr)) {
-  const KArgs &a = kernel_args();
-  const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index (uniform)
-  const Prob &P = a.pr[fr.p];
-  const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
-  const int q0 = fr.qt * kBM + w * kQW;  // first query row of this wave
+    const KArgs &a = kernel_args();
+    const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index (uniform)
+    const Prob &P = a.pr[fr.p];
+    const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
+    const int q0 = fr.qt * kBM + w * kQW;  // first query row of this wave
 
-  // per-lane LDS read offsets from smem (bytes; k-step, key half, buffer and db parts are uniform/immediate)
-  const uint32_t kro = lr * KRS + g * 16;
-  const uint32_t vro = 3 * KT + lr * VRS + g * 16;
+    // per-lane LDS read offsets from smem (bytes; k-step, key half, buffer and db parts are uniform/immediate)
+    const uint32_t kro = lr * KRS + g * 16;
+    const uint32_t vro = 3 * KT + lr * VRS + g * 16;
 
-  // Tile loads.  LDS slot c (16 bytes) of a tile holds chunk c % (n + 1) of
-  // row c / (n + 1) (n data chunks per row; the pad chunk repeats the row's
-  // last chunk).  Per-lane source offsets: keys are tile-invariant; values
-  // keep (row, chunk) packed and scale by the segment's row stride per load.
-  uint32_t koff[KWL], vrc[VWL];
-  // Wave w loads blocks w, w + 4, ...; in the last round the waves past the
-  // tile's end repeat its last block (same bytes to the same place), so that
-  // every wave issues the same, branch-free sequence.
-  auto kblk = [&](int i) { return min(w + i * kWaves, NKL - 1); };
-  auto vblk = [&](int i) { return min(w + i * kWaves, NVL - 1); };
+    // Tile loads.  LDS slot c (16 bytes) of a tile holds chunk c % (n + 1) of
+    // row c / (n + 1) (n data chunks per row; the pad chunk repeats the row's
+    // last chunk).  Per-lane source offsets: keys are tile-invariant; values
+    // keep (row, chunk) packed and scale by the segment's row stride per load.
+    uint32_t koff[KWL], vrc[VWL];
+    // Wave w loads blocks w, w + 4, ...; in the last round the waves past the
+    // tile's end repeat its last block (same bytes to the same place), so that
+    // every wave issues the same, branch-free sequence.
+    auto kblk = [&](int i) { return min(w + i * kWaves, NKL - 1); };
+    auto vblk = [&](int i) { return min(w + i * kWaves, NVL - 1); };
 #pragma unroll
-  for (int i = 0; i < KWL; ++i) {
-    const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
-    koff[i] = row * KROW + chunk * 16;
-  }
+    for (int i = 0; i < KWL; ++i) {
+      const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
+      koff[i] = row * KROW + chunk * 16;
+    }
 #pragma unroll
-  for (int i = 0; i < VWL; ++i) {
-    const int c = vblk(i) * 64 + lane, row = c / 9, chunk = min(c - row * 9, 7);
-    vrc[i] = (uint32_t)row | ((uint32_t)chunk << 20);
-  }
-  // load n of a tile: K blocks first (n < KWL), then V blocks
-  constexpr int NLD = KWL + VWL;
-  static_assert(NLD <= 16, "slot plan bounds");
-  // tile loads spread over the first NS regions (with the early exponentials in the last
-  // regions, 0.7% faster than 1.5 NS in two same-box A/Bs, 2 NS 1.3% slower)
-  // early exponentials: pairs 0..3 of each query half (same-box A/B at 768p, 6 runs each, against
-  // pair 0 placed before the second E / C units: 8.098 -> 7.995 ms; pair 0 alone, placed last:
-  // 8.036 ms; against no early units, pair 0 gave about 1%)
-  constexpr int NX = 8;
-  constexpr SlotPlan PL = make_plan(NQK, NPV, DB, NLD, NS, NX);  // sub-tiles with tile loads
-  constexpr SlotPlan PN = make_plan(NQK, NPV, DB, 0, 1, NX);     // sub-tiles without
-  static_assert(plan_valid(PL, NQK, NPV, DB, NLD, NS, NX) && plan_valid(PN, NQK, NPV, DB, 0, 1, NX),
-                "slot plan orderings");
-  // value source offsets for the V^T row stride of the current load segment
-  uint32_t voff[VWL];
-  auto set_voff = [&](uint32_t vrs2) {
+    for (int i = 0; i < VWL; ++i) {
+      const int c = vblk(i) * 64 + lane, row = c / 9, chunk = min(c - row * 9, 7);
+      vrc[i] = (uint32_t)row | ((uint32_t)chunk << 20);
+    }
+    // load n of a tile: K blocks first (n < KWL), then V blocks
+    constexpr int NLD = KWL + VWL;
+    static_assert(NLD <= 16, "slot plan bounds");
+    // tile loads spread over the first NS regions (with the early exponentials in the last
+    // regions, 0.7% faster than 1.5 NS in two same-box A/Bs, 2 NS 1.3% slower)
+    // early exponentials: pairs 0..3 of each query half (same-box A/B at 768p, 6 runs each, against
+    // pair 0 placed before the second E / C units: 8.098 -> 7.995 ms; pair 0 alone, placed last:
+    // 8.036 ms; against no early units, pair 0 gave about 1%)
+    constexpr int NX = 8;
+    constexpr SlotPlan PL = make_plan(NQK, NPV, DB, NLD, NS, NX);  // sub-tiles with tile loads
+    constexpr SlotPlan PN = make_plan(NQK, NPV, DB, 0, 1, NX);     // sub-tiles without
+    static_assert(plan_valid(PL, NQK, NPV, DB, NLD, NS, NX) && plan_valid(PN, NQK, NPV, DB, 0, 1, NX),
+                  "slot plan orderings");
+    // value source offsets for the V^T row stride of the current load segment
+    uint32_t voff[VWL];
+    auto set_voff = [&](uint32_t vrs2) {
 #pragma unroll
-    for (int i = 0; i < VWL; ++i) voff[i] = (vrc[i] & 0xfffffu) * vrs2 + ((vrc[i] >> 20) << 4);
-  };
-  auto load_one = [&](int n, const char *kbase, uint32_t kdst, const char *vbase, uint32_t vdst) {
-    if (n < KWL)
-      load_lds16(kbase, koff[n], kdst + kblk(n) * 1024);
-    else
-      load_lds16(vbase, voff[n - KWL], vdst + vblk(n - KWL) * 1024);
-  };
-  auto load_k = [&](const Stream &S, int buf) {
-    const char *base = S.kb + (int64_t)S.t * (kBN * KROW);
+      for (int i = 0; i < VWL; ++i) voff[i] = (vrc[i] & 0xfffffu) * vrs2 + ((vrc[i] >> 20) << 4);
+    };
+    auto load_one = [&](int n, const char *kbase, uint32_t kdst, const char *vbase, uint32_t vdst) {
+      if (n < KWL)
+        load_lds16(kbase, koff[n], kdst + kblk(n) * 1024);
+      else
+        load_lds16(vbase, voff[n - KWL], vdst + vblk(n - KWL) * 1024);
+    };
+    auto load_k = [&](const Stream &S, int buf) {
+      const char *base = S.kb + (int64_t)S.t * (kBN * KROW);
 #pragma unroll
-    for (int i = 0; i < KWL; ++i) load_lds16(base, koff[i], lds0 + buf * KT + kblk(i) * 1024);
-  };
-  auto load_v = [&](const Stream &S, int buf) {
-    const char *base = S.vb + S.t * (kBN * 2);
+      for (int i = 0; i < KWL; ++i) load_lds16(base, koff[i], lds0 + buf * KT + kblk(i) * 1024);
+    };
+    auto load_v = [&](const Stream &S, int buf) {
+      const char *base = S.vb + S.t * (kBN * 2);
 #pragma unroll
-    for (int i = 0; i < VWL; ++i)
-      load_lds16(base, (vrc[i] & 0xfffffu) * S.vrs2 + ((vrc[i] >> 20) << 4),
-                 lds0 + 3 * KT + buf * VT + vblk(i) * 1024);
-  };
-  auto lds_read = [&](uint32_t off) { return *(const i32x4 *)(smem + off); };
-  // valid keys of a stream's current tile (1 .. 64)
-  auto tile_valid = [](const Stream &S) { return min(S.tok - S.t * kBN, kBN); };
+      for (int i = 0; i < VWL; ++i)
+        load_lds16(base, (vrc[i] & 0xfffffu) * S.vrs2 + ((vrc[i] >> 20) << 4),
+                   lds0 + 3 * KT + buf * VT + vblk(i) * 1024);
+    };
+    auto lds_read = [&](uint32_t off) { return *(const i32x4 *)(smem + off); };
+    // valid keys of a stream's current tile (1 .. 64)
+    auto tile_valid = [](const Stream &S) { return min(S.tok - S.t * kBN, kBN); };
 
-  // keys of a 32-key sub-tile at or beyond nvalid (relative to the sub-tile) -> -inf
-  // (element r of a lane holds key 8 (r / 4) + 4 g + r % 4; comparing the
-  // constant part with nvalid - 4 g keeps no per-element constants in registers)
-  auto mask_sub = [&](f32x16 (&s)[2], int nvalid) {
-    const int t = nvalid - 4 * g;
+    // keys of a 32-key sub-tile at or beyond nvalid (relative to the sub-tile) -> -inf
+    // (element r of a lane holds key 8 (r / 4) + 4 g + r % 4; comparing the
+    // constant part with nvalid - 4 g keeps no per-element constants in registers)
+    auto mask_sub = [&](f32x16 (&s)[2], int nvalid) {
+      const int t = nvalid - 4 * g;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (8 * (r >> 2) + (r & 3) >= t) s[hf][r] = -INFINITY;
+    };
+    auto sub_max = [](const f32x16 &s) {
+      float m = fmaxf(s[0], s[1]);
+#pragma unroll
+      for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(s[r], s[r + 1]));
+      return m;
+    };
+
+    // ---- prologue: K(0..2), V(0..1) resident; S = scores of sub-tile 0 (minus m)
+    Stream t0, t1, t2, t3;
+    stream_seek<false>(t0, a, h, P.seg0, send, fr.ta);
+    t1 = t0;
+    stream_next<false>(t1, a, h, send);
+    t2 = t1;
+    stream_next<false>(t2, a, h, send);
+    t3 = t2;
+    stream_next<false>(t3, a, h, send);
+    load_k(t0, 0);
+    load_k(t1, 1);
+    load_v(t0, 0);
+    // ---- query operands of both 32-row halves (B operands of S^T = K Q^T), pinned in AGPRs;
+    // all loads issued (behind the tile loads) before any is used, rows past the
+    // end re-read the last row and are zeroed
+    i32x4 qv[2][QST];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const int ql = min(q0 + hf * 32 + lr, P.lq - 1);
+      const int row = P.q_rows ? P.q_rows[ql] : P.q_row0 + ql;
+      const uint16_t *p = P.q + (int64_t)row * a.qts + (int64_t)h * a.qhs + g * 8;
+#pragma unroll
+      for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 16);
+    }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const bool live = q0 + hf * 32 + lr < P.lq;
+#pragma unroll
+      for (int st = 0; st < QST; ++st) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t u = (uint32_t)qv[hf][st][e];
+          const uint32_t x = pack_bf16x2(__uint_as_float(u << 16) * a.c, __uint_as_float(u & 0xffff0000u) * a.c);
+          qv[hf][st][e] = live ? (int)x : 0;
+        }
+        qpin(hf * QST + st, qv[hf][st]);
+      }
+    }
+
+    f32x16 o[2][DB];  // block hf * DB + db lives in AGPRs a[16 b, 16 b + 15]
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + (r & 3) >= t) s[hf][r] = -INFINITY;
-  };
-  auto sub_max = [](const f32x16 &s) {
-    float m = fmaxf(s[0], s[1]);
+      for (int db = 0; db < DB; ++db) {
 #pragma unroll
-    for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(s[r], s[r + 1]));
-    return m;
-  };
-
-  // ---- prologue: K(0..2), V(0..1) resident; S = scores of sub-tile 0 (minus m)
-  Stream t0, t1, t2, t3;
-  stream_seek<false>(t0, a, h, P.seg0, send, fr.ta);
-  t1 = t0;
-  stream_next<false>(t1, a, h, send);
-  t2 = t1;
-  stream_next<false>(t2, a, h, send);
-  t3 = t2;
-  stream_next<false>(t3, a, h, send);
-  load_k(t0, 0);
-  load_k(t1, 1);
-  load_v(t0, 0);
-  // ---- query operands of both 32-row halves (B operands of S^T = K Q^T), pinned in AGPRs;
-  // all loads issued (behind the tile loads) before any is used, rows past the
-  // end re-read the last row and are zeroed
-  i32x4 qv[2][QST];
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const int ql = min(q0 + hf * 32 + lr, P.lq - 1);
-    const int row = P.q_rows ? P.q_rows[ql] : P.q_row0 + ql;
-    const uint16_t *p = P.q + (int64_t)row * a.qts + (int64_t)h * a.qhs + g * 8;
-#pragma unroll
-    for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 16);
-  }
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const bool live = q0 + hf * 32 + lr < P.lq;
-#pragma unroll
-    for (int st = 0; st < QST; ++st) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t u = (uint32_t)qv[hf][st][e];
-        const uint32_t x = pack_bf16x2(__uint_as_float(u << 16) * a.c, __uint_as_float(u & 0xffff0000u) * a.c);
-        qv[hf][st][e] = live ? (int)x : 0;
+        for (int r = 0; r < 16; ++r) o[hf][db][r] = 0.0f;
+        opin(hf * DB + db, o[hf][db]);
       }
-      qpin(hf * QST + st, qv[hf][st]);
-    }
-  }
+    float lsum[2] = {0.0f, 0.0f};
+    float mref[2];   // running reference of each query half (log2 units)
+    f32x16 negm[2];  // -mref in every element, the score accumulator start
+    const f32x16 zero16 = {};
 
-  f32x16 o[2][DB];  // block hf * DB + db lives in AGPRs a[16 b, 16 b + 15]
+    // valid keys of tiles j, j+1, j+2, j+3
+    int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
+    wait_vmem();
+    __syncthreads();
+    // scores (minus m) of the current and the next sub-tile: sub-tiles alternate
+    // between the two sets, so no copies are needed
+    f32x16 sA[2], sB[2];
+    {
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
+      for (int st = 0; st < QST; ++st) {
+        const i32x4 kv = lds_read(kro + st * 32);
 #pragma unroll
-    for (int db = 0; db < DB; ++db) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[hf][db][r] = 0.0f;
-      opin(hf * DB + db, o[hf][db]);
-    }
-  float lsum[2] = {0.0f, 0.0f};
-  float mref[2];   // running reference of each query half (log2 units)
-  f32x16 negm[2];  // -mref in every element, the score accumulator start
-  const f32x16 zero16 = {};
-
-  // valid keys of tiles j, j+1, j+2, j+3
-  int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
-  wait_vmem();
-  __syncthreads();
-  // scores (minus m) of the current and the next sub-tile: sub-tiles alternate
-  // between the two sets, so no copies are needed
-  f32x16 sA[2], sB[2];
-  {
-#pragma unroll
-    for (int st = 0; st < QST; ++st) {
-      const i32x4 kv = lds_read(kro + st * 32);
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        if (st == 0) sA[hf] = zero16;
-        qk_bf16(hf * QST + st, hf, false, sA[hf], kv, qv[hf][st], zero16);
-      }
-    }
-    mfma_drain();
-    if (nv0 < 32) mask_sub(sA, nv0);
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const float lm = sub_max(sA[hf]);
-      mref[hf] = fmaxf(lm, __shfl_xor(lm, 32));
-      sA[hf] -= mref[hf];
-      negm[hf] = -mref[hf];
-      npin(hf, negm[hf]);
-    }
-  }
-  // load streams: K of tile j+3 and V of tile j+2, issued after the barrier of iteration j
-  Stream sk = t3, sv = t2;
-  // operands of the first slots of sub-tile (0, keys 32..63)
-  i32x4 pre[LA];
-#pragma unroll
-  for (int i = 0; i < LA; ++i) pre[i] = lds_read(kro + 32 * KRS + i * 32);
-
-  int j = 0, b0 = 0, b1 = 1, b2 = 2;  // LDS buffers of tiles j, j+1, j+2
-  // exp2 of the first NX / 2 pairs of each query half of the next sub-tile's
-  // scores (the X units of the slot plan; for sub-tile 0, here)
-  float pe_early[16][2];
-  auto early_exp = [&](f32x16 (&s)[2], int hf) {
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if ((u & 7) < NX / 2 && (u >> 3) == hf) {
-        pe_early[u][0] = __builtin_amdgcn_exp2f(s[hf][2 * (u & 7)]);
-        pe_early[u][1] = __builtin_amdgcn_exp2f(s[hf][2 * (u & 7) + 1]);
-      }
-  };
-  early_exp(sA, 0);
-  early_exp(sA, 1);
-
-  // One 32-key sub-tile, software-pipelined by hand in NS slots of two MFMAs
-  // (one per query half), each MFMA fenced with the units the plan puts in
-  // front of it so that the compiler keeps their order.  Slot i also issues
-  // the LDS operand read of slot i + LA:
-  //   slots [0, NQK):  scores of the next sub-tile, K rows at kb (k-step st = i);
-  //   slots [NQK, NS): O^T += V^T P^T of the current sub-tile, V chunks at vb.
-  // sc: scores (minus m) of the current sub-tile; sn: receives those of the
-  // next.  nvs: valid keys of the next sub-tile (<= 0: none); live: the next
-  // sub-tile exists.
-  // With loads, the slots also issue the tile loads of the iteration.  pre:
-  // the operands of the first LA slots, read by the previous sub-tile; on
-  // return, those of the next sub-tile (K rows at kbn).
-  auto sub_tile = [&](f32x16 (&sc)[2], f32x16 (&sn)[2], uint32_t kb, uint32_t vb, uint32_t kbn, i32x4 (&pre)[LA],
-                      int nvs, bool live, auto loads_c, const char *lkb, uint32_t lkd, const char *lvb,
-                      uint32_t lvd) {
-    auto read_op = [&](int i) -> i32x4 {
-      if (i < NQK) return lds_read(kb + i * 32);
-      const int p = i - NQK, st = p / DB, db = p % DB;
-      return lds_read(vb + db * 32 * VRS + 2 * st * 16);
-    };
-    i32x4 ops[NS];
-    i32x4 pk[2][2];  // P as bf16 pairs: [query half][16-key step]
-    float ts[2] = {0.0f, 0.0f};
-    float lm[2] = {-INFINITY, -INFINITY};
-#pragma unroll
-    for (int i = 0; i < LA; ++i) ops[i] = pre[i];
-    float pe[2][8][2];  // exponentials of the current sub-tile, between their E and C units
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if ((u & 7) < NX / 2) {  // computed by the previous sub-tile (or the prologue)
-        pe[u >> 3][u & 7][0] = pe_early[u][0];
-        pe[u >> 3][u & 7][1] = pe_early[u][1];
-      }
-#pragma clang loop unroll(full)
-    for (int r = 0; r < 2 * NS; ++r) {
-      const int i = r >> 1, hr = r & 1;  // slot, query half of MFMA r
-      constexpr bool loads = decltype(loads_c)::value;
-      constexpr SlotPlan pl = loads ? PL : PN;
-      if (hr == 1) {
-        if (i + LA < NS)
-          ops[i + LA] = read_op(i + LA);
-        else
-          pre[i + LA - NS] = lds_read(kbn + (i + LA - NS) * 32);
-      }
-      if (loads)
-#pragma unroll
-        for (int n = 0; n < NLD; ++n)
-          if (pl.l[n] == r) load_one(n, lkb, lkd, lvb, lvd);
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.e[u] == r) {
-          const int hf = u >> 3, q = u & 7;
-          pe[hf][q][0] = __builtin_amdgcn_exp2f(sc[hf][2 * q]);
-          pe[hf][q][1] = __builtin_amdgcn_exp2f(sc[hf][2 * q + 1]);
-          asm volatile("" : "+v"(pe[hf][q][0]), "+v"(pe[hf][q][1]));  // keeps them in this region
+        for (int hf = 0; hf < 2; ++hf) {
+          if (st == 0) sA[hf] = zero16;
+          qk_bf16(hf * QST + st, hf, false, sA[hf], kv, qv[hf][st], zero16);
         }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.c[u] == r) {
-          const int hf = u >> 3, q = u & 7;
-          int pr = (int)pack_bf16x2(pe[hf][q][0], pe[hf][q][1]);
-          ts[hf] += pe[hf][q][0];
-          ts[hf] += pe[hf][q][1];
-          asm volatile("" : "+v"(pr), "+v"(ts[hf]));  // keeps the pack and the row sum in this region
-          pk[hf][q >> 2][q & 3] = pr;
-        }
-      if (r == 2 * NQK + kGuardRegionOffset) {
-        // first reads of the next sub-tile's scores: at least 12 wait states
-        // after the last score MFMA (the MFMA in front of this region and
-        // these 10); naming the results keeps every read below
-        asm volatile("s_nop 10" : "+v"(sn[0]), "+v"(sn[1]));
       }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.m[u] == r) {
-          const int hf = u >> 3, rr = (u & 7) * 2;
-          lm[hf] = fmaxf(lm[hf], fmaxf(sn[hf][rr], sn[hf][rr + 1]));
-          asm volatile("" : "+v"(lm[hf]));  // keeps the row maximum in this region
-        }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.x[u] == r) {
-          const int hf = u >> 3, q = u & 7;
-          pe_early[u][0] = __builtin_amdgcn_exp2f(sn[hf][2 * q]);
-          pe_early[u][1] = __builtin_amdgcn_exp2f(sn[hf][2 * q + 1]);
-          asm volatile("" : "+v"(pe_early[u][0]), "+v"(pe_early[u][1]));  // keeps them in this region
-        }
-      __builtin_amdgcn_sched_barrier(0);
-      if (i < NQK) {
-        qk_bf16(hr * QST + i, hr, i == 0, sn[hr], ops[i], qv[hr][i], negm[hr]);
-      } else {
-        const int p = i - NQK, st = p / DB, db = p % DB;
-        // the P group read here was packed in the region in front of the previous MFMA
-        bool fresh = false;
-#pragma unroll
-        for (int q = 4 * st; q < 4 * st + 4; ++q) fresh = fresh || pl.c[hr * 8 + q] >= r - 1;
-        pv(hr * DB + db, fresh, o[hr][db], ops[i], pk[hr][st]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    lsum[0] += ts[0];
-    lsum[1] += ts[1];
-    if (!live) return;
-    if (nvs < 32) {
-      int nvo = nvs;  // opaque inside the branch: keeps the comparisons from being hoisted
-      asm volatile("" : "+s"(nvo));
-      mask_sub(sn, nvo);
-      lm[0] = sub_max(sn[0]);
-      lm[1] = sub_max(sn[1]);
-      early_exp(sn, 0);  // of the masked scores
-      early_exp(sn, 1);
-    }
-    if (__any(fmaxf(lm[0], lm[1]) > kLazyRescale)) {
       mfma_drain();
+      if (nv0 < 32) mask_sub(sA, nv0);
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
-        const float cm = fmaxf(lm[hf], __shfl_xor(lm[hf], 32));
-        const float delta = fmaxf(cm, 0.0f);
-        const float alpha = __builtin_amdgcn_exp2f(-delta);
-        lsum[hf] *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) orescale(hf * DB + db, o[hf][db], alpha);
-        sn[hf] -= delta;
-        mref[hf] += delta;
-        early_exp(sn, hf);  // against the new reference
+        const float lm = sub_max(sA[hf]);
+        mref[hf] = fmaxf(lm, __shfl_xor(lm, 32));
+        sA[hf] -= mref[hf];
         negm[hf] = -mref[hf];
         npin(hf, negm[hf]);
       }
-      asm volatile("s_nop 2" ::: "memory");
     }
-  };
+    // load streams: K of tile j+3 and V of tile j+2, issued after the barrier of iteration j
+    Stream sk = t3, sv = t2;
+    // operands of the first slots of sub-tile (0, keys 32..63)
+    i32x4 pre[LA];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) pre[i] = lds_read(kro + 32 * KRS + i * 32);
 
-  // Iteration j: sub-tiles (j, keys 0..31) and (j, keys 32..63).  LDS holds
-  // K(j), K(j+1) and V(j); the loads issued from its first sub-tile's slots
-  // (K(j+2) over K(j-1), V(j+1) over V(j-2)) are waited for at its end.
-  // tile loads issued from the slots of iteration j: K(j+2) and V(j+1)
-  const char *lkb = t2.kb + (int64_t)t2.t * (kBN * KROW), *lvb = t1.vb + t1.t * (kBN * 2);
-  uint32_t lvrs = t1.vrs2, lkd = lds0 + 2 * KT, lvd = lds0 + 3 * KT + 1 * VT;
-  set_voff(lvrs);
-  for (;;) {
-    // P of keys 0..31 of tile j; scores of keys 32..63 of tile j come next
-    sub_tile(sA, sB, kro + b0 * KT + 32 * KRS, vro + b0 * VT, kro + b1 * KT, pre, nv0 - 32, true, std::true_type{}, lkb,
-             lkd, lvb, lvd);
-    // P of keys 32..63 of tile j; scores of keys 0..31 of tile j+1 come next
-    // (after the last tile they read a stale in-bounds buffer and are unused)
-    const bool more = j + 1 < cnt;
-    sub_tile(sB, sA, kro + b1 * KT, vro + b0 * VT + 4 * 16, kro + b1 * KT + 32 * KRS, pre, nv1, more, std::false_type{},
-             lkb, lkd, lvb, lvd);
-    if (!more) break;
-    ++j;
-    wait_vmem();     // this wave's loads of K(j+1), V(j) (tile numbers of the new j)
-    __syncthreads();  // everyone's loads landed; K(j-1) and V(j-2) are free
-    nv0 = nv1;
-    nv1 = nv2;
-    nv2 = nv3;
-    const int bf = b0;  // buffers rotate: tile t lives in buffer t % 3
-    b0 = b1;
-    b1 = b2;
-    b2 = bf;
-    // K(j+2) over K(j-1) and V(j+1) over V(j-2), issued from the slots of the
-    // first sub-tile of iteration j
-    lkb = sk.kb + (int64_t)sk.t * (kBN * KROW);
-    lkd = lds0 + b2 * KT;
-    lvb = sv.vb + sv.t * (kBN * 2);
-    if (sv.vrs2 != lvrs) {  // the value loads moved to a segment with another row stride
-      lvrs = sv.vrs2;
-      set_voff(lvrs);
+    int j = 0, b0 = 0, b1 = 1, b2 = 2;  // LDS buffers of tiles j, j+1, j+2
+    // exp2 of the first NX / 2 pairs of each query half of the next sub-tile's
+    // scores (the X units of the slot plan; for sub-tile 0, here)
+    float pe_early[16][2];
+    auto early_exp = [&](f32x16 (&s)[2], int hf) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if ((u & 7) < NX / 2 && (u >> 3) == hf) {
+          pe_early[u][0] = __builtin_amdgcn_exp2f(s[hf][2 * (u & 7)]);
+          pe_early[u][1] = __builtin_amdgcn_exp2f(s[hf][2 * (u & 7) + 1]);
+        }
+    };
+    early_exp(sA, 0);
+    early_exp(sA, 1);
+
+    // One 32-key sub-tile, software-pipelined by hand in NS slots of two MFMAs
+    // (one per query half), each MFMA fenced with the units the plan puts in
+    // front of it so that the compiler keeps their order.  Slot i also issues
+    // the LDS operand read of slot i + LA:
+    //   slots [0, NQK):  scores of the next sub-tile, K rows at kb (k-step st = i);
+    //   slots [NQK, NS): O^T += V^T P^T of the current sub-tile, V chunks at vb.
+    // sc: scores (minus m) of the current sub-tile; sn: receives those of the
+    // next.  nvs: valid keys of the next sub-tile (<= 0: none); live: the next
+    // sub-tile exists.
+    // With loads, the slots also issue the tile loads of the iteration.  pre:
+    // the operands of the first LA slots, read by the previous sub-tile; on
+    // return, those of the next sub-tile (K rows at kbn).
+    auto sub_tile = [&](f32x16 (&sc)[2], f32x16 (&sn)[2], uint32_t kb, uint32_t vb, uint32_t kbn, i32x4 (&pre)[LA],
+                        int nvs, bool live, auto loads_c, const char *lkb, uint32_t lkd, const char *lvb,
+                        uint32_t lvd) {
+      auto read_op = [&](int i) -> i32x4 {
+        if (i < NQK) return lds_read(kb + i * 32);
+        const int p = i - NQK, st = p / DB, db = p % DB;
+        return lds_read(vb + db * 32 * VRS + 2 * st * 16);
+      };
+      i32x4 ops[NS];
+      i32x4 pk[2][2];  // P as bf16 pairs: [query half][16-key step]
+      float ts[2] = {0.0f, 0.0f};
+      float lm[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ops[i] = pre[i];
+      float pe[2][8][2];  // exponentials of the current sub-tile, between their E and C units
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if ((u & 7) < NX / 2) {  // computed by the previous sub-tile (or the prologue)
+          pe[u >> 3][u & 7][0] = pe_early[u][0];
+          pe[u >> 3][u & 7][1] = pe_early[u][1];
+        }
+#pragma clang loop unroll(full)
+      for (int r = 0; r < 2 * NS; ++r) {
+        const int i = r >> 1, hr = r & 1;  // slot, query half of MFMA r
+        constexpr bool loads = decltype(loads_c)::value;
+        constexpr SlotPlan pl = loads ? PL : PN;
+        if (hr == 1) {
+          if (i + LA < NS)
+            ops[i + LA] = read_op(i + LA);
+          else
+            pre[i + LA - NS] = lds_read(kbn + (i + LA - NS) * 32);
+        }
+        if (loads)
+#pragma unroll
+          for (int n = 0; n < NLD; ++n)
+            if (pl.l[n] == r) load_one(n, lkb, lkd, lvb, lvd);
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.e[u] == r) {
+            const int hf = u >> 3, q = u & 7;
+            pe[hf][q][0] = __builtin_amdgcn_exp2f(sc[hf][2 * q]);
+            pe[hf][q][1] = __builtin_amdgcn_exp2f(sc[hf][2 * q + 1]);
+            asm volatile("" : "+v"(pe[hf][q][0]), "+v"(pe[hf][q][1]));  // keeps them in this region
+          }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.c[u] == r) {
+            const int hf = u >> 3, q = u & 7;
+            int pr = (int)pack_bf16x2(pe[hf][q][0], pe[hf][q][1]);
+            ts[hf] += pe[hf][q][0];
+            ts[hf] += pe[hf][q][1];
+            asm volatile("" : "+v"(pr), "+v"(ts[hf]));  // keeps the pack and the row sum in this region
+            pk[hf][q >> 2][q & 3] = pr;
+          }
+        if (r == 2 * NQK + kGuardRegionOffset) {
+          // first reads of the next sub-tile's scores: at least 12 wait states
+          // after the last score MFMA (the MFMA in front of this region and
+          // these 10); naming the results keeps every read below
+          asm volatile("s_nop 10" : "+v"(sn[0]), "+v"(sn[1]));
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.m[u] == r) {
+            const int hf = u >> 3, rr = (u & 7) * 2;
+            lm[hf] = fmaxf(lm[hf], fmaxf(sn[hf][rr], sn[hf][rr + 1]));
+            asm volatile("" : "+v"(lm[hf]));  // keeps the row maximum in this region
+          }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.x[u] == r) {
+            const int hf = u >> 3, q = u & 7;
+            pe_early[u][0] = __builtin_amdgcn_exp2f(sn[hf][2 * q]);
+            pe_early[u][1] = __builtin_amdgcn_exp2f(sn[hf][2 * q + 1]);
+            asm volatile("" : "+v"(pe_early[u][0]), "+v"(pe_early[u][1]));  // keeps them in this region
+          }
+        __builtin_amdgcn_sched_barrier(0);
+        if (i < NQK) {
+          qk_bf16(hr * QST + i, hr, i == 0, sn[hr], ops[i], qv[hr][i], negm[hr]);
+        } else {
+          const int p = i - NQK, st = p / DB, db = p % DB;
+          // the P group read here was packed in the region in front of the previous MFMA
+          bool fresh = false;
+#pragma unroll
+          for (int q = 4 * st; q < 4 * st + 4; ++q) fresh = fresh || pl.c[hr * 8 + q] >= r - 1;
+          pv(hr * DB + db, fresh, o[hr][db], ops[i], pk[hr][st]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      lsum[0] += ts[0];
+      lsum[1] += ts[1];
+      if (!live) return;
+      if (nvs < 32) {
+        int nvo = nvs;  // opaque inside the branch: keeps the comparisons from being hoisted
+        asm volatile("" : "+s"(nvo));
+        mask_sub(sn, nvo);
+        lm[0] = sub_max(sn[0]);
+        lm[1] = sub_max(sn[1]);
+        early_exp(sn, 0);  // of the masked scores
+        early_exp(sn, 1);
+      }
+      if (__any(fmaxf(lm[0], lm[1]) > kLazyRescale)) {
+        mfma_drain();
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          const float cm = fmaxf(lm[hf], __shfl_xor(lm[hf], 32));
+          const float delta = fmaxf(cm, 0.0f);
+          const float alpha = __builtin_amdgcn_exp2f(-delta);
+          lsum[hf] *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) orescale(hf * DB + db, o[hf][db], alpha);
+          sn[hf] -= delta;
+          mref[hf] += delta;
+          early_exp(sn, hf);  // against the new reference
+          negm[hf] = -mref[hf];
+          npin(hf, negm[hf]);
+        }
+        asm volatile("s_nop 2" ::: "memory");
+      }
+    };
+
+    // Iteration j: sub-tiles (j, keys 0..31) and (j, keys 32..63).  LDS holds
+    // K(j), K(j+1) and V(j); the loads issued from its first sub-tile's slots
+    // (K(j+2) over K(j-1), V(j+1) over V(j-2)) are waited for at its end.
+    // tile loads issued from the slots of iteration j: K(j+2) and V(j+1)
+    const char *lkb = t2.kb + (int64_t)t2.t * (kBN * KROW), *lvb = t1.vb + t1.t * (kBN * 2);
+    uint32_t lvrs = t1.vrs2, lkd = lds0 + 2 * KT, lvd = lds0 + 3 * KT + 1 * VT;
+    set_voff(lvrs);
+    for (;;) {
+      // P of keys 0..31 of tile j; scores of keys 32..63 of tile j come next
+      sub_tile(sA, sB, kro + b0 * KT + 32 * KRS, vro + b0 * VT, kro + b1 * KT, pre, nv0 - 32, true, std::true_type{}, lkb,
+               lkd, lvb, lvd);
+      // P of keys 32..63 of tile j; scores of keys 0..31 of tile j+1 come next
+      // (after the last tile they read a stale in-bounds buffer and are unused)
+      const bool more = j + 1 < cnt;
+      sub_tile(sB, sA, kro + b1 * KT, vro + b0 * VT + 4 * 16, kro + b1 * KT + 32 * KRS, pre, nv1, more, std::false_type{},
+               lkb, lkd, lvb, lvd);
+      if (!more) break;
+      ++j;
+      wait_vmem();     // this wave's loads of K(j+1), V(j) (tile numbers of the new j)
+      __syncthreads();  // everyone's loads landed; K(j-1) and V(j-2) are free
+      nv0 = nv1;
+      nv1 = nv2;
+      nv2 = nv3;
+      const int bf = b0;  // buffers rotate: tile t lives in buffer t % 3
+      b0 = b1;
+      b1 = b2;
+      b2 = bf;
+      // K(j+2) over K(j-1) and V(j+1) over V(j-2), issued from the slots of the
+      // first sub-tile of iteration j
+      lkb = sk.kb + (int64_t)sk.t * (kBN * KROW);
+      lkd = lds0 + b2 * KT;
+      lvb = sv.vb + sv.t * (kBN * 2);
+      if (sv.vrs2 != lvrs) {  // the value loads moved to a segment with another row stride
+        lvrs = sv.vrs2;
+        set_voff(lvrs);
+      }
+      lvd = lds0 + 3 * KT + b1 * VT;
+      sv = sk;
+      stream_next<false>(sk, a, h, send);
+      nv3 = tile_valid(sk);
     }
-    lvd = lds0 + 3 * KT + b1 * VT;
-    sv = sk;
-    stream_next<false>(sk, a, h, send);
-    nv3 = tile_valid(sk);
-  }
 
-  // ---- epilogue: O = O^T / l, written token-major (4 consecutive d per store).
-  // The last iteration's tile loads (into buffers nobody reads) land before the
-  // workgroup's LDS is released.
-  wait_vmem();
-  mfma_drain();
+    // ---- epilogue: O = O^T / l, written token-major (4 consecutive d per store).
+    // The last iteration's tile loads (into buffers nobody reads) land before the
+    // workgroup's LDS is released.
+    wait_vmem();
+    mfma_drain();
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
+    for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-    for (int db = 0; db < DB; ++db) opin(hf * DB + db, o[hf][db]);
-  __syncthreads();  // every wave's tile reads and loads are done
-  write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
-  // the next item's first tile loads overwrite rows that other waves may still read
-  __syncthreads();
+      for (int db = 0; db < DB; ++db) opin(hf * DB + db, o[hf][db]);
+    __syncthreads();  // every wave's tile reads and loads are done
+    write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
+    // the next item's first tile loads overwrite rows that other waves may still read
+    __syncthreads();
   }
 }
 
@@ -1164,360 +1164,360 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
   Cursor cur = cursor_begin(args, blockIdx.x);
   Frag fr;
   while (cursor_next(kernel_args(), cur, fr)) {
-  const KArgs &a = kernel_args();
-  const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const Prob &P = a.pr[fr.p];
-  const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
-  const int q0 = fr.qt * kBM + w * kQW;
+    const KArgs &a = kernel_args();
+    const int tid = lane_in_group(), lane = tid & 63, lr = lane & 31, g = lane >> 5;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Prob &P = a.pr[fr.p];
+    const int h = fr.h, cnt = fr.tb - fr.ta, send = P.seg_end;
+    const int q0 = fr.qt * kBM + w * kQW;
 
-  const uint32_t kro = lr * KRS + g * 16;
-  const uint32_t vro = 3 * KT + lr * VRS + g * 16;
+    const uint32_t kro = lr * KRS + g * 16;
+    const uint32_t vro = 3 * KT + lr * VRS + g * 16;
 
-  // per-lane source offsets of the tile loads, kept in LDS (the registers are
-  // the loop's scarcest resource) and read at the start of each loading
-  // sub-tile: keys tile-invariant; values for the V^T row stride of the
-  // segment the loop's value loads are in, rewritten when that changes
-  auto kblk = [&](int i) { return min(w + i * kWaves, NKL - 1); };
-  auto vblk = [&](int i) { return min(w + i * kWaves, NVL - 1); };
-  constexpr int NLD = KWL + VWL;
-  static_assert(NLD <= 8, "eight offset words per lane");
-  auto koff_of = [&](int i) {
-    const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
-    return (uint32_t)(row * KROW + chunk * 16);
-  };
+    // per-lane source offsets of the tile loads, kept in LDS (the registers are
+    // the loop's scarcest resource) and read at the start of each loading
+    // sub-tile: keys tile-invariant; values for the V^T row stride of the
+    // segment the loop's value loads are in, rewritten when that changes
+    auto kblk = [&](int i) { return min(w + i * kWaves, NKL - 1); };
+    auto vblk = [&](int i) { return min(w + i * kWaves, NVL - 1); };
+    constexpr int NLD = KWL + VWL;
+    static_assert(NLD <= 8, "eight offset words per lane");
+    auto koff_of = [&](int i) {
+      const int c = kblk(i) * 64 + lane, row = c / (KCPR + 1), chunk = min(c - row * (KCPR + 1), KCPR - 1);
+      return (uint32_t)(row * KROW + chunk * 16);
+    };
 #pragma unroll
-  for (int i = 0; i < KWL; ++i) *(uint32_t *)(smem + TAB + tid * 32 + i * 4) = koff_of(i);
-  auto read_tab = [&](uint32_t (&t)[8]) {
-    const i32x4 lo = *(const i32x4 *)(smem + TAB + tid * 32), hi = *(const i32x4 *)(smem + TAB + tid * 32 + 16);
+    for (int i = 0; i < KWL; ++i) *(uint32_t *)(smem + TAB + tid * 32 + i * 4) = koff_of(i);
+    auto read_tab = [&](uint32_t (&t)[8]) {
+      const i32x4 lo = *(const i32x4 *)(smem + TAB + tid * 32), hi = *(const i32x4 *)(smem + TAB + tid * 32 + 16);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      t[e] = (uint32_t)lo[e];
-      t[4 + e] = (uint32_t)hi[e];
-    }
-  };
-  // source offset of value load i for a V^T row stride of vrs2 bytes (row <
-  // 128 and vrs2 < 2^24, which the launch checks, so it fits 32 bits)
-  auto voff_of = [&](int i, uint32_t vrs2) {
-    const int c = vblk(i) * 64 + lane, row = c / 9, chunk = min(c - row * 9, 7);
-    return (uint32_t)row * vrs2 + (uint32_t)chunk * 16u;
-  };
-  // the lane's value offsets in the table, for row stride vrs2 (each lane
-  // reads only its own words, so no barrier is needed)
-  auto write_vtab = [&](uint32_t vrs2) {
+      for (int e = 0; e < 4; ++e) {
+        t[e] = (uint32_t)lo[e];
+        t[4 + e] = (uint32_t)hi[e];
+      }
+    };
+    // source offset of value load i for a V^T row stride of vrs2 bytes (row <
+    // 128 and vrs2 < 2^24, which the launch checks, so it fits 32 bits)
+    auto voff_of = [&](int i, uint32_t vrs2) {
+      const int c = vblk(i) * 64 + lane, row = c / 9, chunk = min(c - row * 9, 7);
+      return (uint32_t)row * vrs2 + (uint32_t)chunk * 16u;
+    };
+    // the lane's value offsets in the table, for row stride vrs2 (each lane
+    // reads only its own words, so no barrier is needed)
+    auto write_vtab = [&](uint32_t vrs2) {
 #pragma unroll
-    for (int i = 0; i < VWL; ++i) *(uint32_t *)(smem + TAB + tid * 32 + (KWL + i) * 4) = voff_of(i, vrs2);
-  };
-  // the tile loads go into the last NLD regions (at least the last 8); their
-  // offsets are read from the table TABLEAD regions before the window
-  constexpr int LWLO = 2 * NS - (NLD > 8 ? NLD : 8);
-  constexpr int TABLEAD = 4;
-  static_assert(LWLO >= TABLEAD, "room for the offset-table read");
-  constexpr SlotPlan8 PL = make_plan8(NQK, NPV, DB, NLD, LWLO);
-  constexpr SlotPlan8 PN = make_plan8(NQK, NPV, DB, 0, LWLO);
-  static_assert(plan8_valid(PL, NQK, NPV, DB, NLD, LWLO) && plan8_valid(PN, NQK, NPV, DB, 0, LWLO),
-                "slot plan orderings");
-  auto load_one = [&](int n, const uint32_t (&t)[8], const char *kbase, uint32_t kdst, const char *vbase,
-                      uint32_t vdst) {
-    if (n < KWL)
-      load_lds16(kbase, t[n], kdst + kblk(n) * 1024);
-    else
-      load_lds16(vbase, t[n], vdst + vblk(n - KWL) * 1024);
-  };
-  auto load_k = [&](const Stream &S, int buf) {
-    const char *base = S.kb + (int64_t)S.t * (kBN * KROW);
+      for (int i = 0; i < VWL; ++i) *(uint32_t *)(smem + TAB + tid * 32 + (KWL + i) * 4) = voff_of(i, vrs2);
+    };
+    // the tile loads go into the last NLD regions (at least the last 8); their
+    // offsets are read from the table TABLEAD regions before the window
+    constexpr int LWLO = 2 * NS - (NLD > 8 ? NLD : 8);
+    constexpr int TABLEAD = 4;
+    static_assert(LWLO >= TABLEAD, "room for the offset-table read");
+    constexpr SlotPlan8 PL = make_plan8(NQK, NPV, DB, NLD, LWLO);
+    constexpr SlotPlan8 PN = make_plan8(NQK, NPV, DB, 0, LWLO);
+    static_assert(plan8_valid(PL, NQK, NPV, DB, NLD, LWLO) && plan8_valid(PN, NQK, NPV, DB, 0, LWLO),
+                  "slot plan orderings");
+    auto load_one = [&](int n, const uint32_t (&t)[8], const char *kbase, uint32_t kdst, const char *vbase,
+                        uint32_t vdst) {
+      if (n < KWL)
+        load_lds16(kbase, t[n], kdst + kblk(n) * 1024);
+      else
+        load_lds16(vbase, t[n], vdst + vblk(n - KWL) * 1024);
+    };
+    auto load_k = [&](const Stream &S, int buf) {
+      const char *base = S.kb + (int64_t)S.t * (kBN * KROW);
 #pragma unroll
-    for (int i = 0; i < KWL; ++i) load_lds16(base, koff_of(i), lds0 + buf * KT + kblk(i) * 1024);
-  };
-  auto load_v = [&](const Stream &S, int buf) {
-    const char *base = S.vb + S.t * (kBN * 2);
+      for (int i = 0; i < KWL; ++i) load_lds16(base, koff_of(i), lds0 + buf * KT + kblk(i) * 1024);
+    };
+    auto load_v = [&](const Stream &S, int buf) {
+      const char *base = S.vb + S.t * (kBN * 2);
 #pragma unroll
-    for (int i = 0; i < VWL; ++i) load_lds16(base, voff_of(i, S.vrs2), lds0 + 3 * KT + buf * VT + vblk(i) * 1024);
-  };
-  auto load_ks = [&](const Stream &S) {
-    int idx = S.t >> 1;  // 128-token quant blocks hold two tiles
-    asm volatile("v_mov_b32 %0, %1" : "=v"(idx) : "s"(idx));
-    return S.ks[idx];
-  };
-  auto lds_read = [&](uint32_t off) { return *(const i32x4 *)(smem + off); };
-  auto tile_valid = [](const Stream &S) { return min(S.tok - S.t * kBN, kBN); };
-  f32x16 o[2][DB];
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[hf][db][r] = 0.0f;
-  float lsum[2] = {0.0f, 0.0f};
-  float mref[2] = {0.0f, 0.0f};  // running reference of each query column (log2 units)
-  i32x16 sn[2];                   // scores of the next sub-tile
-  // scores live as the bits of floats in i32x16 (the MFMA writes int32
-  // accumulators, converted in place)
-  auto f = [](int bits) { return __int_as_float(bits); };
-  // the wait states in front of VALU reads of MFMA results, naming the
-  // registers read after them so that no read moves above the wait
-  auto drain_scores = [&]() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" : "+v"(sn[0]), "+v"(sn[1])::"memory"); };
-  auto drain_o = [&]() {
-    mfma_drain();
+      for (int i = 0; i < VWL; ++i) load_lds16(base, voff_of(i, S.vrs2), lds0 + 3 * KT + buf * VT + vblk(i) * 1024);
+    };
+    auto load_ks = [&](const Stream &S) {
+      int idx = S.t >> 1;  // 128-token quant blocks hold two tiles
+      asm volatile("v_mov_b32 %0, %1" : "=v"(idx) : "s"(idx));
+      return S.ks[idx];
+    };
+    auto lds_read = [&](uint32_t off) { return *(const i32x4 *)(smem + off); };
+    auto tile_valid = [](const Stream &S) { return min(S.tok - S.t * kBN, kBN); };
+    f32x16 o[2][DB];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-      for (int db = 0; db < DB; ++db) asm volatile("" : "+v"(o[hf][db]));
-  };
-  auto sub_max = [&](const i32x16 &s) {
-    float m = fmaxf(f(s[0]), f(s[1]));
+      for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(f(s[r]), f(s[r + 1])));
-    return m;
-  };
+        for (int r = 0; r < 16; ++r) o[hf][db][r] = 0.0f;
+    float lsum[2] = {0.0f, 0.0f};
+    float mref[2] = {0.0f, 0.0f};  // running reference of each query column (log2 units)
+    i32x16 sn[2];                   // scores of the next sub-tile
+    // scores live as the bits of floats in i32x16 (the MFMA writes int32
+    // accumulators, converted in place)
+    auto f = [](int bits) { return __int_as_float(bits); };
+    // the wait states in front of VALU reads of MFMA results, naming the
+    // registers read after them so that no read moves above the wait
+    auto drain_scores = [&]() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" : "+v"(sn[0]), "+v"(sn[1])::"memory"); };
+    auto drain_o = [&]() {
+      mfma_drain();
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) asm volatile("" : "+v"(o[hf][db]));
+    };
+    auto sub_max = [&](const i32x16 &s) {
+      float m = fmaxf(f(s[0]), f(s[1]));
+#pragma unroll
+      for (int r = 2; r < 16; r += 2) m = fmaxf(m, fmaxf(f(s[r]), f(s[r + 1])));
+      return m;
+    };
 
 
-  // ---- prologue: K(0), K(1), V(0) resident; P of sub-tile 0
-  Stream t0, t1, t2, t3;
-  stream_seek<true>(t0, a, h, P.seg0, send, fr.ta);
-  t1 = t0;
-  stream_next<true>(t1, a, h, send);
-  t2 = t1;
-  stream_next<true>(t2, a, h, send);
-  t3 = t2;
-  stream_next<true>(t3, a, h, send);
-  load_k(t0, 0);
-  load_k(t1, 1);
-  load_v(t0, 0);
-  write_vtab(t1.vrs2);  // the loop's first value loads are of tile 1
-  // query operands of both 32-row halves (B operands of S^T = K Q^T); rows past the end re-read
-  // the last row and are zeroed
-  i32x4 qv[2][QST];
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf) {
-    const int8_t *p = P.q8 + (int64_t)h * P.q8hs + (int64_t)min(q0 + hf * 32 + lr, P.lq - 1) * D + g * 16;
-#pragma unroll
-    for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 32);
-  }
-  // softmax scale * log2(e) * query block scale (the wave's 64 rows lie in one 128-row block)
-  const float cq = a.c * P.qs[(int64_t)h * P.qshs + q0 / TMHD_QUANT_BLOCK] * (1.0f / kI8Slope);
-
-#pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
-    if (q0 + hf * 32 + lr >= P.lq)
-#pragma unroll
-      for (int st = 0; st < QST; ++st) qv[hf][st] = i32x4{0, 0, 0, 0};
-
-  // Rare path, and the first sub-tile: the scores of a 32-key sub-tile from
-  // LDS (K rows at kb) into sn, dequantised against the reference, keys at or
-  // beyond nvalid masked, the reference moved where a score exceeds it by
-  // more than 2^8 (O and l rescaled; `first`: set to the sub-tile's maximum),
-  // then the probabilities packed into pkn and their row sums added to l.
-  auto full_softmax = [&](uint32_t kb, int nvalid, float ct, bool first, i32x4 (&pkn)[2][2]) {
-#pragma unroll
-    for (int st = 0; st < QST; ++st) {
-      const i32x4 kv = lds_read(kb + st * 32);
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) qk_i8z(st == 0, sn[hf], kv, qv[hf][st]);
-    }
-    drain_scores();  // the score results, and every P.V accumulation in flight
-    const int t = nvalid - 4 * g;  // element r of a lane holds key 8 (r / 4) + 4 g + r % 4
-    float cm[2];
+    // ---- prologue: K(0), K(1), V(0) resident; P of sub-tile 0
+    Stream t0, t1, t2, t3;
+    stream_seek<true>(t0, a, h, P.seg0, send, fr.ta);
+    t1 = t0;
+    stream_next<true>(t1, a, h, send);
+    t2 = t1;
+    stream_next<true>(t2, a, h, send);
+    t3 = t2;
+    stream_next<true>(t3, a, h, send);
+    load_k(t0, 0);
+    load_k(t1, 1);
+    load_v(t0, 0);
+    write_vtab(t1.vrs2);  // the loop's first value loads are of tile 1
+    // query operands of both 32-row halves (B operands of S^T = K Q^T); rows past the end re-read
+    // the last row and are zeroed
+    i32x4 qv[2][QST];
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf) {
+      const int8_t *p = P.q8 + (int64_t)h * P.q8hs + (int64_t)min(q0 + hf * 32 + lr, P.lq - 1) * D + g * 16;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float x = fmaf(f(sn[hf][r]), ct, -fmaf(kI8MagicF, ct, mref[hf]));
-        sn[hf][r] = __float_as_int(8 * (r >> 2) + (r & 3) >= t ? -INFINITY : x);
-      }
-      const float lm = sub_max(sn[hf]);
-      cm[hf] = fmaxf(lm, __shfl_xor(lm, 32));
+      for (int st = 0; st < QST; ++st) qv[hf][st] = *(const i32x4 *)(p + st * 32);
     }
-    if (first) {
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        mref[hf] = cm[hf];  // the wave's first keys set the reference
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sn[hf][r] = __float_as_int(f(sn[hf][r]) - cm[hf]);
-      }
-    } else if (__any(fmaxf(cm[0], cm[1]) > kLazyRescale)) {
-      drain_o();
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const float delta = fmaxf(cm[hf], 0.0f);
-        const float alpha = __builtin_amdgcn_exp2f(-delta);
-        lsum[hf] *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) o[hf][db] *= alpha;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sn[hf][r] = __float_as_int(f(sn[hf][r]) - delta);
-        mref[hf] += delta;
-      }
-      asm volatile("s_nop 2" ::: "memory");  // VALU writes of O before the next accumulation
-    }
+    // softmax scale * log2(e) * query block scale (the wave's 64 rows lie in one 128-row block)
+    const float cq = a.c * P.qs[(int64_t)h * P.qshs + q0 / TMHD_QUANT_BLOCK] * (1.0f / kI8Slope);
+
 #pragma unroll
     for (int hf = 0; hf < 2; ++hf)
+      if (q0 + hf * 32 + lr >= P.lq)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const float e0 = __builtin_amdgcn_exp2f(f(sn[hf][2 * q])), e1 = __builtin_amdgcn_exp2f(f(sn[hf][2 * q + 1]));
-        pkn[hf][q >> 2][q & 3] = (int)pack_bf16x2(e0, e1);
-        lsum[hf] += e0;
-        lsum[hf] += e1;
+        for (int st = 0; st < QST; ++st) qv[hf][st] = i32x4{0, 0, 0, 0};
+
+    // Rare path, and the first sub-tile: the scores of a 32-key sub-tile from
+    // LDS (K rows at kb) into sn, dequantised against the reference, keys at or
+    // beyond nvalid masked, the reference moved where a score exceeds it by
+    // more than 2^8 (O and l rescaled; `first`: set to the sub-tile's maximum),
+    // then the probabilities packed into pkn and their row sums added to l.
+    auto full_softmax = [&](uint32_t kb, int nvalid, float ct, bool first, i32x4 (&pkn)[2][2]) {
+#pragma unroll
+      for (int st = 0; st < QST; ++st) {
+        const i32x4 kv = lds_read(kb + st * 32);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) qk_i8z(st == 0, sn[hf], kv, qv[hf][st]);
       }
-  };
-
-  int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
-  float ks2 = load_ks(t2);
-  float ks0 = load_ks(t0), ks1 = load_ks(t1);
-  wait_vmem();
-  __syncthreads();
-  ks0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks0)));
-  ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks1)));
-  i32x4 pkA[2][2], pkB[2][2];  // packed probabilities of the current / next sub-tile, alternating
-  full_softmax(kro, nv0, cq * ks0, true, pkA);
-  Stream sk = t3, sv = t2;  // K of tile j+3 and V of tile j+2, issued after the barrier of iteration j
-  i32x4 pre[LA];
+      drain_scores();  // the score results, and every P.V accumulation in flight
+      const int t = nvalid - 4 * g;  // element r of a lane holds key 8 (r / 4) + 4 g + r % 4
+      float cm[2];
 #pragma unroll
-  for (int i = 0; i < LA; ++i) pre[i] = lds_read(kro + 32 * KRS + i * 32);
-
-  int j = 0, b0 = 0, b1 = 1, b2 = 2, vb = 0;  // K buffers of tiles j, j+1, j+2; V buffer of tile j
-
-  // One 32-key sub-tile in NS slots of two MFMAs (one per query half), each
-  // MFMA fenced with the units the plan puts in front of it:
-  //   slots [0, NQK):  scores of the next sub-tile into sn, K rows at kb;
-  //   slots [NQK, NS): O^T += V^T P^T of the current sub-tile (packs pk),
-  //                    V chunks at vbo; under them the next sub-tile's
-  //                    probabilities go into pkn.
-  // Slot i issues the LDS operand read of slot i + LA; the last ones read the
-  // first operands of the sub-tile after (K rows at kbn) into pre.
-  auto sub_tile = [&](i32x4 (&pk)[2][2], i32x4 (&pkn)[2][2], uint32_t kb, uint32_t vbo, uint32_t kbn,
-                      i32x4 (&pre)[LA], int nvs, float ctn, bool live, auto loads_c, const char *lkb, uint32_t lkd,
-                      const char *lvb, uint32_t lvd) {
-    const float nbn[2] = {-fmaf(kI8MagicF, ctn, mref[0]), -fmaf(kI8MagicF, ctn, mref[1])};
-    auto read_op = [&](int i) -> i32x4 {
-      if (i < NQK) return lds_read(kb + i * 32);
-      const int p = i - NQK, st = p / DB, db = p % DB;
-      return lds_read(vbo + db * 32 * VRS + 2 * st * 16);
+      for (int hf = 0; hf < 2; ++hf) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = fmaf(f(sn[hf][r]), ct, -fmaf(kI8MagicF, ct, mref[hf]));
+          sn[hf][r] = __float_as_int(8 * (r >> 2) + (r & 3) >= t ? -INFINITY : x);
+        }
+        const float lm = sub_max(sn[hf]);
+        cm[hf] = fmaxf(lm, __shfl_xor(lm, 32));
+      }
+      if (first) {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          mref[hf] = cm[hf];  // the wave's first keys set the reference
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sn[hf][r] = __float_as_int(f(sn[hf][r]) - cm[hf]);
+        }
+      } else if (__any(fmaxf(cm[0], cm[1]) > kLazyRescale)) {
+        drain_o();
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          const float delta = fmaxf(cm[hf], 0.0f);
+          const float alpha = __builtin_amdgcn_exp2f(-delta);
+          lsum[hf] *= alpha;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) o[hf][db] *= alpha;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) sn[hf][r] = __float_as_int(f(sn[hf][r]) - delta);
+          mref[hf] += delta;
+        }
+        asm volatile("s_nop 2" ::: "memory");  // VALU writes of O before the next accumulation
+      }
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float e0 = __builtin_amdgcn_exp2f(f(sn[hf][2 * q])), e1 = __builtin_amdgcn_exp2f(f(sn[hf][2 * q + 1]));
+          pkn[hf][q >> 2][q & 3] = (int)pack_bf16x2(e0, e1);
+          lsum[hf] += e0;
+          lsum[hf] += e1;
+        }
     };
-    i32x4 ops[NS];
-    float ts[2] = {0.0f, 0.0f};
-    constexpr bool loads = decltype(loads_c)::value;
-    uint32_t tab[8];
-#pragma unroll
-    for (int i = 0; i < LA; ++i) ops[i] = pre[i];
-#pragma clang loop unroll(full)
-    for (int r = 0; r < 2 * NS; ++r) {
-      const int i = r >> 1, hr = r & 1;
-      constexpr SlotPlan8 pl = loads ? PL : PN;
-      if (hr == 1) {
-        if (i + LA < NS)
-          ops[i + LA] = read_op(i + LA);
-        else
-          pre[i + LA - NS] = lds_read(kbn + (i + LA - NS) * 32);
-      }
-      if (loads && r == LWLO - TABLEAD) read_tab(tab);
-      if (loads)
-#pragma unroll
-        for (int n = 0; n < NLD; ++n)
-          if (pl.l[n] == r) load_one(n, tab, lkb, lkd, lvb, lvd);
-      if (r == 2 * NQK + kGuardRegionOffset) {
-        // first reads of the scores: at least 12 wait states after the last
-        // score MFMA; naming them keeps every read below
-        asm volatile("s_nop 10" : "+v"(sn[0]), "+v"(sn[1]));
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.m[u] == r) {
-          const int hf = u >> 3, rr = (u & 7) * 2;
-          sn[hf][rr] = __float_as_int(fmaf(f(sn[hf][rr]), ctn, nbn[hf]));
-          sn[hf][rr + 1] = __float_as_int(fmaf(f(sn[hf][rr + 1]), ctn, nbn[hf]));
-          asm volatile("" : "+v"(sn[hf][rr]), "+v"(sn[hf][rr + 1]));
-        }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.e[u] == r) {
-          const int hf = u >> 3, q = u & 7;
-          sn[hf][2 * q] = __float_as_int(__builtin_amdgcn_exp2f(f(sn[hf][2 * q])));
-          sn[hf][2 * q + 1] = __float_as_int(__builtin_amdgcn_exp2f(f(sn[hf][2 * q + 1])));
-          asm volatile("" : "+v"(sn[hf][2 * q]), "+v"(sn[hf][2 * q + 1]));
-        }
-#pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (pl.c[u] == r) {
-          const int hf = u >> 3, q = u & 7;
-          // the adds first, then the pack: the next unit's add does not follow the
-          // statement that pins its operand directly (a wait state each otherwise)
-          ts[hf] += f(sn[hf][2 * q]);
-          ts[hf] += f(sn[hf][2 * q + 1]);
-          asm volatile("" : "+v"(ts[hf]));
-          int pr = (int)pack_bf16x2(f(sn[hf][2 * q]), f(sn[hf][2 * q + 1]));
-          asm volatile("" : "+v"(pr));
-          pkn[hf][q >> 2][q & 3] = pr;
-        }
-      __builtin_amdgcn_sched_barrier(0);
-      if (i < NQK) {
-        qk_i8z(i == 0, sn[hr], ops[i], qv[hr][i]);
-      } else {
-        const int p = i - NQK, st = p / DB, db = p % DB;
-        pv_v(o[hr][db], ops[i], pk[hr][st]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!live) return;
-    // a lane's 16 probabilities sum to at most 16 * 2^12 unless one exceeds
-    // 2^12 (or overflowed): then, or for a partial sub-tile, recompute
-    if (nvs < 32 || __any(!(fmaxf(ts[0], ts[1]) <= kRowSumBound))) {
-      int nvo = nvs;  // opaque inside the branch: keeps the comparisons from being hoisted
-      asm volatile("" : "+s"(nvo));
-      full_softmax(kb, nvo, ctn, false, pkn);
-      return;
-    }
-    lsum[0] += ts[0];
-    lsum[1] += ts[1];
-  };
 
-  // tile loads issued from the slots of iteration j: K(j+2) and V(j+1)
-  const char *lkb = t2.kb + (int64_t)t2.t * (kBN * KROW), *lvb = t1.vb + t1.t * (kBN * 2);
-  uint32_t lvrs = t1.vrs2, lkd = lds0 + 2 * KT, lvd = lds0 + 3 * KT + 1 * VT;
-  for (;;) {
-    // P of keys 0..31 of tile j; scores of keys 32..63 of tile j
-    sub_tile(pkA, pkB, kro + b0 * KT + 32 * KRS, vro + vb * VT, kro + b1 * KT, pre, nv0 - 32, cq * ks0, true,
-             std::true_type{}, lkb, lkd, lvb, lvd);
-    // P of keys 32..63 of tile j; scores of keys 0..31 of tile j+1 (after the
-    // last tile they read a stale in-bounds buffer and are unused)
-    const bool more = j + 1 < cnt;
-    sub_tile(pkB, pkA, kro + b1 * KT, vro + vb * VT + 4 * 16, kro + b1 * KT + 32 * KRS, pre, nv1, cq * ks1, more,
-             std::false_type{}, lkb, lkd, lvb, lvd);
-    if (!more) break;
-    ++j;
+    int nv0 = tile_valid(t0), nv1 = tile_valid(t1), nv2 = tile_valid(t2), nv3 = tile_valid(t3);
+    float ks2 = load_ks(t2);
+    float ks0 = load_ks(t0), ks1 = load_ks(t1);
     wait_vmem();
     __syncthreads();
-    nv0 = nv1;
-    nv1 = nv2;
-    nv2 = nv3;
-    ks0 = ks1;
-    ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks2)));  // uniform: keep it in an SGPR
-    const int bf = b0;
-    b0 = b1;
-    b1 = b2;
-    b2 = bf;
-    vb ^= 1;
-    lkb = sk.kb + (int64_t)sk.t * (kBN * KROW);
-    lkd = lds0 + b2 * KT;
-    lvb = sv.vb + sv.t * (kBN * 2);
-    if (sv.vrs2 != lvrs) {  // the value loads moved to a segment with another row stride
-      lvrs = sv.vrs2;
-      write_vtab(lvrs);
-    }
-    lvd = lds0 + 3 * KT + (vb ^ 1) * VT;
-    ks2 = load_ks(sk);
-    sv = sk;
-    stream_next<true>(sk, a, h, send);
-    nv3 = tile_valid(sk);
-  }
+    ks0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks0)));
+    ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks1)));
+    i32x4 pkA[2][2], pkB[2][2];  // packed probabilities of the current / next sub-tile, alternating
+    full_softmax(kro, nv0, cq * ks0, true, pkA);
+    Stream sk = t3, sv = t2;  // K of tile j+3 and V of tile j+2, issued after the barrier of iteration j
+    i32x4 pre[LA];
+#pragma unroll
+    for (int i = 0; i < LA; ++i) pre[i] = lds_read(kro + 32 * KRS + i * 32);
 
-  // ---- epilogue (as the kernel above)
-  wait_vmem();
-  drain_o();
-  __syncthreads();  // every wave's tile reads and loads are done
-  write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
-  // the next item's first tile loads overwrite rows that other waves may still read
-  __syncthreads();
+    int j = 0, b0 = 0, b1 = 1, b2 = 2, vb = 0;  // K buffers of tiles j, j+1, j+2; V buffer of tile j
+
+    // One 32-key sub-tile in NS slots of two MFMAs (one per query half), each
+    // MFMA fenced with the units the plan puts in front of it:
+    //   slots [0, NQK):  scores of the next sub-tile into sn, K rows at kb;
+    //   slots [NQK, NS): O^T += V^T P^T of the current sub-tile (packs pk),
+    //                    V chunks at vbo; under them the next sub-tile's
+    //                    probabilities go into pkn.
+    // Slot i issues the LDS operand read of slot i + LA; the last ones read the
+    // first operands of the sub-tile after (K rows at kbn) into pre.
+    auto sub_tile = [&](i32x4 (&pk)[2][2], i32x4 (&pkn)[2][2], uint32_t kb, uint32_t vbo, uint32_t kbn,
+                        i32x4 (&pre)[LA], int nvs, float ctn, bool live, auto loads_c, const char *lkb, uint32_t lkd,
+                        const char *lvb, uint32_t lvd) {
+      const float nbn[2] = {-fmaf(kI8MagicF, ctn, mref[0]), -fmaf(kI8MagicF, ctn, mref[1])};
+      auto read_op = [&](int i) -> i32x4 {
+        if (i < NQK) return lds_read(kb + i * 32);
+        const int p = i - NQK, st = p / DB, db = p % DB;
+        return lds_read(vbo + db * 32 * VRS + 2 * st * 16);
+      };
+      i32x4 ops[NS];
+      float ts[2] = {0.0f, 0.0f};
+      constexpr bool loads = decltype(loads_c)::value;
+      uint32_t tab[8];
+#pragma unroll
+      for (int i = 0; i < LA; ++i) ops[i] = pre[i];
+#pragma clang loop unroll(full)
+      for (int r = 0; r < 2 * NS; ++r) {
+        const int i = r >> 1, hr = r & 1;
+        constexpr SlotPlan8 pl = loads ? PL : PN;
+        if (hr == 1) {
+          if (i + LA < NS)
+            ops[i + LA] = read_op(i + LA);
+          else
+            pre[i + LA - NS] = lds_read(kbn + (i + LA - NS) * 32);
+        }
+        if (loads && r == LWLO - TABLEAD) read_tab(tab);
+        if (loads)
+#pragma unroll
+          for (int n = 0; n < NLD; ++n)
+            if (pl.l[n] == r) load_one(n, tab, lkb, lkd, lvb, lvd);
+        if (r == 2 * NQK + kGuardRegionOffset) {
+          // first reads of the scores: at least 12 wait states after the last
+          // score MFMA; naming them keeps every read below
+          asm volatile("s_nop 10" : "+v"(sn[0]), "+v"(sn[1]));
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.m[u] == r) {
+            const int hf = u >> 3, rr = (u & 7) * 2;
+            sn[hf][rr] = __float_as_int(fmaf(f(sn[hf][rr]), ctn, nbn[hf]));
+            sn[hf][rr + 1] = __float_as_int(fmaf(f(sn[hf][rr + 1]), ctn, nbn[hf]));
+            asm volatile("" : "+v"(sn[hf][rr]), "+v"(sn[hf][rr + 1]));
+          }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.e[u] == r) {
+            const int hf = u >> 3, q = u & 7;
+            sn[hf][2 * q] = __float_as_int(__builtin_amdgcn_exp2f(f(sn[hf][2 * q])));
+            sn[hf][2 * q + 1] = __float_as_int(__builtin_amdgcn_exp2f(f(sn[hf][2 * q + 1])));
+            asm volatile("" : "+v"(sn[hf][2 * q]), "+v"(sn[hf][2 * q + 1]));
+          }
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (pl.c[u] == r) {
+            const int hf = u >> 3, q = u & 7;
+            // the adds first, then the pack: the next unit's add does not follow the
+            // statement that pins its operand directly (a wait state each otherwise)
+            ts[hf] += f(sn[hf][2 * q]);
+            ts[hf] += f(sn[hf][2 * q + 1]);
+            asm volatile("" : "+v"(ts[hf]));
+            int pr = (int)pack_bf16x2(f(sn[hf][2 * q]), f(sn[hf][2 * q + 1]));
+            asm volatile("" : "+v"(pr));
+            pkn[hf][q >> 2][q & 3] = pr;
+          }
+        __builtin_amdgcn_sched_barrier(0);
+        if (i < NQK) {
+          qk_i8z(i == 0, sn[hr], ops[i], qv[hr][i]);
+        } else {
+          const int p = i - NQK, st = p / DB, db = p % DB;
+          pv_v(o[hr][db], ops[i], pk[hr][st]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (!live) return;
+      // a lane's 16 probabilities sum to at most 16 * 2^12 unless one exceeds
+      // 2^12 (or overflowed): then, or for a partial sub-tile, recompute
+      if (nvs < 32 || __any(!(fmaxf(ts[0], ts[1]) <= kRowSumBound))) {
+        int nvo = nvs;  // opaque inside the branch: keeps the comparisons from being hoisted
+        asm volatile("" : "+s"(nvo));
+        full_softmax(kb, nvo, ctn, false, pkn);
+        return;
+      }
+      lsum[0] += ts[0];
+      lsum[1] += ts[1];
+    };
+
+    // tile loads issued from the slots of iteration j: K(j+2) and V(j+1)
+    const char *lkb = t2.kb + (int64_t)t2.t * (kBN * KROW), *lvb = t1.vb + t1.t * (kBN * 2);
+    uint32_t lvrs = t1.vrs2, lkd = lds0 + 2 * KT, lvd = lds0 + 3 * KT + 1 * VT;
+    for (;;) {
+      // P of keys 0..31 of tile j; scores of keys 32..63 of tile j
+      sub_tile(pkA, pkB, kro + b0 * KT + 32 * KRS, vro + vb * VT, kro + b1 * KT, pre, nv0 - 32, cq * ks0, true,
+               std::true_type{}, lkb, lkd, lvb, lvd);
+      // P of keys 32..63 of tile j; scores of keys 0..31 of tile j+1 (after the
+      // last tile they read a stale in-bounds buffer and are unused)
+      const bool more = j + 1 < cnt;
+      sub_tile(pkB, pkA, kro + b1 * KT, vro + vb * VT + 4 * 16, kro + b1 * KT + 32 * KRS, pre, nv1, cq * ks1, more,
+               std::false_type{}, lkb, lkd, lvb, lvd);
+      if (!more) break;
+      ++j;
+      wait_vmem();
+      __syncthreads();
+      nv0 = nv1;
+      nv1 = nv2;
+      nv2 = nv3;
+      ks0 = ks1;
+      ks1 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ks2)));  // uniform: keep it in an SGPR
+      const int bf = b0;
+      b0 = b1;
+      b1 = b2;
+      b2 = bf;
+      vb ^= 1;
+      lkb = sk.kb + (int64_t)sk.t * (kBN * KROW);
+      lkd = lds0 + b2 * KT;
+      lvb = sv.vb + sv.t * (kBN * 2);
+      if (sv.vrs2 != lvrs) {  // the value loads moved to a segment with another row stride
+        lvrs = sv.vrs2;
+        write_vtab(lvrs);
+      }
+      lvd = lds0 + 3 * KT + (vb ^ 1) * VT;
+      ks2 = load_ks(sk);
+      sv = sk;
+      stream_next<true>(sk, a, h, send);
+      nv3 = tile_valid(sk);
+    }
+
+    // ---- epilogue (as the kernel above)
+    wait_vmem();
+    drain_o();
+    __syncthreads();  // every wave's tile reads and loads are done
+    write_item<D>(o, lsum, mref, a, P, fr, w, lane, smem);
+    // the next item's first tile loads overwrite rows that other waves may still read
+    __syncthreads();
   }
 }
 
@@ -1736,9 +1736,8 @@ int build_problem(const tmhd_attn_args *args, const tmhd_qk_quant *qq, bool i8, 
 
 // One launch of the problems in k (their segments set), and its merge.
 template <bool I8>
-int launch_group(KArgs &k, int nseg, int D, void *ws, int64_t ws_bytes, hipStream_t s, const char *what) {
+int launch_group(KArgs &k, int D, void *ws, int64_t ws_bytes, hipStream_t s, const char *what) {
   if (k.nprob == 0) return TMHD_OK;
-  (void)nseg;
   std::stable_sort(k.pr, k.pr + k.nprob, [](const Prob &x, const Prob &y) { return x.ntiles > y.ntiles; });
   int64_t items = 0;
   for (int p = 0; p < k.nprob; ++p) {
@@ -1799,7 +1798,7 @@ int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, int n, void
   for (int i = 0; i < n; ++i) {
     if (args[i].lq == 0) continue;
     if (k.nprob == kMaxProb || nseg + args[i].n_segments > kMaxBatchSeg) {
-      if (int st = launch_group<I8>(k, nseg, args->head_dim, args->split_workspace, args->split_workspace_bytes,
+      if (int st = launch_group<I8>(k, args->head_dim, args->split_workspace, args->split_workspace_bytes,
                                     (hipStream_t)stream, what))
         return st;
       reset();
@@ -1812,7 +1811,7 @@ int launch_attn(const tmhd_attn_args *args, const tmhd_qk_quant *qq, int n, void
     k.o16 = k.o16 && aligned(P.o, 16) && k.ots % 8 == 0 && k.ohs % 8 == 0;
     ++k.nprob;
   }
-  return launch_group<I8>(k, nseg, args->head_dim, args->split_workspace, args->split_workspace_bytes,
+  return launch_group<I8>(k, args->head_dim, args->split_workspace, args->split_workspace_bytes,
                           (hipStream_t)stream, what);
 }
 
