@@ -298,7 +298,7 @@ int tmhd_ulysses_qkv_send(const void *qkv, int64_t row_stride, int32_t tokens, i
 /*
  * tmhd_qkv_norm_rope and tmhd_ulysses_qkv_send in one pass: the normalised,
  * rotated Q / K rows go straight into the send buffer (qkv itself is left
- * unchanged); V and the padding come from the plain send.  Same results as
+ * unchanged), V and the padding in the same launch.  Same results as
  * the two calls in sequence, bit for bit.  Replaces fused_qkv_qk_norm_rope_
  * (fused_kernels.py:824-873) followed by merged_qkv_sequence_to_heads's send
  * layout (ulysses.py:183-212) in MiniMaxH3Attention.forward (layers.py:400-438).

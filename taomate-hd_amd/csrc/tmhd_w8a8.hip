@@ -14,19 +14,27 @@ namespace tmhd {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Row quantization, one wave per row.  CH = 8-element chunks held per lane
-// (one pass, row kept in registers); CH = 0 streams the row twice.
+// Row quantization, WPR waves (1 or 4, the whole workgroup) per row.  CH =
+// 8-element chunks held per lane (one pass, row kept in registers); CH = 0
+// streams the row twice.  Bound by HBM.  Four waves from 2,056 columns on: one
+// wave's registers (167 for 5,376 columns) let three rows a SIMD be in flight
+// and rows beyond 8,192 columns not be held at all.  us before / now, 331 rows:
+// 5,376 columns 4.6 / 3.6, 14,336 18.3 / 5.3; 4,836 rows: 17.2 / 14.9 (5.2
+// TB/s), 63.6 / 34.9; 12,252 rows: 35.5 / 32.4, 163 / 96.5.  Below it the wait
+// for the other waves costs more than it gives (12,252 rows of 2,048 columns
+// 13.8 us with one wave, 15.6 with four; 3,072 columns 19.9 and 19.6).
 // WEIGHT selects the weight formula of _quantize_cutlass_w8a8_weight:
 //   scale = max(amax / 127, 1e-12), q = clamp(rint(w / scale), -127, 127)
 // otherwise the activation formula:
 //   scale = amax / 127, q = sat_int8(rint(x * (127 / amax))), amax = 0 -> 0.
-template <int CH, bool WEIGHT>
+template <int WPR, int CH, bool WEIGHT>
 __global__ void __launch_bounds__(256) row_quant_kernel(int8_t *__restrict__ q, float *__restrict__ scale,
                                                         const uint16_t *__restrict__ x, int32_t rows, int32_t cols,
                                                         int64_t xs) {
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  constexpr int L = 64 * WPR;  // lanes of a row
+  const int lane = threadIdx.x % L;
+  const int row = blockIdx.x * (4 / WPR) + threadIdx.x / L;
+  if (row >= rows) return;  // WPR 4: never (a workgroup per row)
   const int nch = cols >> 3;
   const uint16_t *xr = x + (int64_t)row * xs;
   int8_t *qr = q + (int64_t)row * cols;
@@ -35,7 +43,7 @@ __global__ void __launch_bounds__(256) row_quant_kernel(int8_t *__restrict__ q, 
   if constexpr (CH > 0) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      const int c = lane + 64 * j;
+      const int c = lane + L * j;
       raw[j] = c < nch ? *(const i32x4 *)(xr + c * 8) : i32x4{0, 0, 0, 0};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -44,7 +52,7 @@ __global__ void __launch_bounds__(256) row_quant_kernel(int8_t *__restrict__ q, 
       }
     }
   } else {
-    for (int c = lane; c < nch; c += 64) {
+    for (int c = lane; c < nch; c += L) {
       const i32x4 r = *(const i32x4 *)(xr + c * 8);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -54,6 +62,13 @@ __global__ void __launch_bounds__(256) row_quant_kernel(int8_t *__restrict__ q, 
     }
   }
   amax = wave_max(amax);
+  if constexpr (WPR > 1) {
+    __shared__ float part[WPR];
+    if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = amax;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WPR; ++i) amax = fmaxf(amax, part[i]);
+  }
   float sc, inv;
   if constexpr (WEIGHT) {
     sc = fmaxf(__fdiv_rn(amax, 127.0f), 1e-12f);
@@ -87,11 +102,11 @@ __global__ void __launch_bounds__(256) row_quant_kernel(int8_t *__restrict__ q, 
   if constexpr (CH > 0) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      const int c = lane + 64 * j;
+      const int c = lane + L * j;
       if (c < nch) emit(c, raw[j]);
     }
   } else {
-    for (int c = lane; c < nch; c += 64) emit(c, *(const i32x4 *)(xr + c * 8));
+    for (int c = lane; c < nch; c += L) emit(c, *(const i32x4 *)(xr + c * 8));
   }
 }
 
@@ -103,24 +118,31 @@ int launch_row_quant(int8_t *q, float *scale, const void *x, int32_t rows, int32
   if (!q || !scale || !x || ((uintptr_t)x % 16) || ((uintptr_t)q % 8))
     return set_error(TMHD_ERR_INVALID, "%s: null or misaligned pointer", what);
   if (rows == 0) return TMHD_OK;
-  const int need = (cols / 8 + 63) / 64;
-  const dim3 grid((rows + 3) / 4), block(256);
   hipStream_t s = (hipStream_t)stream;
   const uint16_t *xp = (const uint16_t *)x;
-  if (need <= 1)
-    hipLaunchKernelGGL((row_quant_kernel<1, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
-  else if (need <= 2)
-    hipLaunchKernelGGL((row_quant_kernel<2, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
-  else if (need <= 4)
-    hipLaunchKernelGGL((row_quant_kernel<4, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
-  else if (need <= 8)
-    hipLaunchKernelGGL((row_quant_kernel<8, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
-  else if (need <= 10)
-    hipLaunchKernelGGL((row_quant_kernel<10, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
-  else if (need <= 16)
-    hipLaunchKernelGGL((row_quant_kernel<16, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
+  const int nch = cols / 8;
+  auto go = [&](auto wpr, auto ch) {
+    constexpr int WPR = decltype(wpr)::value, CH = decltype(ch)::value;
+    hipLaunchKernelGGL((row_quant_kernel<WPR, CH, WEIGHT>), dim3((rows + 4 / WPR - 1) / (4 / WPR)), dim3(256), 0, s, q,
+                       scale, xp, rows, cols, xs);
+  };
+  using std::integral_constant;
+  if (nch <= 64)
+    go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  else if (nch <= 2 * 64)
+    go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
+  else if (nch <= 4 * 64)
+    go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  else if (nch <= 2 * 256)
+    go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+  else if (nch <= 3 * 256)
+    go(integral_constant<int, 4>{}, integral_constant<int, 3>{});
+  else if (nch <= 4 * 256)
+    go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+  else if (nch <= 8 * 256)
+    go(integral_constant<int, 4>{}, integral_constant<int, 8>{});
   else
-    hipLaunchKernelGGL((row_quant_kernel<0, WEIGHT>), grid, block, 0, s, q, scale, xp, rows, cols, xs);
+    go(integral_constant<int, 4>{}, integral_constant<int, 0>{});
   return check_launch(what);
 }
 
