@@ -162,18 +162,22 @@ def _row_list(torch: Any, rows: Any, device: Any, limit: int, name: str, checked
     return rows.to(torch.int32).contiguous()
 
 
-def _key_sums(torch: Any, segments: Sequence[SlotView], stream: int, qq: Any, out: Any, base: int) -> None:
+def _key_sums(torch: Any, segments: Sequence[SlotView], stream: int, qq: Any, out: Any, base: int,
+              new: dict[tuple[KVSlot, tuple[int, int, int]], Any]) -> None:
     """Where the exact fixed-point key sums of each segment (the smooth-K mean's
     terms) are or go, memoised on its slot per (row0, tokens, stream): a cached
     block's keys are summed once, not on every call.  The slot drops the memo
-    whenever it is written."""
+    whenever it is written.  Sums that this batch takes go to ``new``: the
+    caller memoises them once their kernels are queued (a refused batch must
+    not leave unfilled ones behind)."""
     for j, view in enumerate(segments):
         slot = view.slot
         key = (int(view.row0), int(view.tokens), int(stream))
         hit = slot.key_sums.get(key)
         if hit is None:
-            hit = torch.empty((slot.heads, slot.head_dim), dtype=torch.int64, device=slot.device)
-            slot.key_sums[key] = hit
+            hit = new.get((slot, key))
+        if hit is None:
+            hit = new[slot, key] = torch.empty((slot.heads, slot.head_dim), dtype=torch.int64, device=slot.device)
             out[base + j] = _native.ptr(hit)  # summed by this batch
         else:
             qq.k_sum[j] = _native.ptr(hit)
@@ -364,10 +368,13 @@ def segment_attention_batch(
     )
     with maybe_region(timer, "qk_quant"):
         sums = (ctypes.c_void_p * (_native.MAX_SEGMENTS * len(calls)))()
+        new_sums: dict[tuple[KVSlot, tuple[int, int, int]], Any] = {}
         for i, segs in enumerate(segments):
-            _key_sums(torch, segs, stream, quants[i], sums, i * _native.MAX_SEGMENTS)
+            _key_sums(torch, segs, stream, quants[i], sums, i * _native.MAX_SEGMENTS, new_sums)
         status = lib.tmhd_qk_smooth_quant_batch(args, quants, sums, len(calls), stream)
     _native.check(status, "tmhd_qk_smooth_quant")
+    for (slot, key), value in new_sums.items():
+        slot.key_sums[key] = value
     with maybe_region(timer, "attention"):
         status = lib.tmhd_attn_fwd_i8qk_batch(args, quants, len(calls), stream)
     _native.check(status, "tmhd_attn_fwd_i8qk")
