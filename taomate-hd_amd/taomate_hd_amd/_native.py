@@ -272,11 +272,14 @@ def require_same_gpu(torch: Any, device: Any, **tensors: Any) -> None:
 
 
 def stream_ptr(torch: Any, device: Any) -> int:
-    """Handle of the current stream on ``device`` (read directly: a Stream object
+    """Handle of the current stream on ``device``, given as
+    ``torch.cuda.current_stream`` takes it (read directly: a Stream object
     costs 2 us, and a hook call asks several times)."""
-    index = getattr(device, "index", None)
-    if index is None:
-        index = torch.device(device).index
+    if not isinstance(device, torch.device):
+        device = torch.device("cuda" if device is None else device)
+    if device.type != "cuda":
+        raise ValueError(f"expected a GPU device, got {device}")
+    index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
