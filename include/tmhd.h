@@ -100,12 +100,14 @@ typedef struct tmhd_qk_quant {
   int64_t q_head_stride;        /* elements of q_i8 between heads */
   int32_t q_scale_head_stride;  /* elements of q_scale between heads */
   int32_t reserved0;
+  /* Each segment's own k_i8 and k_scale, each call's own q_i8, q_scale and k_mean: written
+   * by tmhd_qk_smooth_quant, which also keeps partial key sums in k_i8 until the keys go there. */
   int8_t *k_i8[TMHD_MAX_SEGMENTS];      /* [H][cap][D] per segment */
   float *k_scale[TMHD_MAX_SEGMENTS];    /* [H][cap / 128] per segment */
   int64_t k_head_stride[TMHD_MAX_SEGMENTS];       /* elements */
   int32_t k_scale_head_stride[TMHD_MAX_SEGMENTS]; /* elements */
   uint16_t *k_mean;             /* bf16 [H][D] written by tmhd_qk_smooth_quant (16-byte aligned) */
-  int64_t *mean_workspace;      /* int64 [H][D] scratch (8-byte aligned) */
+  int64_t *mean_workspace;      /* not used (may be NULL); kept for the struct's layout */
   /* Optional, per segment: the exact fixed-point key sums of segment i from
    * tmhd_k_fixed_sum (int64 [H][D], 8-byte aligned), used in place of summing
    * its keys again; NULL: summed here.  The mean is the same bits either way. */

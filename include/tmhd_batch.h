@@ -29,7 +29,10 @@ int tmhd_attn_fwd_i8qk_batch(const tmhd_attn_args *args, const tmhd_qk_quant *qu
 
 /*
  * tmhd_qk_smooth_quant of n calls that share heads and head_dim, in three
- * launches (per 16 calls and 24 segments).  k_sum_out (NULL: none) holds n *
+ * launches (per 16 calls and 24 segments).  The q_i8, q_scale, k_mean, k_i8 and
+ * k_scale of one call must not overlap those of another, also where two calls
+ * name the same keys: k_i8 holds partial sums on the way, and each call has its
+ * own mean.  k_sum_out (NULL: none) holds n *
  * TMHD_MAX_SEGMENTS pointers: entry [i * TMHD_MAX_SEGMENTS + j], where set and
  * where call i's k_sum[j] is NULL, receives segment j's exact key sums
  * (tmhd_k_fixed_sum's, 8-byte aligned); a later call of the batch may name the

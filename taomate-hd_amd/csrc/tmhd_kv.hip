@@ -454,10 +454,9 @@ int check_smooth_quant(const tmhd_attn_args *args, const tmhd_qk_quant *quant) {
   if (D != 64 && D != 128) return set_error(TMHD_ERR_UNSUPPORTED, "smooth_quant: head_dim %d", D);
   if (args->n_segments < 1 || args->n_segments > kMaxSeg || args->heads <= 0 || args->lq < 0)
     return set_error(TMHD_ERR_INVALID, "smooth_quant: bad segment count / heads / lq");
-  if (!quant->k_mean || !quant->mean_workspace || !quant->q_i8 || !quant->q_scale)
+  if (!quant->k_mean || !quant->q_i8 || !quant->q_scale)
     return set_error(TMHD_ERR_INVALID, "smooth_quant: null output buffers");
-  if (!aligned(quant->k_mean, 16) || !aligned(quant->mean_workspace, 8))
-    return set_error(TMHD_ERR_INVALID, "smooth_quant: k_mean must be 16-byte and mean_workspace 8-byte aligned");
+  if (!aligned(quant->k_mean, 16)) return set_error(TMHD_ERR_INVALID, "smooth_quant: k_mean must be 16-byte aligned");
   const int qcap = (args->lq + 255) / 256 * 256;
   if (quant->q_head_stride < (int64_t)qcap * D || quant->q_scale_head_stride < qcap / TMHD_QUANT_BLOCK ||
       !aligned(quant->q_i8, 16) || quant->q_head_stride % 16)

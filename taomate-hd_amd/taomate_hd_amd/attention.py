@@ -82,9 +82,7 @@ class QKQuantWorkspace:
         k_i8 = self._grow(store, "k_i8", k_total, torch.int8, device)
         k_scale = self._grow(store, "k_scale", ks_total, torch.float32, device)
         k_mean = self._grow(store, "k_mean", n * width, torch.bfloat16, device)
-        ws = self._grow(store, "mean_ws", width, torch.int64, device)
         q_at, qs_at, k_at, ks_at, mean_at = (_native.ptr(t) for t in (q_i8, q_scale, k_i8, k_scale, k_mean))
-        ws_at = _native.ptr(ws)
         structs = (_native.QKQuant * n)()
         views = []
         for i, (qcap, q_off, qs_off, segs) in enumerate(plan):
@@ -99,7 +97,6 @@ class QKQuantWorkspace:
                 qq.k_head_stride[j] = cap * head_dim
                 qq.k_scale_head_stride[j] = nblk
             qq.k_mean = mean_at + 2 * i * width
-            qq.mean_workspace = ws_at
             if with_views:
                 views.append({
                     "q_i8": q_i8[q_off : q_off + heads * qcap * head_dim].view(heads, qcap, head_dim),
