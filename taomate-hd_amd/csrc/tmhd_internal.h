@@ -6,6 +6,7 @@
 
 #include "tmhd.h"
 #include "tmhd_batch.h"
+#include "tmhd_forms.h"
 
 namespace tmhd {
 

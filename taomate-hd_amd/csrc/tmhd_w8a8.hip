@@ -1060,9 +1060,8 @@ __global__ void __launch_bounds__(256) gemm_split_merge_kernel(const GArgs ga) {
 // fill less than half the CUs) may take: its tiles' 128-byte k blocks are dealt
 // to S parts, S up to CUs / tiles and at least 2 blocks per part, so that the
 // round fills the CUs; the partials are merged by gemm_split_merge_kernel.
-void gemm_split_plan(int32_t m, int32_t n, int32_t k, int &tail, int &parts) {
+void gemm_split_plan(int32_t m, int32_t n, int32_t k, int cus, int &tail, int &parts) {
   tail = 0, parts = 1;
-  const int cus = device_cus();
   if (cus <= 0 || m <= 0 || n <= 0 || k <= 0 || k % HKD) return;
   const int64_t tiles = (int64_t)((m + HBM_ - 1) / HBM_) * ((n + HBN - 1) / HBN);
   const int64_t t = tiles % cus;
@@ -1076,7 +1075,15 @@ int64_t gemm_split_bytes(int tail, int parts) { return (int64_t)tail * parts * H
 
 // How the last, partial round of 256 x 256 tiles runs (all tiles, when they do
 // not fill a round).
-enum Tail { kTailWhole, kTailSplit, kTail64x64, kTail64x128, kTail128, kTail192x128, kTail256x128 };
+enum Tail {
+  kTailWhole = TMHD_GEMM_WHOLE,
+  kTailSplit = TMHD_GEMM_SPLIT_K,
+  kTail64x64 = TMHD_GEMM_64X64,
+  kTail64x128 = TMHD_GEMM_64X128,
+  kTail128 = TMHD_GEMM_128X128,
+  kTail192x128 = TMHD_GEMM_192X128,
+  kTail256x128 = TMHD_GEMM_256X128,
+};
 
 // The tiles of gemm_i8_tile_kernel and, per 128-byte block of k, the
 // microseconds of a round of them: `one` + `fill` * (share of the CUs in use),
@@ -1126,6 +1133,25 @@ Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cu
   return best;
 }
 
+// The last, partial round of an m x n x k product whose rounds the whole-tile
+// kernel runs: its 256 x 256 tiles (0: none, every round is whole), its form
+// with a workspace of ws_bytes, and for the k split the parts.
+struct LastRound {
+  int64_t tiles;
+  Tail form;
+  int parts;
+};
+LastRound last_round(int32_t m, int32_t n, int32_t k, int64_t ws_bytes, int cus) {
+  const int64_t tiles = (int64_t)((m + HBM_ - 1) / HBM_) * ((n + HBN - 1) / HBN);
+  LastRound r{cus > 0 ? tiles % cus : 0, kTailWhole, 1};
+  if (r.tiles == 0) return r;
+  int split_tiles = 0;
+  gemm_split_plan(m, n, k, cus, split_tiles, r.parts);
+  const bool can_split = r.parts > 1 && ws_bytes >= gemm_split_bytes(split_tiles, r.parts);
+  r.form = pick_tail(r.tiles, r.tiles < tiles, m, n, k, cus, can_split ? r.parts : 1);
+  return r;
+}
+
 template <int MH, int NH, int RING, int WPE, bool RAW, bool GLU>
 void launch_tiles(GArgs ga, int64_t tiles, bool part, hipStream_t s) {
   const int64_t wgs = part ? tiles * (HBM_ / (2 * MH)) * (HBN / (2 * NH))
@@ -1138,27 +1164,20 @@ void launch_tiles(GArgs ga, int64_t tiles, bool part, hipStream_t s) {
 // rounds of whole tiles and a last round as pick_tail says.  ga.full: all tiles.
 template <bool RAW, bool GLU>
 void launch_rounds(GArgs ga, void *ws, int64_t ws_bytes, hipStream_t s) {
-  const int64_t tiles = ga.full;
-  const int cus = device_cus();
-  const int64_t last = cus > 0 ? tiles % cus : 0;
-  Tail tail = kTailWhole;
-  int split_tiles = 0, parts = 1;
-  if (last > 0) {
-    gemm_split_plan(ga.m, ga.n, ga.k, split_tiles, parts);
-    const bool can_split = parts > 1 && ws && ((uintptr_t)ws % 16) == 0 && ws_bytes >= gemm_split_bytes(split_tiles, parts);
-    tail = pick_tail(last, last < tiles, ga.m, ga.n, ga.k, cus, can_split ? parts : 1);
-  }
-  if (tail != kTailWhole) ga.full = (int32_t)(tiles - last);
+  const bool ws_ok = ws && ((uintptr_t)ws % 16) == 0;
+  const LastRound r = last_round(ga.m, ga.n, ga.k, ws_ok ? ws_bytes : 0, device_cus());
+  const int64_t last = r.tiles;
+  if (r.form != kTailWhole) ga.full -= (int32_t)last;
   const bool part = ga.full > 0;
   if (part)
     hipLaunchKernelGGL((gemm_i8_wave128_kernel<RAW, false, GLU>), dim3((unsigned)ga.full), dim3(HWAVES * 64), 0, s, ga);
-  switch (tail) {
+  switch (r.form) {
     case kTailWhole:
       break;
     case kTailSplit:
-      ga.nsplit = parts;
+      ga.nsplit = r.parts;
       ga.ws = (int32_t *)ws;
-      hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, true>), dim3((unsigned)(last * parts)), dim3(HWAVES * 64), 0, s, ga);
+      hipLaunchKernelGGL((gemm_i8_wave128_kernel<false, true>), dim3((unsigned)(last * r.parts)), dim3(HWAVES * 64), 0, s, ga);
       if constexpr (GLU)
         hipLaunchKernelGGL(gemm_split_merge_glu_kernel, dim3((unsigned)(last * (HBM_ / 8))), dim3(256), 0, s, ga);
       else
@@ -1254,9 +1273,15 @@ extern "C" int tmhd_gemm_i8_i32(int32_t *out, const int8_t *a, const int8_t *b, 
   return tmhd::launch_gemm<true>(out, a, b, nullptr, nullptr, nullptr, m, n, k, lda, ldb, ldo, nullptr, 0, stream);
 }
 
+extern "C" int tmhd_gemm_last_round_form(int32_t m, int32_t n, int32_t k, int64_t workspace_bytes, int32_t cus) {
+  using namespace tmhd;
+  if (m <= 0 || n <= 0 || k <= 0 || k % HKD) return -1;
+  return last_round(m, n, k, workspace_bytes, cus > 0 ? cus : device_cus()).form;
+}
+
 extern "C" int64_t tmhd_gemm_split_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   int tail = 0, parts = 1;
-  tmhd::gemm_split_plan(m, n, k, tail, parts);
+  tmhd::gemm_split_plan(m, n, k, tmhd::device_cus(), tail, parts);
   return parts > 1 ? tmhd::gemm_split_bytes(tail, parts) : 0;
 }
 

@@ -1,4 +1,5 @@
-"""ctypes binding of libtmhd.so (the C ABI declared in include/tmhd.h and tmhd_batch.h).
+"""ctypes binding of libtmhd.so (the C ABI declared in include/tmhd.h, tmhd_batch.h
+and tmhd_forms.h).
 
 The library is the only compute path of this package: every operator raises
 if it is not built or no GPU is present.  There is no CPU fallback.
@@ -22,6 +23,9 @@ TMHD_OK = 0
 TMHD_ERR_INVALID = 1
 TMHD_ERR_UNSUPPORTED = 2
 TMHD_ERR_HIP = 3
+
+# tmhd_gemm_last_round_form
+GEMM_WHOLE, GEMM_SPLIT_K, GEMM_64X64, GEMM_64X128, GEMM_128X128, GEMM_192X128, GEMM_256X128 = range(7)
 
 
 class KVSegment(ctypes.Structure):
@@ -199,8 +203,9 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     ),
 }
 
-# include/tmhd_batch.h
-_BATCH_SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
+# include/tmhd_batch.h and include/tmhd_forms.h
+_MORE_SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
+    "tmhd_gemm_last_round_form": (c_int, [c_int32, c_int32, c_int32, c_int64, c_int32]),
     "tmhd_attn_fwd_bf16_batch": (c_int, [POINTER(AttnArgs), c_int32, c_void_p]),
     "tmhd_attn_fwd_i8qk_batch": (c_int, [POINTER(AttnArgs), POINTER(QKQuant), c_int32, c_void_p]),
     "tmhd_qk_smooth_quant_batch": (
@@ -234,7 +239,7 @@ def load() -> ctypes.CDLL:
                     "(hipcc --offload-arch=gfx950) before using the HIP operators"
                 )
             lib = ctypes.CDLL(str(LIB_PATH))
-            for name, (restype, argtypes) in (*_SIGNATURES.items(), *_BATCH_SIGNATURES.items()):
+            for name, (restype, argtypes) in (*_SIGNATURES.items(), *_MORE_SIGNATURES.items()):
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes

@@ -1,8 +1,7 @@
 """Seeded random sweep of the scaled INT8 GEMM against the oracle, bit for bit:
 random m, n (odd widths take the scalar scale / bias loads and the per-element
 tail stores), k (odd multiples of 64 run the 8-wave kernel, multiples of 128
-the one-wave-per-SIMD kernel, split along k when its tiles leave the CUs
-idle), padded row strides of both operands and of the output (a row stride
+the one-wave-per-SIMD kernels, here in small tiles), padded row strides of both operands and of the output (a row stride
 that is not a multiple of 8 takes the epilogue without LDS staging), with and
 without bias.
 """

@@ -399,22 +399,22 @@ def test_gemm_accumulators_and_epilogue_bit_exact(torch_mod, dev, m, n, k):
 
 
 def test_gemm_split_round_equals_unsplit(torch_mod, dev):
-    # 8 x 37 = 296 tiles: on 256 CUs one whole round plus a 40-tile round (more
-    # than an eighth of the CUs, at most half) that is split along k; the
-    # split + merge must equal the unsplit GEMM bit for bit
+    # 5 x 58 = 290 tiles: on 256 CUs one whole round plus a 34-tile round that is
+    # split along k where there is a workspace; the split + merge must equal the
+    # GEMM without one (which takes another form) bit for bit
     torch = torch_mod
     from taomate_hd_amd import _native, quant
 
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    m, n, k = 8 * 256 - 100, 37 * 256 - 30, 1024
-    last = (8 * 37) % cus
-    if not (cus < 8 * last and 2 * last <= cus):
-        pytest.skip(f"296 tiles leave a last round of {last} on {cus} CUs: not the k-split case")
+    m, n, k = 5 * 256 - 249, 58 * 256 - 30, 5376
+    lib = _native.load()
+    need = lib.tmhd_gemm_split_workspace_bytes(m, n, k)
+    forms = [lib.tmhd_gemm_last_round_form(m, n, k, ws, 0) for ws in (need, 0)]
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the shape is split along k on 256 CUs")
+    assert need > 0 and forms[0] == _native.GEMM_SPLIT_K and forms[1] != _native.GEMM_SPLIT_K
     rng = np.random.default_rng(5)
     ad = torch.from_numpy(rng.integers(-128, 128, size=(m, k), dtype=np.int8)).to(dev)
     wd = torch.from_numpy(rng.integers(-127, 128, size=(n, k), dtype=np.int8)).to(dev)
-    lib = _native.load()
-    assert lib.tmhd_gemm_split_workspace_bytes(m, n, k) > 0
     stream = _native.stream_ptr(torch, dev)
     plain = torch.empty((m, n), dtype=torch.int32, device=dev)
     _native.check(lib.tmhd_gemm_i8_i32(_native.ptr(plain), _native.ptr(ad), _native.ptr(wd), m, n, k, k, k, n, stream),
@@ -434,18 +434,17 @@ def test_gemm_split_round_equals_unsplit(torch_mod, dev):
 
 
 def test_gemm_sub_tile_last_round(torch_mod, dev):
-    # 15 x 18 = 270 tiles: on 256 CUs one whole round plus a 14-tile round (at
-    # most an eighth of the CUs), which runs as 64 x 128 sub-tiles over the
-    # whole of k; int32 accumulators against an exact float64 product, and the
-    # bf16 epilogue against the oracle, bit for bit (k = 384: a 3-block ring)
+    # 15 x 18 = 270 tiles: on 256 CUs one whole round plus a 14-tile round, which
+    # runs as 64 x 64 tiles over the whole of k; int32 accumulators against an
+    # exact float64 product, and the bf16 epilogue against the oracle, bit for
+    # bit (k = 384: 3 blocks, fewer than the ring holds)
     torch = torch_mod
-    from taomate_hd_amd import quant
+    from taomate_hd_amd import _native, quant
 
-    cus = torch.cuda.get_device_properties(dev).multi_processor_count
     m, n, k = 15 * 256 - 100, 18 * 256 - 30, 384
-    last = (15 * 18) % cus
-    if not (0 < 8 * last <= cus):
-        pytest.skip(f"270 tiles leave a last round of {last} on {cus} CUs: not the sub-tile case")
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the shape leaves 14 tiles on 256 CUs")
+    assert _native.load().tmhd_gemm_last_round_form(m, n, k, 0, 0) == _native.GEMM_64X64
     rng = np.random.default_rng(9)
     a = rng.integers(-128, 128, size=(m, k), dtype=np.int8)
     w = rng.integers(-127, 128, size=(n, k), dtype=np.int8)

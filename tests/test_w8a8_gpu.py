@@ -105,10 +105,11 @@ def test_w8a8_projection_full_size_sampled_rows(torch_mod, dev):
                                              (200, 576, 256, True), (70, 320, 128, False)])
 def test_fused_fc1_swiglu_equals_two_step(torch_mod, dev, m, k, f, with_bias):
     """FC1 with the SwiGLU epilogue (interleaved gate / up rows) against the
-    two-step path (the W8A8 projection, then fused_swiglu), bit for bit; the
-    first and last shapes of the first five run the k-split merge, the middle
-    one does not; the last two have k an odd multiple of 64, which the fused
-    kernel does not take (its projection runs on the 64-byte-block GEMM)."""
+    two-step path (the W8A8 projection, then fused_swiglu), bit for bit, with and
+    without bias: the first five run as 64 x 64 tiles, the middle one of them as
+    64 x 128 (every form is compared in test_gemm_forms.py); the last two have k
+    an odd multiple of 64, which the fused kernel does not take (its projection
+    runs on the 64-byte-block GEMM)."""
     torch = torch_mod
     from taomate_hd_amd import (W8A8Workspace, cutlass_w8a8_linear, cutlass_w8a8_linear_swiglu, fused_swiglu,
                                 interleave_swiglu_rows, quantize_cutlass_w8a8_swiglu_weight,
