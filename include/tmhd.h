@@ -464,9 +464,9 @@ int tmhd_gemm_i8_i32(int32_t *out, const int8_t *a, const int8_t *b, int32_t m,
  * at least 256 bytes of k; the parts' int32 partial tiles go to `workspace`
  * and a second pass adds them (exactly) and applies the same epilogue.
  * Results are bit-identical in every form.  tmhd_gemm_split_workspace_bytes
- * gives the bytes that the k split would need on the current device for the
- * shape (0: none); with a smaller or null workspace the _ws calls do not use
- * that form.  Partial tiles of calls that overlap on one workspace race.  The
+ * gives the bytes that the k split needs on the current device where the shape
+ * takes that form (0: it does not); with a smaller or null workspace the _ws
+ * calls do not use it.  Partial tiles of calls that overlap on one workspace race.  The
  * SwiGLU GEMM below has the same forms.
  */
 int64_t tmhd_gemm_split_workspace_bytes(int32_t m, int32_t n, int32_t k);

@@ -1059,19 +1059,13 @@ __global__ void __launch_bounds__(256) gemm_split_merge_kernel(const GArgs ga) {
 // The k split that a last, partial round of 256 x 256 tiles (all tiles when they
 // fill less than half the CUs) may take: its tiles' 128-byte k blocks are dealt
 // to S parts, S up to CUs / tiles and at least 2 blocks per part, so that the
-// round fills the CUs; the partials are merged by gemm_split_merge_kernel.
-void gemm_split_plan(int32_t m, int32_t n, int32_t k, int cus, int &tail, int &parts) {
-  tail = 0, parts = 1;
-  if (cus <= 0 || m <= 0 || n <= 0 || k <= 0 || k % HKD) return;
-  const int64_t tiles = (int64_t)((m + HBM_ - 1) / HBM_) * ((n + HBN - 1) / HBN);
-  const int64_t t = tiles % cus;
-  if (t == 0 || 2 * t > cus) return;
-  const int64_t s = std::min<int64_t>(cus / t, (k / HKD) / 2);
-  if (s < 2) return;
-  tail = (int)t, parts = (int)s;
+// round fills the CUs (1: no split); the partials are merged by
+// gemm_split_merge_kernel.
+int split_parts(int64_t tail, int32_t k, int cus) {
+  return 2 * tail > cus ? 1 : std::max(1, (int)std::min<int64_t>(cus / tail, (k / HKD) / 2));
 }
 
-int64_t gemm_split_bytes(int tail, int parts) { return (int64_t)tail * parts * HBM_ * HBN * 4; }
+int64_t gemm_split_bytes(int64_t tail, int parts) { return tail * parts * HBM_ * HBN * 4; }
 
 // How the last, partial round of 256 x 256 tiles runs (all tiles, when they do
 // not fill a round).
@@ -1111,13 +1105,13 @@ constexpr double kTileFixedUs = 5.0;  // a launch of them: first loads, epilogue
 //   512 x 5,376 x 5,376: 128 x 128 24, 64 x 64 27, k split 38
 //   1,024 x 5,376 x 10,752 (168 tiles): whole 57, 192 x 128 74, 256 x 128 89
 // The k split remains for long k (8 tiles of 32,768: 24 against 72 us estimated).
-Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cus, int split_parts) {
+Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cus, int parts) {
   const double nd = (double)(k / HKD);
   Tail best = kTailWhole;
   double us = nd * (0.95 + 0.45 * (double)tiles / cus) + 8.0;
-  if (split_parts > 1) {
+  if (parts > 1) {
     // 12 us of launches and merge, and per tile the write and read of its partials
-    const double t = nd / split_parts * 1.35 + 12.0 + 0.165 * (double)tiles;
+    const double t = nd / parts * 1.35 + 12.0 + 0.165 * (double)tiles;
     if (t < us) us = t, best = kTailSplit;
   }
   for (const TileCost &c : kTiles) {
@@ -1145,10 +1139,9 @@ LastRound last_round(int32_t m, int32_t n, int32_t k, int64_t ws_bytes, int cus)
   const int64_t tiles = (int64_t)((m + HBM_ - 1) / HBM_) * ((n + HBN - 1) / HBN);
   LastRound r{cus > 0 ? tiles % cus : 0, kTailWhole, 1};
   if (r.tiles == 0) return r;
-  int split_tiles = 0;
-  gemm_split_plan(m, n, k, cus, split_tiles, r.parts);
-  const bool can_split = r.parts > 1 && ws_bytes >= gemm_split_bytes(split_tiles, r.parts);
-  r.form = pick_tail(r.tiles, r.tiles < tiles, m, n, k, cus, can_split ? r.parts : 1);
+  r.parts = split_parts(r.tiles, k, cus);
+  if (ws_bytes < gemm_split_bytes(r.tiles, r.parts)) r.parts = 1;
+  r.form = pick_tail(r.tiles, r.tiles < tiles, m, n, k, cus, r.parts);
   return r;
 }
 
@@ -1280,9 +1273,10 @@ extern "C" int tmhd_gemm_last_round_form(int32_t m, int32_t n, int32_t k, int64_
 }
 
 extern "C" int64_t tmhd_gemm_split_workspace_bytes(int32_t m, int32_t n, int32_t k) {
-  int tail = 0, parts = 1;
-  tmhd::gemm_split_plan(m, n, k, tmhd::device_cus(), tail, parts);
-  return parts > 1 ? tmhd::gemm_split_bytes(tail, parts) : 0;
+  using namespace tmhd;
+  if (m <= 0 || n <= 0 || k <= 0 || k % HKD) return 0;
+  const LastRound r = last_round(m, n, k, INT64_MAX, device_cus());
+  return r.form == kTailSplit ? gemm_split_bytes(r.tiles, r.parts) : 0;
 }
 
 extern "C" int tmhd_gemm_w8a8_ws(void *out, const int8_t *a, const int8_t *b, const float *a_scale,

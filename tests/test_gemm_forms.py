@@ -76,6 +76,17 @@ def _here(dev, form, m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", [s[1:] for s in SHAPES] + [(12252, 13824, 5120), (331, 13824, 5120), (16, 256, 192)])
+def test_workspace_is_asked_for_only_where_the_split_runs(dev, m, n, k):
+    lib = _native.load()
+    need = lib.tmhd_gemm_split_workspace_bytes(m, n, k)
+    assert (need > 0) == (lib.tmhd_gemm_last_round_form(m, n, k, WS, 0) == S)
+    if need:
+        assert lib.tmhd_gemm_last_round_form(m, n, k, need, 0) == S
+        assert lib.tmhd_gemm_last_round_form(m, n, k, need - 1, 0) != S
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("form,m,n,k", SHAPES, ids=IDS)
 def test_plain(dev, form, m, n, k):
     from taomate_hd_amd import quant
