@@ -1081,9 +1081,7 @@ enum Tail {
 
 // The tiles of gemm_i8_tile_kernel and, per 128-byte block of k, the
 // microseconds of a round of them: `one` + `fill` * (share of the CUs in use),
-// or `two` with a second workgroup on each CU.  From k = 5,120 and 5,376 at 16
-// to 2,048 rows and 5,376 to 13,824 columns; with them the choice among the
-// forms below is within 10% of the best one measured there.
+// or `two` with a second workgroup on each CU.
 struct TileCost {
   Tail tail;
   int bm, bn, per_cu;
@@ -1094,24 +1092,30 @@ constexpr TileCost kTiles[] = {
     {kTail128, 128, 128, 1, 0.42, 0.14, 0.0},      {kTail192x128, 192, 128, 1, 0.58, 0.22, 0.0},
     {kTail256x128, 256, 128, 1, 0.78, 0.26, 0.0},
 };
-constexpr double kTileFixedUs = 5.0;  // a launch of them: first loads, epilogue
+constexpr double kTileRoundUs = 5.0;  // a round of them besides its k blocks: first loads, epilogue
 
 // Cheapest form for `tiles` 256 x 256 tiles (fewer than cus) of an m x n x k
-// product; `part`: they are the last round of more.  Measured, us (before:
-// whole tiles, the k split, and 64 x 128 tiles for a small last round):
-//   16 x 5,120 x 13,824: 64 x 64 tiles 14, 64 x 128 22, k split 34
-//   331 x 5,120 x 13,824: 192 x 128 tiles 40, k split 50, 64 x 128 55, 64 x 64 55
-//   331 x 5,376 x 10,752: 128 x 128 27, 64 x 128 31, 192 x 128 32, k split 48
-//   512 x 5,376 x 5,376: 128 x 128 24, 64 x 64 27, k split 38
-//   1,024 x 5,376 x 10,752 (168 tiles): whole 57, 192 x 128 74, 256 x 128 89
-// The k split remains for long k (8 tiles of 32,768: 24 against 72 us estimated).
+// product; `part`: they are the last round of more.  Fitted to k = 5,120 and
+// 5,376, and checked with every form forced, on weights not read shortly
+// before, over 768 products of 1 to 5,000 rows, 16 to 28,672 columns and k of
+// 128 to 13,824 (profiles/gemm_form_sweep.txt): within 10% of the best form in
+// all but one of 658 with k up to 7,168 (that one 15%); with longer k the split
+// is taken for few tiles where 64 x 64 tiles would be up to 1.6 times as fast.
+// us, m x n x k:
+//   16 x 13,824 x 5,120: 64 x 64 tiles 17, 64 x 128 25, k split 34, whole 51
+//   331 x 13,824 x 5,120: 192 x 128 tiles 39, k split 49, whole 55, 64 x 64 58
+//   331 x 10,752 x 5,376: 128 x 128 30, 192 x 128 36, 64 x 128 38, k split 45
+//   512 x 5,376 x 5,376: 128 x 128 31, 64 x 64 38, k split 40, whole 59
+//   1,024 x 10,752 x 5,376 (168 tiles): whole 60, 192 x 128 68, 256 x 128 84
+//   1,024 x 28,672 x 640: whole 37, 64 x 128 to 256 x 128 48 (two rounds or more)
+// The k split remains for long k (8 tiles of 32,768: 26 against 56 us estimated).
 Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cus, int parts) {
   const double nd = (double)(k / HKD);
   Tail best = kTailWhole;
   double us = nd * (0.95 + 0.45 * (double)tiles / cus) + 8.0;
   if (parts > 1) {
-    // 12 us of launches and merge, and per tile the write and read of its partials
-    const double t = nd / parts * 1.35 + 12.0 + 0.165 * (double)tiles;
+    // 14 us of launches and merge, and per tile the write and read of its partials
+    const double t = nd / parts * 1.35 + 14.0 + 0.165 * (double)tiles;
     if (t < us) us = t, best = kTailSplit;
   }
   for (const TileCost &c : kTiles) {
@@ -1121,7 +1125,7 @@ Tail pick_tail(int64_t tiles, bool part, int32_t m, int32_t n, int32_t k, int cu
     const int64_t slots = (int64_t)cus * c.per_cu, rest = wgs % slots;
     const double full = c.per_cu == 2 ? c.two : c.one + c.fill;
     const double last = rest == 0 ? 0.0 : rest <= cus ? c.one + c.fill * (double)rest / cus : c.two;
-    const double t = kTileFixedUs + nd * ((double)(wgs / slots) * full + last);
+    const double t = kTileRoundUs * (double)((wgs + slots - 1) / slots) + nd * ((double)(wgs / slots) * full + last);
     if (t < us) us = t, best = c.tail;
   }
   return best;
