@@ -489,8 +489,12 @@ __device__ __forceinline__ void write_rows(const char *stage, const KArgs &a, co
 // its own rows) and out as whole rows: a round of items of one key tile takes
 // 13.0 us (BF16, head_dim 128; INT8-QK 16.3), against 14.5 (18.7) with the rows
 // stored straight from the registers, 16 bytes of 32 rows at a time; the output
-// alone is 3.3 us of memory time.  Parts go to their slot in register order, 1
-// KiB per store, which the merge reads back.
+// alone is 3.3 us of memory time.  Items of so few rows that a wave has none
+// store straight from the registers: their stores do not bound them, and the
+// staging costs about 2 us then (40 items of 77 rows and two key tiles 12.7 us
+// staged, 10.6 straight; of 128 rows 12.9 and 11.6, of 190 13.2 and 12.8; INT8-QK
+// the same).  Parts go to their slot in register order, 1 KiB per store, which
+// the merge reads back.
 template <int D>
 __device__ __forceinline__ void write_item(f32x16 (&o)[2][D / 32], const float (&lsum)[2], const float (&mref)[2],
                                            const KArgs &a, const Prob &P, const Frag &fr, int w, int lane, char *smem) {
@@ -511,6 +515,26 @@ __device__ __forceinline__ void write_item(f32x16 (&o)[2][D / 32], const float (
             *(f32x4 *)(op + (db * 4 + u) * 256) = f32x4{o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv,
                                                         o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv};
         if (g == 0) wo[kBM * D + w * kQW + hf * 32 + lr] = mref[hf] + __log2f(lt);
+      }
+    }
+    return;
+  }
+  if (P.lq - fr.qt * kBM <= kBM - kQW) {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const float lt = lsum[hf] + __shfl_xor(lsum[hf], 32);
+      const float inv = 1.0f / lt;
+      const int ql = q0 + hf * 32 + lr;
+      if (ql < P.lq) {
+        const int row = P.o_rows ? P.o_rows[ql] : P.o_row0 + ql;
+        uint16_t *op = P.o + (int64_t)row * a.ots + (int64_t)fr.h * a.ohs + 4 * g;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            *(i32x2 *)(op + db * 32 + 8 * u) =
+                i32x2{(int)pack_bf16x2(o[hf][db][4 * u] * inv, o[hf][db][4 * u + 1] * inv),
+                      (int)pack_bf16x2(o[hf][db][4 * u + 2] * inv, o[hf][db][4 * u + 3] * inv)};
       }
     }
     return;
