@@ -30,6 +30,17 @@ enum {
 };
 int tmhd_gemm_last_round_form(int32_t m, int32_t n, int32_t k, int64_t workspace_bytes, int32_t cus);
 
+/*
+ * Into how many key ranges an attention call of `items` 256-row query tiles
+ * (over all heads) and `key_tiles` 64-key tiles cuts the items of its last,
+ * partial round, on either backend (i8qk != 0: INT8-QK), with workspace_bytes
+ * of split workspace on a device of `cus` CUs (0: the current one); 1: it runs
+ * them whole.  -1 for sizes or a head_dim that no call has.  Launches nothing,
+ * and needs no GPU if cus > 0.  No counterpart in the reference.
+ */
+int tmhd_attn_last_round_ranges(int32_t items, int32_t key_tiles, int32_t head_dim, int32_t i8qk,
+                                int64_t workspace_bytes, int32_t cus);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1613,9 +1613,10 @@ bool aligned(const void *p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
 int64_t split_slot_bytes(int D) { return (int64_t)kBM * (D + 1) * 4; }
 
-// Times behind the split rule, in microseconds, fitted to calls of 8 to 280
-// items (6 to 252 key tiles, both head dims and backends) timed at 1 to 15
-// ranges per item: the rule's choice is within 8% of the best of them.
+// Times behind the split rule, in microseconds.  Checked with every number of
+// ranges forced over 700 drawn calls of 1 to 900 items, 1 to 252 key tiles,
+// both head dims and backends (profiles/attn_split_sweep.txt): the choice is
+// within 8% of the best number of ranges in all but four of them, at worst 10%.
 // A key tile of a workgroup, by how many run: more of them run at a lower
 // clock (the card's power limit), and two INT8-QK workgroups share a CU.
 double tile_us(bool i8, int D, int workgroups, int cus) {
@@ -1624,23 +1625,24 @@ double tile_us(bool i8, int D, int workgroups, int cus) {
   return one * (1.0 + 0.2 * workgroups / cus);
 }
 // What an item costs besides its tiles (5 rounds of 256 items of 1 to 64 key
-// tiles, extrapolated to none), and the merge: its launch, and a
-// partial slot's write and read (at head_dim 128).
-constexpr double kItemUs = 10.0, kItemUs64 = 6.0, kMergeUs = 8.0, kMergeUsPerSlot = 0.02;
+// tiles, extrapolated to none), and the merge: its launch (4 to 5 us in the
+// trace), a partial slot's write and read (at head_dim 128), and the parts of
+// an item, which are read four at a time.
+constexpr double kItemUs = 10.0, kItemUs64 = 6.0, kMergeUs = 4.0, kMergeUsPerSlot = 0.04, kMergeUsPerPart = 0.1;
 constexpr int kMaxParts = 16, kItemTiles = 8;  // kItemTiles: kItemUs in tiles
 
 // Decides how the last, partial round of items runs: whole, or as key ranges
 // dealt evenly to workgroups (see KArgs).  `slots` workgroups are resident at
 // once.  n ranges per item of the longest problem (fewer of the others, of
 // about the same length) are shared out `share` to a workgroup; the n whose
-// estimated time is least, if it beats whole items.
-void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
-  const int cus = device_cus(), slots = (i8 ? 2 : 1) * cus;
+// estimated time is least, if it beats whole items.  Returns it (1: whole).
+int plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes, int cus) {
+  const int slots = (i8 ? 2 : 1) * cus;
   const Prob &last = k.pr[k.nprob - 1];
   const int items = last.item0 + last.nqt * k.heads;
   k.full = items;
   for (int p = 0; p < k.nprob; ++p) k.pr[p].nwhole = k.pr[p].nqt * k.heads;
-  if (cus <= 0 || !k.ws || items % slots == 0) return;
+  if (cus <= 0 || !k.ws || items % slots == 0) return 1;
   const int full = items - items % slots;
   int nwhole[kMaxProb], rest[kMaxProb], longest = 0;  // longest: key tiles of the round's longest item
   for (int p = 0; p < k.nprob; ++p) {
@@ -1658,7 +1660,7 @@ void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
     return q < 1 ? 1 : q;
   };
   const double item = D == 128 ? kItemUs : kItemUs64;
-  double best = 0.93 * (longest * tile_us(i8, D, items - full, cus) + item);
+  double best = longest * tile_us(i8, D, items - full, cus) + item;
   int best_n = 0;
   for (int n = 2; n <= kMaxParts && 2 * n <= longest; ++n) {
     int64_t line = 0;
@@ -1669,10 +1671,11 @@ void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
     const int64_t begun = n % share == 0 ? 1 : share / n + 2;  // long items a share touches
     const int64_t slots_used = pieces + (n % share == 0 ? 0 : items - full);
     const double us = (double)share * longest / n * tile_us(i8, D, (int)pieces, cus) +
-                      item * (1 + 0.7 * (double)(begun - 1)) + kMergeUs + D / 128.0 * kMergeUsPerSlot * (double)slots_used;
+                      item * (1 + 0.7 * (double)(begun - 1)) + kMergeUs + D / 128.0 * kMergeUsPerSlot * (double)slots_used +
+                      kMergeUsPerPart * n;
     if (us < best) best = us, best_n = n;
   }
-  if (!best_n) return;
+  if (!best_n) return 1;
   k.full = full;
   k.line = 0;
   for (int p = 0; p < k.nprob; ++p) {
@@ -1685,6 +1688,7 @@ void plan_split(KArgs &k, bool i8, int D, int64_t ws_bytes) {
   }
   k.share = (k.line + slots - 1) / slots;
   k.pieces = (k.line + k.share - 1) / k.share;
+  return best_n;
 }
 
 // Checks one call's arguments and fills its problem and segments (tables
@@ -1770,7 +1774,7 @@ int launch_group(KArgs &k, int D, void *ws, int64_t ws_bytes, hipStream_t s, con
     if (items > 0x3fffffff) return set_error(TMHD_ERR_UNSUPPORTED, "attention: grid too large");
   }
   k.ws = (float *)ws;
-  plan_split(k, I8, D, ws_bytes);
+  plan_split(k, I8, D, ws_bytes, device_cus());
   const unsigned grid = (unsigned)(k.full + k.pieces);
   if (I8 && D == 128)
     hipLaunchKernelGGL((attn_i8_kernel<128>), dim3(grid), dim3(kWaves * 64), 0, s, k);
@@ -1887,6 +1891,18 @@ extern "C" int tmhd_attn_fwd_bf16_noalloc(const tmhd_attn_args *args, void *stre
   a.split_workspace = ws;
   a.split_workspace_bytes = (int64_t)sizeof(scratch);
   return launch_attn<false>(&a, nullptr, 1, stream);
+}
+
+extern "C" int tmhd_attn_last_round_ranges(int32_t items, int32_t key_tiles, int32_t head_dim, int32_t i8qk,
+                                           int64_t workspace_bytes, int32_t cus) {
+  using namespace tmhd;
+  if (items <= 0 || items > 0x3fffffff || key_tiles <= 0 || (head_dim != 64 && head_dim != 128)) return -1;
+  float slot;  // stands for a workspace; only its presence is looked at
+  KArgs k{};
+  k.heads = items, k.nprob = 1;
+  k.pr[0].nqt = 1, k.pr[0].ntiles = key_tiles;
+  k.ws = workspace_bytes > 0 ? &slot : nullptr;
+  return plan_split(k, i8qk != 0, head_dim, workspace_bytes, cus > 0 ? cus : device_cus());
 }
 
 extern "C" int64_t tmhd_attn_split_workspace_bytes(int32_t head_dim) {

@@ -206,6 +206,7 @@ _SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
 # include/tmhd_batch.h and include/tmhd_forms.h
 _MORE_SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "tmhd_gemm_last_round_form": (c_int, [c_int32, c_int32, c_int32, c_int64, c_int32]),
+    "tmhd_attn_last_round_ranges": (c_int, [c_int32, c_int32, c_int32, c_int32, c_int64, c_int32]),
     "tmhd_attn_fwd_bf16_batch": (c_int, [POINTER(AttnArgs), c_int32, c_void_p]),
     "tmhd_attn_fwd_i8qk_batch": (c_int, [POINTER(AttnArgs), POINTER(QKQuant), c_int32, c_void_p]),
     "tmhd_qk_smooth_quant_batch": (
