@@ -277,16 +277,27 @@ def require_same_gpu(torch: Any, device: Any, **tensors: Any) -> None:
             raise ValueError(f"{name} must be on {device} (found {tensor.device})")
 
 
+_gpu_index: dict[Any, int] = {}  # devices that name a GPU by its index -> the index
+
+
 def stream_ptr(torch: Any, device: Any) -> int:
     """Handle of the current stream on ``device``, given as
     ``torch.cuda.current_stream`` takes it (read directly: a Stream object
-    costs 2 us, and a hook call asks several times)."""
-    if not isinstance(device, torch.device):
-        device = torch.device("cuda" if device is None else device)
-    if device.type != "cuda":
-        raise ValueError(f"expected a GPU device, got {device}")
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    costs 2 us, and a hook call asks several times; reading ``device.type``
+    each time would cost as much again as the handle, 0.25 us)."""
+    index = _gpu_index.get(device)
+    if index is None:
+        given = device
+        if not isinstance(device, torch.device):
+            device = torch.device("cuda" if device is None else device)
+        if device.type != "cuda":
+            raise ValueError(f"expected a GPU device, got {device}")
+        index = device.index
+        if index is None:
+            index = torch.cuda.current_device()
+        else:
+            _gpu_index[given] = index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(tensor: Any) -> int:
