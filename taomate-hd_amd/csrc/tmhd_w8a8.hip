@@ -16,13 +16,15 @@ namespace {
 // ---------------------------------------------------------------------------
 // Row quantization, WPR waves (1 or 4, the whole workgroup) per row.  CH =
 // 8-element chunks held per lane (one pass, row kept in registers); CH = 0
-// streams the row twice.  Bound by HBM.  Four waves from 2,056 columns on: one
-// wave's registers (167 for 5,376 columns) let three rows a SIMD be in flight
-// and rows beyond 8,192 columns not be held at all.  us before / now, 331 rows:
+// streams the row twice.  Bound by HBM.  Four waves for long rows: one wave's
+// registers (167 for 5,376 columns) let three rows a SIMD be in flight and rows
+// beyond 8,192 columns not be held at all.  us with one wave / four, 331 rows:
 // 5,376 columns 4.6 / 3.6, 14,336 18.3 / 5.3; 4,836 rows: 17.2 / 14.9 (5.2
-// TB/s), 63.6 / 34.9; 12,252 rows: 35.5 / 32.4, 163 / 96.5.  Below it the wait
-// for the other waves costs more than it gives (12,252 rows of 2,048 columns
-// 13.8 us with one wave, 15.6 with four; 3,072 columns 19.9 and 19.6).
+// TB/s), 63.6 / 34.9; 12,252 rows: 35.5 / 32.4, 163 / 96.5.  Shorter rows lose
+// more by the wait for the other waves: 4,836 rows of 2,056 columns 6.6 / 8.4, of
+// 2,560 7.2 / 8.4, of 3,072 8.4 / 9.0; 12,252 rows 13.8 / 16.8, 15.8 / 16.9, 18.5
+// both.  Between them the rows decide: 3,584 columns, 2,048 rows 4.9 / 5.2, 4,836
+// 10.1 both, 12,252 21.4 / 20.8; 4,096 columns 5.3 / 5.5, 11.2 both, 24.0 / 23.0.
 // WEIGHT selects the weight formula of _quantize_cutlass_w8a8_weight:
 //   scale = max(amax / 127, 1e-12), q = clamp(rint(w / scale), -127, 127)
 // otherwise the activation formula:
@@ -133,6 +135,12 @@ int launch_row_quant(int8_t *q, float *scale, const void *x, int32_t rows, int32
     go(integral_constant<int, 1>{}, integral_constant<int, 2>{});
   else if (nch <= 4 * 64)
     go(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+  else if (nch <= 5 * 64)
+    go(integral_constant<int, 1>{}, integral_constant<int, 5>{});
+  else if (nch <= 6 * 64)
+    go(integral_constant<int, 1>{}, integral_constant<int, 6>{});
+  else if (nch <= 8 * 64 && rows <= 4096)
+    go(integral_constant<int, 1>{}, integral_constant<int, 8>{});
   else if (nch <= 2 * 256)
     go(integral_constant<int, 4>{}, integral_constant<int, 2>{});
   else if (nch <= 3 * 256)

@@ -12,8 +12,13 @@ from tests.helpers import randn_bf16, to_dev
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [1, 5])
-@pytest.mark.parametrize("cols", [8, 512, 520, 1024, 1032, 2048, 2056, 4096, 4104, 6144, 6152, 8192, 8200, 16384, 16392])
+@pytest.mark.parametrize(
+    "rows,cols",
+    [(rows, cols) for rows in (1, 5) for cols in (8, 512, 520, 1024, 1032, 2048, 2056, 2560, 2568, 3072, 3080, 4096,
+                                                  4104, 6144, 6152, 8192, 8200, 16384, 16392)]
+    # four waves from 4,097 rows on
+    + [(rows, cols) for rows in (4096, 4097) for cols in (3080, 4096)],
+)
 def test_row_quant_at_form_edges(torch_mod, dev, rows, cols):
     from taomate_hd_amd import quant
 
