@@ -18,7 +18,10 @@ and runs SDPA or SageAttention.  Here the history is read in place from the
 cache's slots, the chunk's own K/V rows are packed once into a slot (for a
 commit, that slot *is* the staged block), and one HIP kernel launch computes
 every attention of the call over its segments.  Query rows are read and output
-rows written in place through contiguous ranges or row lists.
+rows written in place through contiguous ranges or row lists.  The launch's
+last, partial round is cut into key ranges over all of them, so the rounding of
+the condition or padding rows' outputs may depend on the media rows and the
+history beside them; the same call gives the same bits.
 
 Backends: ``"sdpa"`` -> BF16 kernel (serial mode); ``"sage_attn"`` -> INT8-QK
 kernel (accelerated mode: smooth-K, per-128-block INT8 Q/K, bf16 P.V).

@@ -10,7 +10,10 @@ rows, as the reference's concatenation does).
 The non-empty documents' K/V rows are packed by one launch into one slot of a
 pooled head-major buffer (each at a 64-row-aligned offset, tile tail zeroed);
 one BF16 launch (per 16 documents) then reads their query rows in place and
-writes their output rows in place, with no per-document concatenation.
+writes their output rows in place, with no per-document concatenation.  The
+launch's last, partial round is cut into key ranges over all of its documents,
+so the rounding of a document's output (bf16, from fp32 parts) may depend on
+which others are in the call; the same call gives the same bits.
 """
 
 from __future__ import annotations

@@ -202,9 +202,10 @@ class SlotPool:
 
     Streams: a slot is handed out again only on the stream it was released
     on, where the kernels that last read it are queued ahead of any new
-    writer; and ``release`` records that stream on the slot's memory, so a
-    slot returned to the allocator is not reused on its allocation stream
-    before those kernels end.  A slot in use (between ``acquire`` and
+    writer; and ``release`` records that stream on the slot's memory where it
+    is not the stream of the allocation (which needs no record), so a slot
+    returned to the allocator is not reused on its allocation stream before
+    those kernels end.  A slot in use (between ``acquire`` and
     ``release``) is the caller's to order across streams.
     """
 
